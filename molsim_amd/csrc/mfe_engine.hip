@@ -262,6 +262,17 @@ int pair_lanes_for(const mfe_engine *e) {
   return m <= 12.0 ? 1 : (m <= 48.0 ? 2 : 4);
 }
 
+// log2 of the lanes sharing a particle in the list build: they test four
+// candidates each of a row of three cells at a time, so short rows keep one
+// lane busy; long ones are split as far as the particles leave the chip's
+// ~260,000 resident threads idle (beyond that the split only adds partly
+// filled batches).
+int list_lsh_for(const mfe_engine *e) {
+  const double row = 3.0 * e->np / std::max(e->cg.ncells, 1);
+  if (row < 8.0) return 0;
+  return row >= 48.0 && e->np <= 32768 ? 4 : (e->np <= 262144 ? 2 : 0);
+}
+
 int auto_maxnn(const mfe_engine *e) {
   int m = (int)(2.0 * mean_partners(e) + 64.0);
   return std::min(m, std::max(e->np - 1, 1));
@@ -318,7 +329,8 @@ void mfe_fill_view(const mfe_engine *e, mfe::SysDev &v) {
   v.drnlist = e->drnlist;
   v.maxnn = e->maxnn;
   v.cg = e->cg;
-  MFE_SETP(v.c_count, e->c_count); MFE_SETP(v.c_start, e->c_start); MFE_SETP(v.c_of, e->c_of); MFE_SETP(v.c_slot, e->c_slot);
+  MFE_SETP(v.c_count, e->c_count); MFE_SETP(v.c_start, e->c_start); MFE_SETP(v.c_bsum, e->rebuild_sum);
+  v.list_lsh = list_lsh_for(e); MFE_SETP(v.c_of, e->c_of); MFE_SETP(v.c_slot, e->c_slot);
   MFE_SETP(v.c_sorted, e->c_sorted); MFE_SETP(v.c_pos, e->c_pos); MFE_SETP(v.ro_s, e->ro_s); MFE_SETP(v.type_s, e->type_s); MFE_SETP(v.nn, e->nn);
   MFE_SETP(v.pos_f, e->pos_f);
   MFE_SETP(v.nbr, e->nbr); MFE_SETP(v.flags, e->flags);
@@ -464,7 +476,7 @@ int mfe_group_build(mfe_engine *const *eng, int R, const mfe::SysDev *d, hipStre
     if (e->nknot > 0) g.knots = true;
     if (pair_pos64_for(e)) g.pair_any64 = true;
     else g.pair_any32 = true;
-    g.cell_blocks = std::max(g.cell_blocks, nblocks256(e->cg.ncells));
+    g.list_blocks = std::max(g.list_blocks, nblocks256(e->np << list_lsh_for(e)));
     g.kvec = std::max(g.kvec, e->nkvec);
     if (e->ewald == MFE_EWALD_SPME) {
       int fx_rpb, fx_nblk, fy_T, fy_nbx, fz_T, fz_nbx;
@@ -513,7 +525,6 @@ void sync_view(mfe_engine *e) {
   e->grp.side = e->side;
   e->grp.flags = e->flags;
   e->grp.rebuild_bar = e->rebuild_bar;
-  e->grp.rebuild_sum = e->rebuild_sum;
   e->grp.ncu = e->ncu;
   e->grp.sync_spin = e->sync_spin;
   e->sys_dirty = false;
@@ -691,7 +702,7 @@ int mfe_create(const mfe_config *cfg, mfe_engine **out) {
     MFE_HIP_TRY(hipGetDeviceProperties(&prop, e->device));
     e->ncu = prop.multiProcessorCount;
     dalloc(e->rebuild_bar, mfe::kBarWords);
-    dalloc(e->rebuild_sum, (size_t)e->ncu);
+    dalloc(e->rebuild_sum, (size_t)mfe::kScanBlocks);
     mfe::launch_fill_int((int *)e->rebuild_bar, mfe::kBarWords, 0, e->stream);
     dalloc(e->flags, 4);
     dalloc(e->en, mfe::kEnLen);

@@ -161,6 +161,8 @@ constexpr int kBarStride = 32;
 constexpr int kBarTop = kBarGroups * kBarStride;
 constexpr int kBarGen = kBarTop + kBarStride;
 constexpr int kBarWords = kBarGen + kBarStride;
+// ranges of the rebuild's scan of the cell counts
+constexpr int kScanBlocks = 256;
 // threads per block of the pair kernel and its dynamic LDS budget
 constexpr int kPairBlock = 512;
 // blocks of the persistent pair kernel (two per CU)
@@ -260,6 +262,8 @@ struct SysDev {
   CellGeom cg;
   MFE_DPTR(int) c_count;
   MFE_DPTR(int) c_start;
+  MFE_DPTR(int) c_bsum;         // count totals of the scan's ranges [kScanBlocks]
+  int list_lsh;                 // log2 of the lanes per particle of the list build
   MFE_DPTR(int) c_of;
   MFE_DPTR(int) c_slot;
   MFE_DPTR(int) c_sorted;
@@ -421,7 +425,7 @@ struct Group {
   int prec = 0, ewald = 0, order = 0;
   bool chains = false, surf = false, cells = false;
   // maxima over the replicas of each launch's per-replica block counts
-  int np_blocks = 0, pair_blocks = 0, cell_blocks = 0, bricks = 0, kvec = 0;
+  int np_blocks = 0, pair_blocks = 0, list_blocks = 0, bricks = 0, kvec = 0;
   int mesh_blocks = 0;   // blocks of 256 over the real mesh
   int fx_blocks = 0, fy_x = 0, fy_y = 0, fz_x = 0, fz_y = 0;
   size_t lds_spread = 0, lds_gather = 0, lds_fx = 0, lds_fy = 0, lds_fz = 0;
@@ -431,7 +435,6 @@ struct Group {
   // count
   int *flags = nullptr;
   unsigned *rebuild_bar = nullptr;
-  int *rebuild_sum = nullptr;
   int ncu = 0;
   int sync_spin = -1;       // polls before a barrier wait gives up (-1: default)
   bool pair_cf_lds = true;  // every replica's coefficients fit in LDS
@@ -472,7 +475,7 @@ struct mfe_engine {
   // particle state (device, xyz-interleaved FP64)
   double *ro = nullptr, *rod = nullptr, *rodd = nullptr;
   unsigned *rebuild_bar = nullptr;  // grid barrier of k_rebuild [kBarWords]
-  int *rebuild_sum = nullptr;       // its per-block scan totals [ncu]
+  int *rebuild_sum = nullptr;       // the scan's range totals [kScanBlocks]
   int ncu = 0;                      // compute units of the device
   int sync_spin = -1;               // k_rebuild's barrier poll bound (-1: default)
   double *force = nullptr;   // UTotal's force(3,na) before unit scaling

@@ -78,63 +78,66 @@ __device__ __forceinline__ void ph_scan(int *count, int *start, int n) {
   if (threadIdx.x == blockDim.x - 1) start[n] = wpre + x;
 }
 
-// The same scan over all blocks of a grid (k_rebuild): each block scans its
-// contiguous range into start[] and leaves its total in bsum[block]; after
-// a grid barrier each block adds the totals of the blocks before it.
-__device__ __forceinline__ void ph_scan_local(const int *count, int *start, int n, int *bsum) {
+// The scan of the cell counts split over kScanBlocks contiguous ranges:
+// each range's exclusive prefix is left in place of its counts and its
+// total in c_bsum (this phase); after a barrier the scatter adds the totals
+// of the earlier ranges (scan_bases) to what it reads.
+__device__ __forceinline__ int scan_range(const SysDev &V) {
+  return (V.cg.ncells + kScanBlocks - 1) / kScanBlocks;
+}
+
+__device__ __forceinline__ void ph_scan_local(const SysDev &V, int blk, int nblk) {
   __shared__ int wsum[16];
-  const int nb = gridDim.x, C = (n + nb - 1) / nb;
-  const int lo = min(n, blockIdx.x * C), hi = min(n, lo + C);
+  int *count = V.c_count;
+  const int n = V.cg.ncells, C = scan_range(V);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  int carry = 0;
-  for (int base = lo; base < hi; base += blockDim.x) {
-    const int i = base + threadIdx.x;
-    const int v = i < hi ? count[i] : 0;
-    int x = v;
+  for (int sb = blk; sb < kScanBlocks; sb += nblk) {
+    const int lo = min(n, sb * C), hi = min(n, lo + C);
+    int carry = 0;
+    for (int base = lo; base < hi; base += blockDim.x) {
+      const int i = base + threadIdx.x;
+      const int v = i < hi ? count[i] : 0;
+      int x = v;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+      }
+      if (lane == 63) wsum[wave] = x;
+      __syncthreads();
+      int wpre = 0, tot = 0;
+      for (int w = 0; w < nw; ++w) {
+        wpre += w < wave ? wsum[w] : 0;
+        tot += wsum[w];
+      }
+      if (i < hi) count[i] = carry + wpre + x - v;
+      carry += tot;
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) V.c_bsum[sb] = carry;
+  }
+}
+
+// the totals before each range, base[0..kScanBlocks), by the whole block
+__device__ __forceinline__ void scan_bases(const SysDev &V, int *base) {
+  __shared__ int wsum[kScanBlocks / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int v = 0, x = 0;
+  if (threadIdx.x < kScanBlocks) {
+    v = V.c_bsum[threadIdx.x];
+    x = v;
     for (int o = 1; o < 64; o <<= 1) {
       const int y = __shfl_up(x, o, 64);
       if (lane >= o) x += y;
     }
     if (lane == 63) wsum[wave] = x;
-    __syncthreads();
-    int wpre = 0, tot = 0;
-    for (int w = 0; w < nw; ++w) {
-      wpre += w < wave ? wsum[w] : 0;
-      tot += wsum[w];
-    }
-    if (i < hi) start[i] = carry + wpre + x - v;
-    carry += tot;
-    __syncthreads();
   }
-  if (threadIdx.x == 0) bsum[blockIdx.x] = carry;
-}
-
-__device__ __forceinline__ void ph_scan_offset(int *count, int *start, int n, const int *bsum) {
-  __shared__ int wsum[16];
-  const int nb = gridDim.x, C = (n + nb - 1) / nb;
-  const int lo = min(n, blockIdx.x * C), hi = min(n, lo + C);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  // totals of the blocks before this one (nb <= blockDim), in a fixed order
-  int v = 0;
-  for (int k = threadIdx.x; k < (int)blockIdx.x; k += blockDim.x) v += bsum[k];
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-  if (lane == 0) wsum[wave] = v;
   __syncthreads();
-  int off = 0;
-  for (int w = 0; w < nw; ++w) off += wsum[w];
-  for (int i = lo + threadIdx.x; i < hi; i += blockDim.x) {
-    start[i] += off;
-    count[i] = 0;
+  if (threadIdx.x < kScanBlocks) {
+    int pre = 0;
+    for (int w = 0; w < wave; ++w) pre += wsum[w];
+    base[threadIdx.x] = pre + x - v;
   }
-  if (blockIdx.x == nb - 1 && threadIdx.x == 0) start[n] = off + bsum[nb - 1];
-}
-
-__global__ void __launch_bounds__(1024) k_scan(const SysDev *__restrict__ sys,
-                                               int which, int gated) {
-  const SysDev &V = sys[blockIdx.z];
-  if (gated && V.flags[1] == 0) return;
-  if (which) ph_scan(V.b_count, V.b_start, V.nbricks);
-  else ph_scan(V.c_count, V.c_start, V.cg.ncells);
+  __syncthreads();
 }
 
 // ------------------------------------------------------- neighbour lists
@@ -182,25 +185,60 @@ __device__ __forceinline__ void ph_cell_count(const SysDev &V, int t0, int nt) {
   }
 }
 
-__device__ __forceinline__ void ph_cell_scatter(const SysDev &V, int t0, int nt) {
-  for (int i = t0; i < V.np; i += nt) V.c_sorted[V.c_start[V.c_of[i]] + V.c_slot[i]] = i;
+// Particles placed into their cells in the order of the count's atomics,
+// in c_pos (free until the list build writes it); base: the ranges' totals
+// (scan_bases), with the final cell starts written here, or null when
+// c_start already holds them.
+__device__ __forceinline__ void ph_cell_scatter(const SysDev &V, int t0, int nt,
+                                                const int *base) {
+  const int C = scan_range(V), nc = V.cg.ncells;
+  for (int i = t0; i < V.np; i += nt) {
+    const int c = V.c_of[i];
+    const int st = base ? V.c_count[c] + base[c / C] : V.c_start[c];
+    V.c_pos[st + V.c_slot[i]] = i;
+  }
+  if (!base) return;
+  for (int c = t0; c < nc; c += nt) V.c_start[c] = V.c_count[c] + base[c / C];
+  if (t0 == 0) V.c_start[nc] = V.np;
 }
 
-// members of each cell in ascending particle index (deterministic lists)
-__device__ __forceinline__ void ph_cell_sort(const SysDev &V, int t0, int nt) {
-  const int *start = V.c_start;
-  int *sorted = V.c_sorted;
-  for (int c = t0; c < V.cg.ncells; c += nt) {
+// Members of each cell in ascending particle index (deterministic lists),
+// and the positions and types in that order.  A particle's place is the
+// number of its cell's members with a smaller index: a thread per particle
+// counts them, so a crowded cell (a box of fewer than three cells per axis
+// is one cell) costs its occupancy, not a serial sort by one thread:
+// 1000 ions in one cell 31 ms -> 12 us.  Also clears the counts.
+__device__ __forceinline__ void ph_cell_rank(const SysDev &V, int t0, int nt) {
+  const int *__restrict__ tmp = V.c_pos;
+  const int *__restrict__ start = V.c_start;
+  for (int t = t0; t < V.np; t += nt) {
+    const int i = tmp[t];
+    const int c = V.c_of[i];
+    const double x = V.ro[3 * i], y = V.ro[3 * i + 1], z = V.ro[3 * i + 2];
+    const int ty = V.type[i];
     const int lo = start[c], hi = start[c + 1];
-    for (int i = lo + 1; i < hi; ++i) {
-      int v = sorted[i], j = i - 1;
-      while (j >= lo && sorted[j] > v) {
-        sorted[j + 1] = sorted[j];
-        --j;
-      }
-      sorted[j + 1] = v;
+    int rank = 0;
+    int k = lo;
+    for (; k + 8 <= hi; k += 8) {
+      int v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = tmp[k + u];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) rank += v[u] < i ? 1 : 0;
+    }
+    for (; k < hi; ++k) rank += tmp[k] < i ? 1 : 0;
+    const int p = lo + rank;
+    V.c_sorted[p] = i;
+    V.ro_s[3 * p] = x;
+    V.ro_s[3 * p + 1] = y;
+    V.ro_s[3 * p + 2] = z;
+    V.type_s[p] = ty;
+    if (V.pos_f) {
+      const double r[3] = {x, y, z};
+      V.pos_f[p] = rel_pos(V, r, c, ty);
     }
   }
+  for (int c = t0; c < V.cg.ncells; c += nt) V.c_count[c] = 0;
 }
 
 // positions and types in cell order (ro_s, type_s)
@@ -222,16 +260,18 @@ __device__ __forceinline__ void ph_sort_pos(const SysDev &V, int t0, int nt) {
 }
 
 // Full Verlet list: every j != i with r2 < (rcut+drnlist)^2 (SetVListMD's
-// test, Src/nlist.F90:746-750).  Threads take particles in cell order
-// (t -> i = sorted[t]) and store partners by their cell-order position, so
-// the pair kernel reads neighbouring positions from neighbouring memory;
-// the list is column-major, nbr[k*np + t].  The half list the reference
-// keeps is the checkerboard subset of this set.  POS_S: the cell-ordered
-// positions are already in ro_s (read there, contiguously); else they are
-// read through sorted[] and ro_s / type_s are written here.
-template <bool POS_S>
-__device__ __forceinline__ void ph_nlist_build(const SysDev &V, int t0, int nt) {
-  const double *__restrict__ ro = V.ro;
+// test, Src/nlist.F90:746-750).  Particles are taken in cell order
+// (t -> i = sorted[t], positions from ro_s) and partners stored by their
+// cell-order position, so the pair kernel reads neighbouring positions from
+// neighbouring memory; the list is column-major, nbr[k*np + t].  The half
+// list the reference keeps is the checkerboard subset of this set.
+//
+// 1 << lsh lanes share a particle: of each row of cells they test 4 << lsh
+// candidates at a time and append the hits in candidate order (ballot
+// prefix), so the list is the same for any lsh.  The test is a dependent
+// load and some 20 FP64 operations, and one lane per particle leaves
+// crowded cells to a few wavefronts (see list_lanes for the choice).
+__device__ __forceinline__ void ph_nlist_build(const SysDev &V, int t0, int nt, int lsh) {
   const double *__restrict__ ros = V.ro_s;
   const int np = V.np;
   const CellGeom g = V.cg;
@@ -245,11 +285,13 @@ __device__ __forceinline__ void ph_nlist_build(const SysDev &V, int t0, int nt) 
   int *__restrict__ nbr = V.nbr;
   int *flags = V.flags;
   double *drosum = V.drosum;
-  for (int t = t0; t < np; t += nt) {
+  const int lanes = 1 << lsh, sub = t0 & (lanes - 1);
+  const int gsh = (threadIdx.x & 63) & ~(lanes - 1);
+  const unsigned gmask = lanes == 1 ? 1u : ((1u << lanes) - 1u);
+  const unsigned below = (1u << sub) - 1u;
+  for (int t = t0 >> lsh; t < np; t += nt >> lsh) {
     const int i = sorted[t];
-    const double xi = POS_S ? ros[3 * t] : ro[3 * i];
-    const double yi = POS_S ? ros[3 * t + 1] : ro[3 * i + 1];
-    const double zi = POS_S ? ros[3 * t + 2] : ro[3 * i + 2];
+    const double xi = ros[3 * t], yi = ros[3 * t + 1], zi = ros[3 * t + 2];
     const int c = cof[i];
     const int cx = c % g.n[0], cy = (c / g.n[0]) % g.n[1], cz = c / (g.n[0] * g.n[1]);
     const int rx = g.n[0] > 1 ? 1 : 0, ry = g.n[1] > 1 ? 1 : 0, rz = g.n[2] > 1 ? 1 : 0;
@@ -265,7 +307,7 @@ __device__ __forceinline__ void ph_nlist_build(const SysDev &V, int t0, int nt) 
         // the row's cells x-1, x, x+1 (one on an axis of one cell): their
         // bounds loaded together, then their particles taken as one
         // sequence in the same order (cell by cell, p ascending), four
-        // positions in flight at a time
+        // positions per lane in flight at a time
         int cs[3] = {0, 0, 0}, cn[3] = {0, 0, 0};
         unsigned cd[3] = {0u, 0u, 0u};
 #pragma unroll
@@ -283,11 +325,11 @@ __device__ __forceinline__ void ph_nlist_build(const SysDev &V, int t0, int nt) 
 #pragma unroll
         for (int k = 0; k < 3; ++k) cn[k] -= cs[k];
         const int n01 = cn[0] + cn[1], tot = n01 + cn[2];
-        for (int q0 = 0; q0 < tot; q0 += 4) {
+        for (int q0 = 0; q0 < tot; q0 += 4 << lsh) {
           int pp[4], kk[4];
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            const int q = q0 + u;
+            const int q = q0 + (u << lsh) + sub;
             const int k = q < cn[0] ? 0 : (q < n01 ? 1 : 2);
             kk[u] = k;
             // past the row's end: the particle itself (skipped below)
@@ -296,53 +338,40 @@ __device__ __forceinline__ void ph_nlist_build(const SysDev &V, int t0, int nt) 
           double xj[4], yj[4], zj[4];
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            if (POS_S) {
-              xj[u] = ros[3 * pp[u]];
-              yj[u] = ros[3 * pp[u] + 1];
-              zj[u] = ros[3 * pp[u] + 2];
-            } else {
-              const int j = sorted[pp[u]];
-              xj[u] = ro[3 * j];
-              yj[u] = ro[3 * j + 1];
-              zj[u] = ro[3 * j + 2];
-            }
+            xj[u] = ros[3 * pp[u]];
+            yj[u] = ros[3 * pp[u] + 1];
+            zj[u] = ros[3 * pp[u] + 2];
           }
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            if (pp[u] == t) continue;
             double ddx = xi - xj[u], ddy = yi - yj[u], ddz = zi - zj[u];
             const double r2 = pbcr2(ddx, ddy, ddz, b);
-            if (r2 < rs2) {
+            const bool hit = pp[u] != t && r2 < rs2;
+            const unsigned m = lanes == 1 ? (hit ? 1u : 0u)
+                                          : (unsigned)(__ballot(hit) >> gsh) & gmask;
+            if (hit) {
+              const int at = n + __popc(m & below);
               const unsigned code = kk[u] == 0 ? cd[0] : (kk[u] == 1 ? cd[1] : cd[2]);
-              if (n < maxnn) nbr[(size_t)n * np + t] = (int)((unsigned)pp[u] | code);
-              ++n;
+              if (at < maxnn) nbr[(size_t)at * np + t] = (int)((unsigned)pp[u] | code);
             }
+            n += __popc(m);
           }
         }
       }
     }
-    // on overflow only the stored maxnn partners are visible to the pair
-    // kernel; the call reports MFE_E_NEIGH_CAPACITY
-    nn[t] = min(n, maxnn);
-    if (n > maxnn) atomicOr(&flags[0], ERR_CAPACITY);
-    // cell-ordered positions and types for the pair kernel; k_move keeps
-    // them current through c_pos until the next rebuild
-    V.c_pos[i] = t;
-    if (!POS_S) {
-      V.ro_s[3 * t] = xi;
-      V.ro_s[3 * t + 1] = yi;
-      V.ro_s[3 * t + 2] = zi;
-      const int ty = V.type[i];
-      V.type_s[t] = ty;
-      if (V.pos_f) {
-        const double r[3] = {xi, yi, zi};
-        V.pos_f[t] = rel_pos(V, r, c, ty);
+    if (sub == 0) {
+      // on overflow only the stored maxnn partners are visible to the pair
+      // kernel; the call reports MFE_E_NEIGH_CAPACITY
+      nn[t] = min(n, maxnn);
+      if (n > maxnn) atomicOr(&flags[0], ERR_CAPACITY);
+      // k_move keeps the cell-ordered positions current through c_pos
+      // until the next rebuild
+      V.c_pos[i] = t;
+      if (drosum) {
+        drosum[3 * i] = 0.0;
+        drosum[3 * i + 1] = 0.0;
+        drosum[3 * i + 2] = 0.0;
       }
-    }
-    if (drosum) {
-      drosum[3 * i] = 0.0;
-      drosum[3 * i + 1] = 0.0;
-      drosum[3 * i + 2] = 0.0;
     }
   }
 }
@@ -357,20 +386,29 @@ __global__ void k_cell_count(const SysDev *__restrict__ sys, int gated) {
   ph_cell_count(V, t0, nt);
 }
 
-__global__ void k_cell_scatter(const SysDev *__restrict__ sys, int gated) {
-  MFE_GATE
-  ph_cell_scatter(V, t0, nt);
+__global__ void __launch_bounds__(1024) k_cell_scan(const SysDev *__restrict__ sys, int gated) {
+  const SysDev &V = sys[blockIdx.z];
+  if (gated && V.flags[1] == 0) return;
+  ph_scan_local(V, blockIdx.x, gridDim.x);
 }
 
-__global__ void k_cell_sort(const SysDev *__restrict__ sys, int gated) {
+__global__ void __launch_bounds__(kBlock) k_cell_scatter(const SysDev *__restrict__ sys,
+                                                         int gated) {
   MFE_GATE
-  ph_cell_sort(V, t0, nt);
+  __shared__ int base[kScanBlocks];
+  scan_bases(V, base);
+  ph_cell_scatter(V, t0, nt, base);
+}
+
+__global__ void k_cell_rank(const SysDev *__restrict__ sys, int gated) {
+  MFE_GATE
+  ph_cell_rank(V, t0, nt);
 }
 
 __global__ void __launch_bounds__(kBlock) k_nlist_build(const SysDev *__restrict__ sys,
                                                         int gated) {
   MFE_GATE
-  ph_nlist_build<false>(V, t0, nt);
+  ph_nlist_build(V, t0, nt, V.list_lsh);
   if (t0 == 0 && gated) V.flags[2] += 1;
 }
 #undef MFE_GATE
@@ -444,22 +482,19 @@ __device__ __forceinline__ bool grid_sync(unsigned *bar, int *flags, int spin) {
 // The list rebuild's phases in order, separated by grid barriers, run by
 // every block of a launch whose blocks are all resident (one 1024-thread
 // block per CU).  A block leaves as soon as a barrier gives up.
-__device__ __forceinline__ void rebuild_phases(const SysDev &V, unsigned *bar, int *bsum,
-                                               int spin) {
+__device__ __forceinline__ void rebuild_phases(const SysDev &V, unsigned *bar, int spin) {
   const int t0 = blockIdx.x * blockDim.x + threadIdx.x, nt = gridDim.x * blockDim.x;
+  __shared__ int base[kScanBlocks];
   ph_cell_count(V, t0, nt);
   if (!grid_sync(bar, V.flags, spin)) return;
-  ph_scan_local(V.c_count, V.c_start, V.cg.ncells, bsum);
+  ph_scan_local(V, blockIdx.x, gridDim.x);
   if (!grid_sync(bar, V.flags, spin)) return;
-  ph_scan_offset(V.c_count, V.c_start, V.cg.ncells, bsum);
+  scan_bases(V, base);
+  ph_cell_scatter(V, t0, nt, base);
   if (!grid_sync(bar, V.flags, spin)) return;
-  ph_cell_scatter(V, t0, nt);
+  ph_cell_rank(V, t0, nt);
   if (!grid_sync(bar, V.flags, spin)) return;
-  ph_cell_sort(V, t0, nt);
-  if (!grid_sync(bar, V.flags, spin)) return;
-  ph_sort_pos(V, t0, nt);
-  if (!grid_sync(bar, V.flags, spin)) return;
-  ph_nlist_build<true>(V, t0, nt);
+  ph_nlist_build(V, t0, nt, V.list_lsh);
   if (t0 == 0) V.flags[2] += 1;
 }
 
@@ -472,9 +507,9 @@ __device__ __forceinline__ void rebuild_phases(const SysDev &V, unsigned *bar, i
 // decision is one load away rather than behind the view's.
 __global__ void __launch_bounds__(1024) k_rebuild(const SysDev *__restrict__ sys,
                                                   const int *__restrict__ gate, unsigned *bar,
-                                                  int *bsum, int spin) {
+                                                  int spin) {
   if (gate[1] == 0 || (gate[0] & ERR_SYNC)) return;
-  rebuild_phases(sys[0], bar, bsum, spin);
+  rebuild_phases(sys[0], bar, spin);
 }
 
 // positions and types in cell order for the pair kernel (every UTotal)
@@ -2684,7 +2719,7 @@ __global__ void __launch_bounds__(kReduceThreads) k_reduce_finalize(const SysDev
 // require.
 __global__ void __launch_bounds__(kReduceThreads) k_finalize_rebuild(
     const SysDev *__restrict__ sys, int energy, int bd, int mode, double dt, int split,
-    unsigned *bar, int *bsum, int spin) {
+    unsigned *bar, int spin) {
   const SysDev &V = sys[0];
   const int nb = V.nblk_np;
   const double *pmove = V.part + V.off_move, *pcand = V.part + V.off_skin;
@@ -2723,7 +2758,7 @@ __global__ void __launch_bounds__(kReduceThreads) k_finalize_rebuild(
   // after a failed rebuild earlier in the call the list stays void
   if (__hip_atomic_load(&V.flags[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ERR_SYNC)
     return;
-  rebuild_phases(V, bar, bsum, spin);
+  rebuild_phases(V, bar, spin);
 }
 
 // ------------------------------------------------- persistent batched BD
@@ -3224,13 +3259,11 @@ MFE_STAGE void p_rebuild(const SysDev &V, int *wi) {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   block_scan_counts(V.c_count, V.c_start, nc, wi);
   __syncthreads();
-  ph_cell_scatter(V, tid, NT);
+  ph_cell_scatter(V, tid, NT, nullptr);
   __syncthreads();
-  ph_cell_sort(V, tid, NT);
+  ph_cell_rank(V, tid, NT);
   __syncthreads();
-  ph_sort_pos(V, tid, NT);
-  __syncthreads();
-  ph_nlist_build<true>(V, tid, NT);
+  ph_nlist_build(V, tid, NT, 0);
   if (tid == 0) V.flags[2] += 1;
   __syncthreads();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -3371,19 +3404,20 @@ void launch_fill_double(double *p, int n, double v, hipStream_t s) {
 void launch_nlist_rebuild(const Group &g, bool gated) {
   if (gated && g.R == 1 && g.rebuild_bar && g.flags && g.ncu > 0) {
     hipLaunchKernelGGL(k_rebuild, dim3(g.ncu), dim3(1024), 0, g.stream, g.d, g.flags,
-                       g.rebuild_bar, g.rebuild_sum, g.sync_spin >= 0 ? g.sync_spin : kGridSpin);
+                       g.rebuild_bar, g.sync_spin >= 0 ? g.sync_spin : kGridSpin);
     return;
   }
   // gated kernels run on small grids (grid-stride loops): when the skin
   // test does not fire they cost one dispatch of a few hundred wavefronts
   const int gb = gated ? std::min(g.np_blocks, 256) : g.np_blocks;
-  const int gc = gated ? std::min(g.cell_blocks, 256) : g.cell_blocks;
+  const int gl = gated ? std::min(g.list_blocks, 1024) : g.list_blocks;
+  const int gs = gated && g.R > 1 ? 16 : kScanBlocks;
   const int gt = gated ? 1 : 0;
   hipLaunchKernelGGL(k_cell_count, grid(gb, g), dim3(kBlock), 0, g.stream, g.d, gt);
-  hipLaunchKernelGGL(k_scan, grid(1, g), dim3(1024), 0, g.stream, g.d, 0, gt);
+  hipLaunchKernelGGL(k_cell_scan, grid(gs, g), dim3(1024), 0, g.stream, g.d, gt);
   hipLaunchKernelGGL(k_cell_scatter, grid(gb, g), dim3(kBlock), 0, g.stream, g.d, gt);
-  hipLaunchKernelGGL(k_cell_sort, grid(gc, g), dim3(kBlock), 0, g.stream, g.d, gt);
-  hipLaunchKernelGGL(k_nlist_build, grid(gb, g), dim3(kBlock), 0, g.stream, g.d, gt);
+  hipLaunchKernelGGL(k_cell_rank, grid(gb, g), dim3(kBlock), 0, g.stream, g.d, gt);
+  hipLaunchKernelGGL(k_nlist_build, grid(gl, g), dim3(kBlock), 0, g.stream, g.d, gt);
 }
 
 void launch_sort_pos(const Group &g) {
@@ -3584,7 +3618,7 @@ bool launch_finalize_rebuild(const Group &g, unsigned flags, bool bd, int mode, 
   if (!(g.R == 1 && g.rebuild_bar && g.flags && g.ncu > 1)) return false;
   const int energy = (flags & (MFE_ENERGY | MFE_VIRIAL)) ? 1 : 0;
   hipLaunchKernelGGL(k_finalize_rebuild, dim3(g.ncu), dim3(kReduceThreads), 0, g.stream, g.d,
-                     energy, bd ? 1 : 0, mode, dt, split ? 1 : 0, g.rebuild_bar, g.rebuild_sum,
+                     energy, bd ? 1 : 0, mode, dt, split ? 1 : 0, g.rebuild_bar,
                      g.sync_spin >= 0 ? g.sync_spin : kGridSpin);
   return true;
 }
