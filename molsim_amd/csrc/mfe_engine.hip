@@ -162,7 +162,7 @@ void free_all(mfe_engine *e) {
   dfree(e->ax_g); dfree(e->ax_kk);
   for (auto &t : e->tw) dfree(t);
   dfree(e->tw_half);
-  dfree(e->k_vec); dfree(e->k_sum); dfree(e->ch_prev); dfree(e->ch_next);
+  dfree(e->k_vec); dfree(e->k_sum); dfree(e->k_n); dfree(e->ch_prev); dfree(e->ch_next);
   dfree(e->part); dfree(e->en);
   dfree(e->bd_fac1); dfree(e->bd_fac2); dfree(e->bd_noise); dfree(e->d_sys);
   dfree(e->ro_stage);
@@ -391,6 +391,8 @@ void mfe_fill_view(const mfe_engine *e, mfe::SysDev &v) {
     v.f_fzT = mfe::make_fastdiv(v.fz_T);
   }
   MFE_SETP(v.k_vec, e->k_vec); MFE_SETP(v.k_sum, e->k_sum); v.nkvec = e->nkvec;
+  MFE_SETP(v.k_n, e->k_n); v.ncut = e->ncut;
+  for (int m = 0; m < 3; ++m) v.tpb[m] = e->k_tpb[m];
   v.nchain = e->nchain; v.bond_p = e->bond_p; MFE_SETP(v.ch_prev, e->ch_prev); MFE_SETP(v.ch_next, e->ch_next);
   v.bond_k = e->bond_k; v.bond_eq = e->bond_eq;
   v.ang_k = e->ang_k; v.ang_eq = e->ang_eq; v.ang_p = e->ang_p;
@@ -478,6 +480,7 @@ int mfe_group_build(mfe_engine *const *eng, int R, const mfe::SysDev *d, hipStre
     else g.pair_any32 = true;
     g.list_blocks = std::max(g.list_blocks, nblocks256(e->np << list_lsh_for(e)));
     g.kvec = std::max(g.kvec, e->nkvec);
+    if (e->ewald == MFE_EWALD_STD) g.ncut = std::max(g.ncut, e->ncut);
     if (e->ewald == MFE_EWALD_SPME) {
       int fx_rpb, fx_nblk, fy_T, fy_nbx, fz_T, fz_nbx;
       size_t lfx, lfy, lfz;
@@ -1117,6 +1120,7 @@ int mfe_set_ewald(mfe_engine *e, int32_t kind, double alpha, int32_t order,
       double tpb[3];
       for (int m = 0; m < 3; ++m) tpb[m] = 2.0 * kPi * (1.0 / e->box.L[m]);
       std::vector<double> kv;
+      std::vector<ushort4> kn;
       // kfac in the reference's order (Src/energy.F90:6757-6783)
       for (int nz = 0; nz <= ncut; ++nz) {
         const double facz = nz == 0 ? 1.0 : 2.0;
@@ -1128,6 +1132,7 @@ int mfe_set_ewald(mfe_engine *e, int32_t kind, double alpha, int32_t order,
             const double facx = nx == 0 ? 0.5 : 1.0;
             const double k2 = (nx * tpb[0]) * (nx * tpb[0]) + (ny * tpb[1]) * (ny * tpb[1]) +
                               (nz * tpb[2]) * (nz * tpb[2]);
+            kn.push_back(make_ushort4((unsigned short)nx, (unsigned short)ny, (unsigned short)nz, 0));
             kv.push_back(nx * tpb[0]);
             kv.push_back(ny * tpb[1]);
             kv.push_back(nz * tpb[2]);
@@ -1138,7 +1143,11 @@ int mfe_set_ewald(mfe_engine *e, int32_t kind, double alpha, int32_t order,
       e->nkvec = (int)(kv.size() / 4);
       dalloc(e->k_vec, kv.size());
       dalloc(e->k_sum, 8 * (size_t)e->nkvec);
+      dalloc(e->k_n, kn.size());
       upload(e->k_vec, kv.data(), kv.size(), e->stream);
+      upload(e->k_n, kn.data(), kn.size(), e->stream);
+      MFE_HIP_TRY(hipStreamSynchronize(e->stream));
+      for (int m = 0; m < 3; ++m) e->k_tpb[m] = tpb[m];
     }
     layout_partials(e);
     MFE_HIP_TRY(hipStreamSynchronize(e->stream));

@@ -309,7 +309,9 @@ struct SysDev {
   // standard Ewald
   MFE_DPTR(const double) k_vec;
   MFE_DPTR(double) k_sum;
-  int nkvec;
+  MFE_DPTR(const ushort4) k_n;  // wave numbers of k_vec along the axes
+  int nkvec, ncut;
+  double tpb[3];                // 2 pi / L of k_vec's box
   // chains
   int nchain, bond_p;
   MFE_DPTR(const int) ch_prev;
@@ -425,7 +427,7 @@ struct Group {
   int prec = 0, ewald = 0, order = 0;
   bool chains = false, surf = false, cells = false;
   // maxima over the replicas of each launch's per-replica block counts
-  int np_blocks = 0, pair_blocks = 0, list_blocks = 0, bricks = 0, kvec = 0;
+  int np_blocks = 0, pair_blocks = 0, list_blocks = 0, bricks = 0, kvec = 0, ncut = 0;
   int mesh_blocks = 0;   // blocks of 256 over the real mesh
   int fx_blocks = 0, fy_x = 0, fy_y = 0, fz_x = 0, fz_y = 0;
   size_t lds_spread = 0, lds_gather = 0, lds_fx = 0, lds_fy = 0, lds_fz = 0;
@@ -565,6 +567,8 @@ struct mfe_engine {
   int ncut = 0, ncut_cube = 0, nkvec = 0;
   double *k_vec = nullptr;   // [nkvec][4]: kx, ky, kz (2*pi*n/L), kfac
   double *k_sum = nullptr;   // [nkvec][2] structure factor (re, im)
+  ushort4 *k_n = nullptr;    // [nkvec] wave numbers along the axes
+  double k_tpb[3] = {0.0, 0.0, 0.0};  // 2 pi / L of the table's box
 
   // chains
   int nchain = 0;

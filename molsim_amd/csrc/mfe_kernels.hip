@@ -207,7 +207,7 @@ __device__ __forceinline__ void ph_cell_scatter(const SysDev &V, int t0, int nt,
 // number of its cell's members with a smaller index: a thread per particle
 // counts them, so a crowded cell (a box of fewer than three cells per axis
 // is one cell) costs its occupancy, not a serial sort by one thread:
-// 1000 ions in one cell 31 ms -> 12 us.  Also clears the counts.
+// 1000 ions in one cell 31 ms -> 27 us.  Also clears the counts.
 __device__ __forceinline__ void ph_cell_rank(const SysDev &V, int t0, int nt) {
   const int *__restrict__ tmp = V.c_pos;
   const int *__restrict__ start = V.c_start;
@@ -270,7 +270,7 @@ __device__ __forceinline__ void ph_sort_pos(const SysDev &V, int t0, int nt) {
 // candidates at a time and append the hits in candidate order (ballot
 // prefix), so the list is the same for any lsh.  The test is a dependent
 // load and some 20 FP64 operations, and one lane per particle leaves
-// crowded cells to a few wavefronts (see list_lanes for the choice).
+// crowded cells to a few wavefronts (list_lsh_for chooses).
 __device__ __forceinline__ void ph_nlist_build(const SysDev &V, int t0, int nt, int lsh) {
   const double *__restrict__ ros = V.ro_s;
   const int np = V.np;
@@ -1911,42 +1911,76 @@ __global__ void __launch_bounds__(64) k_mc_pair_sum(const double *__restrict__ p
 // UEwaldRecStd (Src/energy.F90:1050-1096) over the k-vectors of its kfac
 // table: one block per k-vector sums the four sign combinations of the
 // structure factor; a second kernel gives each particle its force.
-__global__ void __launch_bounds__(kBlock) k_ewald_sk(const SysDev *__restrict__ sys,
-                                                     int energy) {
+//
+// The phases of a k-vector's four combinations (-x,-y,+z), (-x,+y,+z),
+// (+x,-y,+z), (+x,+y,+z) are products of the three axes' phases, so a
+// particle takes three sincos (or none, from a table per axis) in place of
+// four, and at smaller arguments.
+__device__ __forceinline__ double2 cmul(double2 a, double2 b) {
+  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+}
+__device__ __forceinline__ void four_phases(double2 ex, double2 ey, double2 ez, double2 e[4]) {
+  const double2 exc = make_double2(ex.x, -ex.y);
+  const double2 A = cmul(ey, ez), B = cmul(make_double2(ey.x, -ey.y), ez);
+  e[0] = cmul(exc, B);
+  e[1] = cmul(exc, A);
+  e[2] = cmul(ex, B);
+  e[3] = cmul(ex, A);
+}
+__device__ __forceinline__ double2 phase(double x) {
+  double2 e;
+  sincos(x, &e.y, &e.x);
+  return e;
+}
+
+// 512 threads per k-vector (a thousand particles are two rounds), the eight
+// sums combined through one LDS exchange: 1000 ions, 8 wave numbers per
+// axis: 9.4 us (11.5 with 256 threads, four sincos, eight block sums); bound
+// by the FP64 sincos chain of each thread.
+constexpr int kSkThreads = 512;
+__global__ void __launch_bounds__(kSkThreads) k_ewald_sk(const SysDev *__restrict__ sys,
+                                                         int energy) {
   const SysDev &V = sys[blockIdx.z];
   if ((int)blockIdx.x >= V.nkvec) return;
   const double *__restrict__ ro = V.ro;
   const double *__restrict__ q = V.q;
   const int np = V.np;
   const double *__restrict__ kv = V.k_vec;
-  double *__restrict__ ksum = V.k_sum;
   const double alpha2 = V.alpha * V.alpha;
-  double *part = V.part + V.off_std;
-  __shared__ double sh[kBlock];
+  __shared__ double red[8][kSkThreads / 64];
   const int kn = blockIdx.x;
   const double kx = kv[4 * kn], ky = kv[4 * kn + 1], kz = kv[4 * kn + 2];
   double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int i = threadIdx.x; i < np; i += blockDim.x) {
-    const double x = kx * ro[3 * i], y = ky * ro[3 * i + 1], z = kz * ro[3 * i + 2];
-    double sa, ca;
-    // combinations (-x,-y,+z), (-x,+y,+z), (+x,-y,+z), (+x,+y,+z)
-    sincos(-x - y + z, &sa, &ca);
-    s[0] += q[i] * ca; s[1] += q[i] * sa;
-    sincos(-x + y + z, &sa, &ca);
-    s[2] += q[i] * ca; s[3] += q[i] * sa;
-    sincos(x - y + z, &sa, &ca);
-    s[4] += q[i] * ca; s[5] += q[i] * sa;
-    sincos(x + y + z, &sa, &ca);
-    s[6] += q[i] * ca; s[7] += q[i] * sa;
+  for (int i = threadIdx.x; i < np; i += kSkThreads) {
+    const double qi = q[i];
+    double2 e[4];
+    four_phases(phase(kx * ro[3 * i]), phase(ky * ro[3 * i + 1]), phase(kz * ro[3 * i + 2]), e);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      s[2 * c] += qi * e[c].x;
+      s[2 * c + 1] += qi * e[c].y;
+    }
   }
-  double tot[8];
-  for (int c = 0; c < 8; ++c) tot[c] = block_sum(s[c], sh);
-  if (threadIdx.x == 0) {
-    for (int c = 0; c < 8; ++c) ksum[8 * kn + c] = tot[c];
-    if (energy) {
-      double ssum = 0.0;
-      for (int c = 0; c < 8; ++c) ssum += tot[c] * tot[c];
-      const double term = kv[4 * kn + 3] * ssum;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    for (int w = 32; w > 0; w >>= 1) s[c] += __shfl_down(s[c], w, 64);
+    if (lane == 0) red[c][wave] = s[c];
+  }
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  // lane c of the first wavefront: component c, the wavefronts in order
+  double t = 0.0;
+  if (lane < 8) {
+    for (int w = 0; w < kSkThreads / 64; ++w) t += red[lane][w];
+    V.k_sum[8 * kn + lane] = t;
+  }
+  if (energy) {
+    double t2 = t * t;
+    for (int w = 4; w > 0; w >>= 1) t2 += __shfl_down(t2, w, 64);
+    if (lane == 0) {
+      double *part = V.part + V.off_std;
+      const double term = kv[4 * kn + 3] * t2;
       const double k2 = kx * kx + ky * ky + kz * kz;
       part[kn] = term;
       part[V.nkvec + kn] = -(1.0 - k2 / (2.0 * alpha2)) * term;
@@ -1954,39 +1988,74 @@ __global__ void __launch_bounds__(kBlock) k_ewald_sk(const SysDev *__restrict__ 
   }
 }
 
-__global__ void __launch_bounds__(kBlock) k_ewald_force(const SysDev *__restrict__ sys) {
+// One wavefront per particle, its lanes over the k-vectors: a thread per
+// particle ran every k-vector's four sincos one after another, on a few
+// wavefronts (1000 ions, 8 wave numbers per axis: 259 us, now 5.8, bound by
+// the reads of the structure factors and the launch).  TAB: the axes'
+// phases e^{i n 2 pi x / L}, n = 0..ncut, are computed once per particle
+// into LDS; without it (tables beyond the launch's LDS) per k-vector.
+constexpr int kEwParticles = 4;
+template <bool TAB>
+__global__ void __launch_bounds__(64 * kEwParticles) k_ewald_force(
+    const SysDev *__restrict__ sys) {
   const SysDev &V = sys[blockIdx.z];
-  const double *__restrict__ ro = V.ro;
-  const double *__restrict__ q = V.q;
+  extern __shared__ __align__(16) double2 ew_tab[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int i = blockIdx.x * kEwParticles + wave;
+  if (blockIdx.x * kEwParticles >= V.np) return;
+  const bool act = i < V.np;
   const double *__restrict__ kv = V.k_vec;
   const double *__restrict__ ksum = V.k_sum;
-  const int nk = V.nkvec;
-  const double efp = V.efp;
-  double *__restrict__ force = V.force;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= V.np) return;
-  const double xi = ro[3 * i], yi = ro[3 * i + 1], zi = ro[3 * i + 2];
-  double fx = 0.0, fy = 0.0, fz = 0.0;
-  for (int kn = 0; kn < nk; ++kn) {
-    const double kx = kv[4 * kn], ky = kv[4 * kn + 1], kz = kv[4 * kn + 2];
-    const double kfac2 = efp * 2.0 * kv[4 * kn + 3];
-    const double *S = ksum + 8 * kn;
-    const double x = kx * xi, y = ky * yi, z = kz * zi;
-    double f[4];
-    const double args[4] = {-x - y + z, -x + y + z, x - y + z, x + y + z};
-    for (int c = 0; c < 4; ++c) {
-      double sa, ca;
-      sincos(args[c], &sa, &ca);
-      // -Re(q e) Im(S) + Im(q e) Re(S)
-      f[c] = q[i] * (-ca * S[2 * c + 1] + sa * S[2 * c]);
+  const int nk = V.nkvec, nt = V.ncut + 1;
+  double2 *tab = ew_tab + (size_t)wave * 3 * nt;
+  double r[3] = {0.0, 0.0, 0.0}, qi = 0.0;
+  if (act) {
+#pragma unroll
+    for (int m = 0; m < 3; ++m) r[m] = V.ro[3 * i + m];
+    qi = V.q[i];
+  }
+  if (TAB) {
+    for (int e = lane; e < 3 * nt; e += 64) {
+      const int m = e / nt, n = e - m * nt;
+      tab[e] = phase((n * V.tpb[m]) * (m == 0 ? r[0] : (m == 1 ? r[1] : r[2])));
     }
+    __syncthreads();
+  }
+  double fx = 0.0, fy = 0.0, fz = 0.0;
+  for (int kn = lane; kn < nk; kn += 64) {
+    const double kx = kv[4 * kn], ky = kv[4 * kn + 1], kz = kv[4 * kn + 2];
+    const double kfac2 = V.efp * 2.0 * kv[4 * kn + 3];
+    const double *S = ksum + 8 * kn;
+    double2 ex, ey, ez, e[4];
+    if (TAB) {
+      const ushort4 n = V.k_n[kn];
+      ex = tab[n.x];
+      ey = tab[nt + n.y];
+      ez = tab[2 * nt + n.z];
+    } else {
+      ex = phase(kx * r[0]);
+      ey = phase(ky * r[1]);
+      ez = phase(kz * r[2]);
+    }
+    four_phases(ex, ey, ez, e);
+    double f[4];
+    // -Re(q e) Im(S) + Im(q e) Re(S)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) f[c] = qi * (-e[c].x * S[2 * c + 1] + e[c].y * S[2 * c]);
     fx += kfac2 * kx * (-f[0] - f[1] + f[2] + f[3]);
     fy += kfac2 * ky * (-f[0] + f[1] - f[2] + f[3]);
     fz += kfac2 * kz * (f[0] + f[1] + f[2] + f[3]);
   }
-  force[3 * i] += fx;
-  force[3 * i + 1] += fy;
-  force[3 * i + 2] += fz;
+  for (int w = 32; w > 0; w >>= 1) {
+    fx += __shfl_down(fx, w, 64);
+    fy += __shfl_down(fy, w, 64);
+    fz += __shfl_down(fz, w, 64);
+  }
+  if (act && lane == 0) {
+    V.force[3 * i] += fx;
+    V.force[3 * i + 1] += fy;
+    V.force[3 * i + 2] += fz;
+  }
 }
 
 // ------------------------------------------------------------------ bonds
@@ -3587,8 +3656,13 @@ void launch_spme(const Group &g, bool energy, int first, int last, int gmode,
 }
 
 void launch_std_ewald(const Group &g) {
-  hipLaunchKernelGGL(k_ewald_sk, grid(g.kvec, g), dim3(kBlock), 0, g.stream, g.d, 1);
-  hipLaunchKernelGGL(k_ewald_force, grid(g.np_blocks, g), dim3(kBlock), 0, g.stream, g.d);
+  hipLaunchKernelGGL(k_ewald_sk, grid(g.kvec, g), dim3(kSkThreads), 0, g.stream, g.d, 1);
+  const dim3 gr = grid((g.np_blocks * kBlock + kEwParticles - 1) / kEwParticles, g);
+  const size_t lds = (size_t)kEwParticles * 3 * (g.ncut + 1) * sizeof(double2);
+  if (lds <= 64 * 1024)
+    hipLaunchKernelGGL(k_ewald_force<true>, gr, dim3(64 * kEwParticles), lds, g.stream, g.d);
+  else
+    hipLaunchKernelGGL(k_ewald_force<false>, gr, dim3(64 * kEwParticles), 0, g.stream, g.d);
 }
 
 void launch_bonds(const Group &g) {
