@@ -68,6 +68,24 @@ __device__ __forceinline__ double quad_swap(double x) {
   return __hiloint2double(hi, lo);
 }
 
+// Sum over the wavefront of an FP64 value, by DPP exchanges inside each row
+// of 16 lanes (quads, half rows, rows) and lane reads across the four rows:
+// no LDS round trips (a shuffle tree of FP64 takes twelve).  Every lane of
+// the wavefront must be active; every lane gets the sum.
+constexpr int kHalfMirror = 0x141;  // lane 7 - l of each 8
+constexpr int kMirror = 0x140;      // lane 15 - l of each 16
+__device__ __forceinline__ double read_lane(double x, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), lane),
+                          __builtin_amdgcn_readlane(__double2loint(x), lane));
+}
+__device__ __forceinline__ double wave_sum(double x) {
+  x += quad_swap<kXor1>(x);
+  x += quad_swap<kXor2>(x);
+  x += quad_swap<kHalfMirror>(x);
+  x += quad_swap<kMirror>(x);
+  return (read_lane(x, 0) + read_lane(x, 16)) + (read_lane(x, 32) + read_lane(x, 48));
+}
+
 // ------------------------------------------------- spline pair term
 // Uniform cubic B-spline on knots r0 + k/dinv: on interval i (fraction f)
 // the weights of coefficients i..i+3 are (1-f)^3/6, (3f^3-6f^2+4)/6,

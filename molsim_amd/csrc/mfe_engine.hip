@@ -143,7 +143,7 @@ void free_all(mfe_engine *e) {
   dfree(e->drosum); dfree(e->r2disp); dfree(e->type); dfree(e->q); dfree(e->massip);
   dfree(e->t_zlow); dfree(e->t_coef); dfree(e->t_coef_f); dfree(e->t_off);
   dfree(e->t_nint); dfree(e->t_pairidx); dfree(e->t_r2atat); dfree(e->t_r2umin);
-  dfree(e->t_bin_k); dfree(e->t_rec);
+  dfree(e->t_img); dfree(e->t_rec);
   dfree(e->c_count); dfree(e->c_start); dfree(e->c_of); dfree(e->c_slot);
   dfree(e->c_sorted); dfree(e->c_pos); dfree(e->nn); dfree(e->nbr); dfree(e->flags);
   dfree(e->rebuild_bar); dfree(e->rebuild_sum);
@@ -176,11 +176,42 @@ void free_all(mfe_engine *e) {
   e->h_flags = nullptr;
 }
 
+// expected Verlet-list length (partners within rcut + drnlist)
+double mean_partners(const mfe_engine *e) {
+  const double rs = e->rcut + e->drnlist;
+  const double vol = e->box.L[0] * e->box.L[1] * e->box.L[2];
+  return 4.0 / 3.0 * kPi * rs * rs * rs * e->np / vol;
+}
+
+// Boxes with an axis of fewer than three list cells: the mixed path forms
+// separations in FP64.
+bool pair_pos64_for(const mfe_engine *e) {
+  return e->cg.n[0] < 3 || e->cg.n[1] < 3 || e->cg.n[2] < 3;
+}
+
+// Lanes per particle of the pair kernels.  A lane evaluates batches of four
+// entries: on the mixed path lists of up to ~12 keep one lane busy, up to
+// ~48 two, longer ones (and the FP64 separations and the FP64 path) take
+// four.  A small system does not fill the chip that way (6000 particles:
+// 47 blocks), so the lanes double while they keep a batch each and the
+// launch stays under kPairThreads threads.
+constexpr int kPairThreads = 131072;
+int pair_lanes_for(const mfe_engine *e) {
+  const double m = mean_partners(e);
+  int lanes = 4;
+  if (e->prec == MFE_PREC_MIXED && !pair_pos64_for(e)) lanes = m <= 12.0 ? 1 : (m <= 48.0 ? 2 : 4);
+  while (lanes < 64 && 2 * lanes * (long long)e->np <= kPairThreads &&
+         m >= 4.0 * (2 * lanes))
+    lanes *= 2;
+  return lanes;
+}
+
 // partial-sum regions of the reductions (see k_reduce)
 void layout_partials(mfe_engine *e) {
   const int nb = (e->np + 255) / 256;
   e->nblk_pair = std::min(mfe::kPairGridMax,
-                          (e->np * mfe::kPairLanes + mfe::kPairBlock - 1) / mfe::kPairBlock);
+                          (int)(((long long)e->np * pair_lanes_for(e) + mfe::kPairBlock - 1) /
+                                mfe::kPairBlock));
   e->nblk_bond = nb;
   e->nblk_surf = nb;
   e->nblk_move = nb;
@@ -242,26 +273,6 @@ void set_cell_geom(mfe_engine *e) {
   e->cg = g;
 }
 
-// expected Verlet-list length (partners within rcut + drnlist)
-double mean_partners(const mfe_engine *e) {
-  const double rs = e->rcut + e->drnlist;
-  const double vol = e->box.L[0] * e->box.L[1] * e->box.L[2];
-  return 4.0 / 3.0 * kPi * rs * rs * rs * e->np / vol;
-}
-
-// lanes per particle of the mixed pair kernel: a lane evaluates batches of
-// four entries, so lists of up to ~12 keep one lane busy, up to ~48 two.
-// Boxes with an axis of fewer than three list cells take four (their
-// kernel variant forms separations in FP64).
-bool pair_pos64_for(const mfe_engine *e) {
-  return e->cg.n[0] < 3 || e->cg.n[1] < 3 || e->cg.n[2] < 3;
-}
-int pair_lanes_for(const mfe_engine *e) {
-  if (pair_pos64_for(e)) return 4;
-  const double m = mean_partners(e);
-  return m <= 12.0 ? 1 : (m <= 48.0 ? 2 : 4);
-}
-
 // log2 of the lanes sharing a particle in the list build: they test four
 // candidates each of a row of three cells at a time, so short rows keep one
 // lane busy; long ones are split as far as the particles leave the chip's
@@ -319,7 +330,7 @@ void mfe_fill_view(const mfe_engine *e, mfe::SysDev &v) {
   mfe::TableDev &t = v.tab;
   MFE_SETP(t.zlow, e->t_zlow); MFE_SETP(t.coef, e->t_coef); MFE_SETP(t.coef_f, e->t_coef_f); MFE_SETP(t.off, e->t_off);
   MFE_SETP(t.nint, e->t_nint); MFE_SETP(t.r2atat, e->t_r2atat); MFE_SETP(t.r2umin, e->t_r2umin); MFE_SETP(t.pairidx, e->t_pairidx);
-  MFE_SETP(t.bin_k, e->t_bin_k); MFE_SETP(t.rec, e->t_rec);
+  MFE_SETP(t.img, e->t_img); MFE_SETP(t.rec, e->t_rec);
   MFE_SETP(t.rec_f, e->t_rec_f); MFE_SETP(t.zlow_f, e->t_zlow_f);
   t.nbin = e->t_nbin;
   t.lds_mode = e->t_lds_mode;
@@ -956,8 +967,7 @@ int mfe_set_tables(mfe_engine *e, const double *ubuf, int32_t nbuf, const int32_
     dalloc(e->t_zlow, zl.size()); dalloc(e->t_coef, cf.size()); dalloc(e->t_coef_f, cf.size());
     dalloc(e->t_off, (size_t)P); dalloc(e->t_nint, (size_t)P); dalloc(e->t_pairidx, pidx.size());
     dalloc(e->t_r2atat, (size_t)P); dalloc(e->t_r2umin, (size_t)P);
-    dalloc(e->t_bin_k, bin_k.size()); dalloc(e->t_rec, (size_t)P);
-    upload(e->t_bin_k, bin_k.data(), bin_k.size(), e->stream);
+    dalloc(e->t_rec, (size_t)P);
     upload(e->t_rec, rec.data(), (size_t)P, e->stream);
     std::vector<mfe::PairRecF> rec_f(P);
     for (int p = 0; p < P; ++p) {
@@ -974,6 +984,18 @@ int mfe_set_tables(mfe_engine *e, const double *ubuf, int32_t nbuf, const int32_
     const size_t csz = e->prec == MFE_PREC_MIXED ? 4 : 8;
     const size_t bb = mfe::pair_bin_bytes(P, nbin), zb = mfe::pair_zl_bytes((int)zl.size());
     const size_t cb = zl.size() * mfe::kCoefStride * csz;
+    std::vector<unsigned char> img(bb + zb + cb, 0);
+    std::memcpy(img.data(), bin_k.data(), bin_k.size() * sizeof(unsigned short));
+    if (e->prec == MFE_PREC_MIXED) {
+      std::memcpy(img.data() + bb, zl_f.data(), zl_f.size() * sizeof(float));
+      std::memcpy(img.data() + bb + zb, cff.data(), cb);
+    } else {
+      std::memcpy(img.data() + bb, zl.data(), zl.size() * sizeof(double));
+      std::memcpy(img.data() + bb + zb, cf.data(), cb);
+    }
+    dalloc(e->t_img, img.size() / sizeof(uint4));
+    MFE_HIP_TRY(hipMemcpyAsync(e->t_img, img.data(), img.size(), hipMemcpyHostToDevice,
+                               e->stream));
     e->t_lds_mode = 0;
     e->t_lds_bytes = bb;
     if (bb + zb <= mfe::kPairLdsBudget) {
@@ -1173,6 +1195,8 @@ int mfe_set_neighbor(mfe_engine *e, int32_t kind, double drnlist, int32_t maxnne
       e->maxnn = m;
     }
     int rc = prepare_neighbor(e);
+    // the pair launch's blocks follow the lanes, these the list length
+    layout_partials(e);
     MFE_HIP_TRY(hipStreamSynchronize(e->stream));
     e->list_valid = false;
     touch(e);

@@ -37,9 +37,6 @@ namespace mfe {
 constexpr int kEnAngle = 8 + MFE_MAX_PAIRS;
 constexpr int kEnLen = kEnAngle + 1;
 
-// lanes of the pair kernel that share one particle's neighbour list
-constexpr int kPairLanes = 4;
-
 struct HipError {
   hipError_t code;
   const char *expr;
@@ -138,7 +135,10 @@ struct TableDev {
   // bins of s = 1/r2 per pair (see PairRec): entry kb means the interval
   // of any r2 in the bin is kb or kb + 1; kb | kSlowBin means the bin
   // spans more intervals and the search walks from kb
-  MFE_DPTR(const unsigned short) bin_k;  // [nptpt * nbin]
+  // [nptpt * nbin], the first part of the image
+  // what the pair kernels stage in LDS, in its layout there: bins, interval
+  // bounds, coefficients (of the engine's precision), each from 16 bytes on
+  MFE_DPTR(const uint4) img;
   MFE_DPTR(const PairRec) rec;           // [nptpt]
   MFE_DPTR(const PairRecF) rec_f;        // [nptpt]
   MFE_DPTR(const float) zlow_f;          // zlow in FP32
@@ -353,8 +353,9 @@ struct SysDev {
   MFE_DPTR(double) en;
   int off_pair, off_conv, off_bond, off_surf, off_std, off_move, off_skin;
   int nblk_np, nblk_pair, nblk_conv;
-  // mixed pair kernel: lanes per particle (1, 2, 4) and whether the box
-  // has an axis of fewer than three list cells (separations in FP64)
+  // pair kernels: lanes per particle (a power of two up to 64); mixed path:
+  // whether the box has an axis of fewer than three list cells (separations
+  // in FP64)
   int pair_lanes, pair_pos64;
   double ffac, surf_fac;
 };
@@ -496,7 +497,7 @@ struct mfe_engine {
   float *t_coef_f = nullptr;
   int *t_off = nullptr, *t_nint = nullptr, *t_pairidx = nullptr;
   double *t_r2atat = nullptr, *t_r2umin = nullptr;
-  unsigned short *t_bin_k = nullptr;
+  uint4 *t_img = nullptr;  // the pair kernels' LDS image of the tables
   mfe::PairRec *t_rec = nullptr;
   mfe::PairRecF *t_rec_f = nullptr;
   float *t_zlow_f = nullptr;

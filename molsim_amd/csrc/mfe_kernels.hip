@@ -537,6 +537,30 @@ __device__ __forceinline__ int find_interval(const Z &zl, int n, double r2, int 
 // list entries a lane loads together (indices, then positions)
 constexpr int kPairBatch = 4;
 
+// The first `bytes` (a multiple of 16) of the tables' image copied into LDS,
+// 16 bytes per load and eight loads in flight per thread: one memory round
+// trip for what element-wise copies of the bins, bounds and coefficients
+// took a dozen for (about 12 us of a small system's pair launch).
+__device__ __forceinline__ void stage_image(unsigned char *lds, const TableDev &t,
+                                            size_t bytes) {
+  uint4 *dst = reinterpret_cast<uint4 *>(lds);
+  batched_copy(
+      (int)(bytes / 16), [&](int e) -> uint4 { return t.img[e]; },
+      [&](int e, uint4 v) { dst[e] = v; });
+}
+
+// The sum of a particle's lanes' values (lanes a power of two, the same for
+// the whole block), in a fixed order.
+__device__ __forceinline__ double lane_sum(double x, int lanes) {
+  if (lanes >= 2) x += quad_swap<kXor1>(x);
+  if (lanes >= 4) x += quad_swap<kXor2>(x);
+  if (lanes >= 8) x += quad_swap<kHalfMirror>(x);
+  if (lanes >= 16) x += quad_swap<kMirror>(x);
+  if (lanes >= 32) x += __shfl_xor(x, 16, 64);
+  if (lanes >= 64) x += __shfl_xor(x, 32, 64);
+  return x;
+}
+
 // k_skin_blocks' computation for skin blocks sb0 and sb0 + 1 (256
 // particles each, the k_move partition), one per half of a 512-thread
 // block: the same maxima in the same order, so the same candidates.
@@ -581,9 +605,9 @@ __device__ __forceinline__ void skin_two_blocks(const SysDev &V, int sb0) {
         fmax(fmax(wred[w0], wred[w0 + 1]), fmax(wred[w0 + 2], wred[w0 + 3]));
 }
 
-// Pair forces over the Verlet list.  kPairLanes lanes share one particle
-// (cell order i) and split its list k = lane, lane + kPairLanes, ...; their
-// partial forces are combined by shuffles in FP64 in a fixed order, so
+// Pair forces over the Verlet list.  V.pair_lanes lanes share one particle
+// (cell order i) and split its list k = lane, lane + lanes, ...; their
+// partial forces are combined by lane exchanges in FP64 in a fixed order, so
 // forces need no atomics and stay deterministic.  Every pair is seen from
 // both ends, so its energy and virial carry weight 1/2.  semantics: 0 =
 // vlist (r2 <= rcut2 kept), 1 = cell list (r2 < rcut2 kept).
@@ -591,7 +615,7 @@ __device__ __forceinline__ void skin_two_blocks(const SysDev &V, int sb0) {
 // The grid is persistent: nblk_pair (<= kPairGridMax) blocks each stage
 // the tables in LDS once -- r2 bins, interval bounds and, with CF, the
 // polynomial coefficients -- and then walk one contiguous range of chunks
-// of kPairBlock / kPairLanes particles.  A lane loads the indices of
+// of kPairBlock / lanes particles.  A lane loads the indices of
 // kPairBatch of its entries together, then their positions, then
 // evaluates them.  NT bounds the number of types: up to 4 the energies
 // accumulate per pair type in registers over all chunks, else per partner
@@ -630,12 +654,9 @@ k_pair(const SysDev *__restrict__ sys, int energy, int pgrid, int skin) {
   unsigned short *bin_s = reinterpret_cast<unsigned short *>(pair_lds);
   double *zl_s = reinterpret_cast<double *>(pair_lds + bb);
   CT *cf_s = reinterpret_cast<CT *>(pair_lds + bb + pair_zl_bytes(nzl));
-  for (int k = threadIdx.x; k < P * nbin; k += blockDim.x) bin_s[k] = t.bin_k[k];
-  if (lds_zl)
-    for (int k = threadIdx.x; k < nzl; k += blockDim.x) zl_s[k] = t.zlow[k];
-  if (CF) {
-    for (int k = threadIdx.x; k < nzl * kCoefStride; k += blockDim.x) cf_s[k] = t.coef[k];
-  }
+  stage_image(pair_lds, t,
+              bb + (lds_zl ? pair_zl_bytes(nzl) : 0) +
+                  (CF ? (size_t)nzl * kCoefStride * sizeof(CT) : 0));
   for (int k = threadIdx.x; k < P; k += blockDim.x) rec_s[k] = t.rec[k];
   for (int k = threadIdx.x; k < npt * npt; k += blockDim.x) pidx_s[k] = t.pairidx[k];
   const int l64 = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -656,7 +677,9 @@ k_pair(const SysDev *__restrict__ sys, int energy, int pgrid, int skin) {
     if constexpr (CF) return zl_s[idx];
     else return lds_zl ? zl_s[idx] : t.zlow[idx];
   };
-  const int lane = threadIdx.x % kPairLanes;
+  // lanes per particle (lsh their log2)
+  const int LANES = V.pair_lanes, lsh = __builtin_ctz(LANES);
+  const int lane = threadIdx.x & (LANES - 1);
   // energy accumulators: per pair type for up to 4 types (kept over all
   // chunks), else per partner type (converted to pair types per chunk)
   constexpr bool kRegE = NT <= 4;
@@ -733,11 +756,11 @@ k_pair(const SysDev *__restrict__ sys, int energy, int pgrid, int skin) {
     }
   };
   // this block's chunks: an even share of the contiguous chunk range
-  constexpr int kChunk = kPairBlock / kPairLanes;
+  const int kChunk = kPairBlock >> lsh;
   const int nch = (np + kChunk - 1) / kChunk;
   const int ch0 = (int)((long long)blk * nch / nb), ch1 = (int)((long long)(blk + 1) * nch / nb);
   for (int ch = ch0; ch < ch1; ++ch) {
-    const int i = ch * kChunk + threadIdx.x / kPairLanes;
+    const int i = ch * kChunk + (threadIdx.x >> lsh);
     if (!kRegE) {
 #pragma unroll
       for (int k = 0; k < NA; ++k) ej[k] = 0.0;
@@ -755,11 +778,11 @@ k_pair(const SysDev *__restrict__ sys, int energy, int pgrid, int skin) {
       // end the particle itself) so no branch makes the compiler wait for
       // them one by one
       const int last = n - 1;
-      for (int k0 = lane; k0 < n; k0 += kPairBatch * kPairLanes) {
+      for (int k0 = lane; k0 < n; k0 += kPairBatch * LANES) {
         int js[kPairBatch];
 #pragma unroll
         for (int g = 0; g < kPairBatch; ++g) {
-          const int kk = k0 + g * kPairLanes;
+          const int kk = k0 + g * LANES;
           const int jr = (int)((unsigned)nbr[(size_t)max(0, min(kk, last)) * np + i] & kNbrIdxMask);
           js[g] = kk < n ? jr : i;
         }
@@ -774,17 +797,12 @@ k_pair(const SysDev *__restrict__ sys, int energy, int pgrid, int skin) {
         }
 #pragma unroll
         for (int g = 0; g < kPairBatch; ++g)
-          if (k0 + g * kPairLanes < n) eval(xi - xs[g], yi - ys[g], zi - zs[g], ts[g]);
+          if (k0 + g * LANES < n) eval(xi - xs[g], yi - ys[g], zi - zs[g], ts[g]);
       }
     }
-    // the four lanes' partial forces: exchanges within the quad by DPP
-    static_assert(kPairLanes == 4, "quad exchanges assume four lanes per particle");
-    fx += quad_swap<kXor1>(fx);
-    fy += quad_swap<kXor1>(fy);
-    fz += quad_swap<kXor1>(fz);
-    fx += quad_swap<kXor2>(fx);
-    fy += quad_swap<kXor2>(fy);
-    fz += quad_swap<kXor2>(fz);
+    fx = lane_sum(fx, LANES);
+    fy = lane_sum(fy, LANES);
+    fz = lane_sum(fz, LANES);
     if (i < np && lane == 0) {
       const int io = V.c_sorted[i];
       V.force[3 * io] = fx;
@@ -801,7 +819,7 @@ k_pair(const SysDev *__restrict__ sys, int energy, int pgrid, int skin) {
           for (int u = 0; u < NA; ++u)
             if (u < npt && pidx_s[ti * npt + u] == k) v += ej[u];
         }
-        for (int w = 32; w > 0; w >>= 1) v += __shfl_down(v, w, 64);
+        v = wave_sum(v);
         if (l64 == 0) wacc[wv][k] += v;
       }
     }
@@ -813,15 +831,13 @@ k_pair(const SysDev *__restrict__ sys, int energy, int pgrid, int skin) {
       // wavefront
 #pragma unroll
       for (int k = 0; k < NA; ++k) {
-        double v = ej[k];
-        for (int w = 32; w > 0; w >>= 1) v += __shfl_down(v, w, 64);
+        const double v = wave_sum(ej[k]);
         if (l64 == 0 && k < P) wacc[wv][k] = v;
       }
     }
     // the virial, then per-block partials, component-major (component k
     // of block b at k * nblk_pair + b), the wavefronts summed in order
-    double v = vir;
-    for (int w = 32; w > 0; w >>= 1) v += __shfl_down(v, w, 64);
+    const double v = wave_sum(vir);
     if (l64 == 0) wacc[wv][P] = v;
     __syncthreads();
     double *out = V.part + V.off_pair + blk;
@@ -918,10 +934,8 @@ __device__ __forceinline__ bool pair_eval_f(const SysDev &V, const PairTabF &T, 
 // edge or so.  Forces are Kahan-compensated FP32 sums, energies FP64 per
 // partner type, flushed into the wavefront's LDS row per chunk.  KN:
 // some replica carries the additive spline term.  V.pair_lanes lanes share
-// a particle's list: 4 for dense systems, fewer where lists are short (a
-// lane then keeps its batch slots busy and the per-particle work is not
-// repeated on idle lanes); a replica's choice is its own, so it computes
-// the same alone and in a batch.  POS64: the replicas whose box has an
+// a particle's list (pair_lanes_for); a replica's choice is its own, so it
+// computes the same alone and in a batch.  POS64: the replicas whose box has an
 // axis of fewer than three list cells, where cell-relative coordinates
 // would span half the box -- the pair's separation is formed in FP64 from
 // the cell-ordered positions and rounded once; the other replicas' blocks
@@ -955,10 +969,10 @@ __device__ __forceinline__ void pair_f_body(const SysDev *__restrict__ sys, int 
   unsigned short *bin_s = reinterpret_cast<unsigned short *>(pair_lds);
   float *zl_s = reinterpret_cast<float *>(pair_lds + bb);
   float *cf_s = reinterpret_cast<float *>(pair_lds + bb + pair_zl_bytes(nzl));
-  for (int k = threadIdx.x; k < P * nbin; k += blockDim.x) bin_s[k] = t.bin_k[k];
-  for (int k = threadIdx.x; k < nzl; k += blockDim.x) zl_s[k] = t.zlow_f[k];
-  if (CF)
-    for (int k = threadIdx.x; k < nzl * kCoefStride; k += blockDim.x) cf_s[k] = t.coef_f[k];
+  const bool lds_zl = CF || t.lds_mode >= 1;
+  stage_image(pair_lds, t,
+              bb + (lds_zl ? pair_zl_bytes(nzl) : 0) +
+                  (CF ? (size_t)nzl * kCoefStride * sizeof(float) : 0));
   for (int k = threadIdx.x; k < P; k += blockDim.x) rec_s[k] = t.rec_f[k];
   for (int k = threadIdx.x; k < npt * npt; k += blockDim.x) pidx_s[k] = t.pairidx[k];
   for (int k = threadIdx.x; k < 125; k += blockDim.x)
@@ -969,8 +983,8 @@ __device__ __forceinline__ void pair_f_body(const SysDev *__restrict__ sys, int 
   const float rc2 = (float)t.rcut2;
   const float L0 = V.cg.L[0], L1 = V.cg.L[1], L2 = V.cg.L[2];
   const float H0 = V.cg.L2[0], H1 = V.cg.L2[1], H2 = V.cg.L2[2];
-  // lanes per particle: 1, 2 or 4 (lsh its log2)
-  const int LANES = V.pair_lanes, lsh = LANES == 4 ? 2 : LANES - 1;
+  // lanes per particle (lsh their log2)
+  const int LANES = V.pair_lanes, lsh = __builtin_ctz(LANES);
   const int lane = threadIdx.x & (LANES - 1);
   double ej[NT];
   double vir = 0.0;
@@ -990,7 +1004,8 @@ __device__ __forceinline__ void pair_f_body(const SysDev *__restrict__ sys, int 
     if (fabsf(dy) > H1) dy -= copysignf(L1, dy);
     if (fabsf(dz) > H2) dz -= copysignf(L2, dz);
   };
-  const PairTabF T{bin_s, zl_s, CF ? cf_s : (const float *)t.coef_f, rec_s, nbin, semantics, rc2};
+  const PairTabF T{bin_s, lds_zl ? zl_s : (const float *)t.zlow_f,
+                   CF ? cf_s : (const float *)t.coef_f, rec_s, nbin, semantics, rc2};
   // one list entry: a partner of type tj at separation (dx, dy, dz)
   auto eval = [&](float dx, float dy, float dz, int tj) {
     const int p = (int)((ptp >> (8 * tj)) & 0xffu);
@@ -1080,18 +1095,9 @@ __device__ __forceinline__ void pair_f_body(const SysDev *__restrict__ sys, int 
       fy = fyf.value();
       fz = fzf.value();
     }
-    // the lanes' partial forces: exchanges within pairs / quads by DPP
-    // (LANES is uniform over the block, so every lane takes part)
-    if (LANES >= 2) {
-      fx += quad_swap<kXor1>(fx);
-      fy += quad_swap<kXor1>(fy);
-      fz += quad_swap<kXor1>(fz);
-    }
-    if (LANES == 4) {
-      fx += quad_swap<kXor2>(fx);
-      fy += quad_swap<kXor2>(fy);
-      fz += quad_swap<kXor2>(fz);
-    }
+    fx = lane_sum(fx, LANES);
+    fy = lane_sum(fy, LANES);
+    fz = lane_sum(fz, LANES);
     if (i < np && lane == 0) {
       const int io = V.c_sorted[i];
       V.force[3 * io] = fx;
@@ -1106,17 +1112,16 @@ __device__ __forceinline__ void pair_f_body(const SysDev *__restrict__ sys, int 
         if (i < np) {
 #pragma unroll
           for (int u = 0; u < NT; ++u)
-            if (u < npt && pidx_s[ti * npt + u] == k) v += ej[u];
+            if (u < npt && (int)((ptp >> (8 * u)) & 0xffu) == k) v += ej[u];
         }
-        for (int w = 32; w > 0; w >>= 1) v += __shfl_down(v, w, 64);
+        v = wave_sum(v);
         if (l64 == 0) wacc[wv][k] += v;
       }
     }
   }
   if (err) atomicOr(&V.flags[0], err);
   if (energy) {
-    double v = vir;
-    for (int w = 32; w > 0; w >>= 1) v += __shfl_down(v, w, 64);
+    const double v = wave_sum(vir);
     if (l64 == 0) wacc[wv][P] = v;
     __syncthreads();
     double *out = V.part + V.off_pair + blk;
@@ -3003,10 +3008,8 @@ MFE_STAGE void p_pair(const SysDev &V, int energy, char *smem, int lds, double (
   float *zl_s = reinterpret_cast<float *>(smem + bb);
   float *cf_s = reinterpret_cast<float *>(smem + bb + pair_zl_bytes(nzl));
   const bool cf_lds = t.lds_mode >= 2;
-  for (int k = tid; k < P * nbin; k += NT) bin_s[k] = t.bin_k[k];
-  for (int k = tid; k < nzl; k += NT) zl_s[k] = t.zlow_f[k];
-  if (cf_lds)
-    for (int k = tid; k < nzl * kCoefStride; k += NT) cf_s[k] = t.coef_f[k];
+  stage_image(reinterpret_cast<unsigned char *>(smem), t,
+              bb + pair_zl_bytes(nzl) + (cf_lds ? (size_t)nzl * kCoefStride * sizeof(float) : 0));
   for (int k = tid; k < P; k += NT) rec_s[k] = t.rec_f[k];
   for (int k = tid; k < npt * npt; k += NT) pidx_s[k] = t.pairidx[k];
   for (int k = tid; k < 125; k += NT)
