@@ -220,7 +220,9 @@ void layout_partials(mfe_engine *e) {
     int a, b, c, d, fz_T, fz_nbx;
     size_t l0, l1, l2;
     mfe::fft_geometry(e->prec, e->s, &a, &b, &c, &d, &fz_T, &fz_nbx, &l0, &l1, &l2);
-    conv = fz_nbx * e->s[1];
+    mfe::ColPlan cy, cz;
+    mfe::column_plans(e->prec, e->s, &cy, &cz);
+    conv = cz.ns ? cz.nblk : fz_nbx * e->s[1];
   }
   e->nblk_conv = conv;
   int off = 0;
@@ -393,6 +395,7 @@ void mfe_fill_view(const mfe_engine *e, mfe::SysDev &v) {
     size_t l0, l1, l2;
     mfe::fft_geometry(e->prec, e->s, &v.fx_rpb, &v.fx_nblk, &v.fy_T, &v.fy_nbx, &v.fz_T,
                       &v.fz_nbx, &l0, &l1, &l2);
+    mfe::column_plans(e->prec, e->s, &v.cy, &v.cz);
     v.f_s1 = mfe::make_fastdiv(e->s[0]);
     v.f_s2 = mfe::make_fastdiv(e->s[1]);
     v.f_s3 = mfe::make_fastdiv(e->s[2]);
@@ -501,10 +504,24 @@ int mfe_group_build(mfe_engine *const *eng, int R, const mfe::SysDev *d, hipStre
       for (int m = 0; m < 3; ++m) g.mc_s[m] = std::max(g.mc_s[m], e->s[m]);
       g.mesh_blocks = std::max(g.mesh_blocks, (e->s[0] * e->s[1] * e->s[2] + 255) / 256);
       g.fx_blocks = std::max(g.fx_blocks, fx_nblk);
-      g.fy_x = std::max(g.fy_x, fy_nbx);
-      g.fy_y = std::max(g.fy_y, e->s[2]);
-      g.fz_x = std::max(g.fz_x, fz_nbx);
-      g.fz_y = std::max(g.fz_y, e->s[1]);
+      mfe::ColPlan cy, cz;
+      mfe::column_plans(e->prec, e->s, &cy, &cz);
+      if (cy.ns) {
+        g.cy_blocks = std::max(g.cy_blocks, cy.nblk);
+        g.cy_thr = std::max(g.cy_thr, cy.nthr);
+        g.lds_cy = std::max(g.lds_cy, (size_t)cy.lds);
+      } else {
+        g.fy_x = std::max(g.fy_x, fy_nbx);
+        g.fy_y = std::max(g.fy_y, e->s[2]);
+      }
+      if (cz.ns) {
+        g.cz_blocks = std::max(g.cz_blocks, cz.nblk);
+        g.cz_thr = std::max(g.cz_thr, cz.nthr);
+        g.lds_cz = std::max(g.lds_cz, (size_t)cz.lds);
+      } else {
+        g.fz_x = std::max(g.fz_x, fz_nbx);
+        g.fz_y = std::max(g.fz_y, e->s[1]);
+      }
       g.lds_fx = std::max(g.lds_fx, lfx);
       g.lds_fy = std::max(g.lds_fy, lfy);
       g.lds_fz = std::max(g.lds_fz, lfz);

@@ -8,6 +8,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+#include <utility>
+
 #include "mfe_internal.h"
 
 namespace mfe {
@@ -232,6 +235,309 @@ __device__ __forceinline__ cplx<R> *lds_fft(cplx<R> *a, cplx<R> *b, const FftPla
     Ns *= r;
   }
   return a;
+}
+
+// ------------------------------------------------ transforms in registers
+// The column passes (y and z) transform a length n = r1 r2 (r3) of radices
+// up to 16 with one radix per stage held in a thread's registers: the first
+// stage reads global memory, the last writes it, and only the one or two
+// exchanges between go through LDS.  A Stockham transform staged through
+// LDS on both ends (lds_fft) moves every value through LDS once more per
+// end and waits at twice as many barriers: 128 points in three stages took
+// eight LDS passes and five barriers, 16 x 8 in registers takes two and one.
+
+// cos and sin of 2 pi k / n, reduced to the first octant (Taylor series)
+struct Trig {
+  double c, s;
+};
+constexpr Trig trig_root(int k, int n) {
+  k %= n;
+  if (2 * k > n) {
+    const Trig t = trig_root(n - k, n);
+    return {t.c, -t.s};
+  }
+  if (4 * k > n) {
+    const Trig t = trig_root(n - 2 * k, 2 * n);
+    return {-t.c, t.s};
+  }
+  if (8 * k > n) {
+    const Trig t = trig_root(n - 4 * k, 4 * n);
+    return {t.s, t.c};
+  }
+  const double x = 6.283185307179586476925286766559 * k / n;
+  double c = 0.0, s = 0.0;
+  // Horner from x^21 and x^20 down: below 1e-20 of the sum for x <= pi/4
+  for (int j = 10; j >= 0; --j) {
+    s = 1.0 - s * x * x / ((2 * j + 2) * (2 * j + 3));
+    c = 1.0 - c * x * x / ((2 * j + 1) * (2 * j + 2));
+  }
+  return {c, s * x};
+}
+
+template <int N, typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F &&f) {
+  static_for_impl<N>(f, std::make_integer_sequence<int, N>{});
+}
+
+// acc + x * C for a constant C; FP32 forward with the constant's rounding
+// residual added by FMA (see Twiddle)
+template <typename R, bool INV>
+__device__ __forceinline__ R mac_const(R acc, R x, double c) {
+  if constexpr (sizeof(R) == 4) {
+    const float hi = (float)c;
+    if constexpr (INV) return __builtin_fmaf(x, hi, acc);
+    return __builtin_fmaf(x, hi, __builtin_fmaf(x, (float)(c - (double)hi), acc));
+  } else {
+    return __builtin_fma(x, c, acc);
+  }
+}
+
+// v * exp(-2 pi i K / N) (forward) or its conjugate (inverse)
+template <typename R, int K, int N, bool INV>
+__device__ __forceinline__ cplx<R> mul_root(cplx<R> v) {
+  constexpr int k = K % N;
+  constexpr R sg = INV ? R(1) : R(-1);  // w = c + i sg s
+  if constexpr (k == 0) {
+    return v;
+  } else if constexpr (4 * k == N) {
+    return {-sg * v.y, sg * v.x};
+  } else if constexpr (2 * k == N) {
+    return {-v.x, -v.y};
+  } else if constexpr (4 * k == 3 * N) {
+    return {sg * v.y, -sg * v.x};
+  } else {
+    constexpr Trig t = trig_root(k, N);
+    constexpr double s = INV ? t.s : -t.s;
+    return {mac_const<R, INV>(mac_const<R, INV>(R(0), v.x, t.c), v.y, -s),
+            mac_const<R, INV>(mac_const<R, INV>(R(0), v.y, t.c), v.x, s)};
+  }
+}
+
+// RAD-point DFT in registers, natural order in and out
+template <typename R, int RAD, bool INV>
+__device__ __forceinline__ void reg_dft(cplx<R> *v) {
+  if constexpr (RAD == 2 || RAD == 4 || RAD == 8) {
+    small_dft<R, RAD>(v, INV, nullptr, 0);
+  } else if constexpr (RAD == 3 || RAD == 5 || RAD == 7) {
+    constexpr int H = (RAD - 1) / 2;
+    cplx<R> t[H], u[H];
+#pragma unroll
+    for (int j = 0; j < H; ++j) {
+      t[j] = cadd(v[j + 1], v[RAD - 1 - j]);
+      u[j] = csub(v[j + 1], v[RAD - 1 - j]);
+    }
+    const cplx<R> v0 = v[0];
+#pragma unroll
+    for (int j = 0; j < H; ++j) v[0] = cadd(v[0], t[j]);
+    static_for<H>([&](auto qi) {
+      constexpr int q = decltype(qi)::value + 1;
+      cplx<R> a = v0, b = {R(0), R(0)};
+      static_for<H>([&](auto ji) {
+        constexpr int j = decltype(ji)::value + 1;
+        constexpr Trig w = trig_root(j * q, RAD);
+        a.x = mac_const<R, INV>(a.x, t[j - 1].x, w.c);
+        a.y = mac_const<R, INV>(a.y, t[j - 1].y, w.c);
+        b.x = mac_const<R, INV>(b.x, u[j - 1].x, w.s);
+        b.y = mac_const<R, INV>(b.y, u[j - 1].y, w.s);
+      });
+      // a -+ i b
+      const cplx<R> ib = INV ? cplx<R>{-b.y, b.x} : cplx<R>{b.y, -b.x};
+      v[q] = cadd(a, ib);
+      v[RAD - q] = csub(a, ib);
+    });
+  } else {
+    // A x B: A-point DFTs over stride B, the roots of RAD, B-point DFTs
+    constexpr int A = RAD % 7 == 0 ? 7 : (RAD % 5 == 0 ? 5 : (RAD == 12 || RAD == 16 ? 4 : 3));
+    constexpr int B = RAD / A;
+    static_assert(A * B == RAD, "radix of two factors");
+    cplx<R> y[RAD];  // y[k1 B + n2]
+    static_for<B>([&](auto n2i) {
+      constexpr int n2 = decltype(n2i)::value;
+      cplx<R> x[A];
+#pragma unroll
+      for (int n1 = 0; n1 < A; ++n1) x[n1] = v[n1 * B + n2];
+      reg_dft<R, A, INV>(x);
+      static_for<A>([&](auto k1i) {
+        constexpr int k1 = decltype(k1i)::value;
+        y[k1 * B + n2] = mul_root<R, k1 * n2, RAD, INV>(x[k1]);
+      });
+    });
+#pragma unroll
+    for (int k1 = 0; k1 < A; ++k1) {
+      reg_dft<R, B, INV>(y + k1 * B);
+#pragma unroll
+      for (int k2 = 0; k2 < B; ++k2) v[k1 + A * k2] = y[k1 * B + k2];
+    }
+  }
+}
+
+// One stage of radix RAD for T = 1 << lgT columns of length n, Ns points
+// already combined: butterfly j of column c reads positions j + q n/RAD,
+// multiplies by w_{Ns RAD}^{q (j mod Ns)}, transforms and writes positions
+// (j / Ns) Ns RAD + j mod Ns + q Ns.  POS: first stage (Ns 1, no twiddles),
+// middle, last (Ns RAD = n, so j < Ns).  rd(pos, c), wr(pos, c, v).
+enum { ST_FIRST = 0, ST_MID = 1, ST_LAST = 2 };
+template <typename R, int RAD, bool INV, int POS>
+__device__ __forceinline__ void stage_twiddle(cplx<R> *v, int j, int n, int Ns, int &base,
+                                              const Twiddle<R> *tw) {
+  if constexpr (POS == ST_FIRST) {
+    base = j * RAD;
+  } else {
+    const int jb = POS == ST_LAST ? 0 : j / Ns, k = j - jb * Ns;
+    const int kt = POS == ST_LAST ? k : k * (n / (Ns * RAD));
+#pragma unroll
+    for (int q = 1; q < RAD; ++q) v[q] = twmul(v[q], tw[kt * q], INV);
+    base = jb * Ns * RAD + k;
+  }
+}
+template <typename R, int RAD, bool INV, int POS, typename Rd, typename Wr>
+__device__ __forceinline__ void col_stage(int n, int lgT, int nt, int Ns, const Twiddle<R> *tw,
+                                          Rd rd, Wr wr) {
+  const int nb = n / RAD, step = POS == ST_FIRST ? 1 : Ns;
+  for (int t = threadIdx.x; t < nb << lgT; t += blockDim.x) {
+    const int c = t & ((1 << lgT) - 1), j = t >> lgT;
+    if (c >= nt) continue;
+    cplx<R> v[RAD];
+#pragma unroll
+    for (int q = 0; q < RAD; ++q) v[q] = rd(j + q * nb, c);
+    int base;
+    stage_twiddle<R, RAD, INV, POS>(v, j, n, Ns, base, tw);
+    reg_dft<R, RAD, INV>(v);
+#pragma unroll
+    for (int q = 0; q < RAD; ++q) wr(base + q * step, c, v[q]);
+  }
+}
+
+#define MFE_FOR_RADIX(r, CALL) \
+  switch (r) {                 \
+    case 2: CALL(2); break;    \
+    case 3: CALL(3); break;    \
+    case 4: CALL(4); break;    \
+    case 5: CALL(5); break;    \
+    case 6: CALL(6); break;    \
+    case 7: CALL(7); break;    \
+    case 8: CALL(8); break;    \
+    case 9: CALL(9); break;    \
+    case 10: CALL(10); break;  \
+    case 12: CALL(12); break;  \
+    case 14: CALL(14); break;  \
+    case 15: CALL(15); break;  \
+    default: CALL(16); break;  \
+  }
+
+template <typename R, bool INV, int POS, typename Rd, typename Wr>
+__device__ __forceinline__ void any_stage(int rad, int n, int lgT, int nt, int Ns,
+                                          const Twiddle<R> *tw, Rd rd, Wr wr) {
+#define MFE_CALL(RAD) col_stage<R, RAD, INV, POS>(n, lgT, nt, Ns, tw, rd, wr)
+  MFE_FOR_RADIX(rad, MFE_CALL)
+#undef MFE_CALL
+}
+
+// The transform of one block's columns: rd(pos, c) reads the input, wr
+// writes the output; A and B hold T n values each (B only for three stages).
+// tw: the length-n twiddles (in LDS: staged by the caller before, read
+// after the first barrier).
+template <typename R, bool INV, typename Rd, typename Wr>
+__device__ __forceinline__ void col_fft(const ColPlan &p, int nt, cplx<R> *A, cplx<R> *B,
+                                        const Twiddle<R> *tw, Rd rd, Wr wr) {
+  const int n = p.n, lgT = p.lgT;
+  auto put = [&](cplx<R> *buf) {
+    return [=](int pos, int c, cplx<R> v) { buf[(pos << lgT) + c] = v; };
+  };
+  auto get = [&](const cplx<R> *buf) {
+    return [=](int pos, int c) { return buf[(pos << lgT) + c]; };
+  };
+  if (p.ns == 1) {
+    any_stage<R, INV, ST_FIRST>(p.r[0], n, lgT, nt, 1, tw, rd, wr);
+    return;
+  }
+  any_stage<R, INV, ST_FIRST>(p.r[0], n, lgT, nt, 1, tw, rd, put(A));
+  __syncthreads();
+  if (p.ns == 2) {
+    any_stage<R, INV, ST_LAST>(p.r[1], n, lgT, nt, p.r[0], tw, get(A), wr);
+    return;
+  }
+  any_stage<R, INV, ST_MID>(p.r[1], n, lgT, nt, p.r[0], tw, get(A), put(B));
+  __syncthreads();
+  any_stage<R, INV, ST_LAST>(p.r[2], n, lgT, nt, p.r[0] * p.r[1], tw, get(B), wr);
+}
+
+// The forward transform's last stage, f(pos, c, v) applied to each output,
+// and the inverse transform's first stage (the radices in reverse order) in
+// the same registers: the outputs j + q n/RAD of one are the inputs of the
+// other.
+// ONE: rd and wr share a buffer; every thread has at most one butterfly and
+// all have read before any writes.
+template <typename R, int RAD, bool ONE, typename Rd, typename Fn, typename Wr>
+__device__ __forceinline__ void conv_stage(int n, int lgT, int nt, const Twiddle<R> *tw, Rd rd,
+                                           Fn f, Wr wr) {
+  const int nb = n / RAD, items = nb << lgT;
+  const int t_end = ONE ? (int)threadIdx.x + 1 : items;
+  for (int t = threadIdx.x; t < t_end; t += blockDim.x) {
+    const int c = t & ((1 << lgT) - 1), j = t >> lgT;
+    const bool act = t < items && c < nt;
+    cplx<R> v[RAD];
+    if (act) {
+#pragma unroll
+      for (int q = 0; q < RAD; ++q) v[q] = rd(j + q * nb, c);
+    }
+    if (ONE) __syncthreads();
+    if (!act) continue;
+    if (nb > 1) {
+#pragma unroll
+      for (int q = 1; q < RAD; ++q) v[q] = twmul(v[q], tw[j * q], false);
+    }
+    reg_dft<R, RAD, false>(v);
+#pragma unroll
+    for (int q = 0; q < RAD; ++q) v[q] = f(j + q * nb, c, v[q]);
+    reg_dft<R, RAD, true>(v);
+#pragma unroll
+    for (int q = 0; q < RAD; ++q) wr(j * RAD + q, c, v[q]);
+  }
+}
+template <typename R, bool ONE, typename Rd, typename Fn, typename Wr>
+__device__ __forceinline__ void any_conv_stage(int rad, int n, int lgT, int nt,
+                                               const Twiddle<R> *tw, Rd rd, Fn f, Wr wr) {
+#define MFE_CALL(RAD) conv_stage<R, RAD, ONE>(n, lgT, nt, tw, rd, f, wr)
+  MFE_FOR_RADIX(rad, MFE_CALL)
+#undef MFE_CALL
+}
+
+// forward transform, f on every element, inverse transform, of one block's
+// columns
+template <typename R, typename Rd, typename Fn, typename Wr>
+__device__ __forceinline__ void col_conv(const ColPlan &p, int nt, cplx<R> *A, cplx<R> *B,
+                                         const Twiddle<R> *tw, Rd rd, Fn f, Wr wr) {
+  const int n = p.n, lgT = p.lgT;
+  auto put = [&](cplx<R> *buf) {
+    return [=](int pos, int c, cplx<R> v) { buf[(pos << lgT) + c] = v; };
+  };
+  auto get = [&](const cplx<R> *buf) {
+    return [=](int pos, int c) { return buf[(pos << lgT) + c]; };
+  };
+  if (p.ns == 1) {
+    any_conv_stage<R, false>(p.r[0], n, lgT, nt, tw, rd, f, wr);
+    return;
+  }
+  any_stage<R, false, ST_FIRST>(p.r[0], n, lgT, nt, 1, tw, rd, put(A));
+  __syncthreads();
+  if (p.ns == 2) {
+    any_conv_stage<R, true>(p.r[1], n, lgT, nt, tw, get(A), f, put(A));
+    __syncthreads();
+    any_stage<R, true, ST_LAST>(p.r[0], n, lgT, nt, p.r[1], tw, get(A), wr);
+    return;
+  }
+  any_stage<R, false, ST_MID>(p.r[1], n, lgT, nt, p.r[0], tw, get(A), put(B));
+  __syncthreads();
+  any_conv_stage<R, false>(p.r[2], n, lgT, nt, tw, get(B), f, put(A));
+  __syncthreads();
+  any_stage<R, true, ST_MID>(p.r[1], n, lgT, nt, p.r[2], tw, get(A), put(B));
+  __syncthreads();
+  any_stage<R, true, ST_LAST>(p.r[0], n, lgT, nt, p.r[2] * p.r[1], tw, get(B), wr);
 }
 
 // ----------------------------------------------------------------- x pass

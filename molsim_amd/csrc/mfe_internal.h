@@ -184,6 +184,15 @@ struct FftPlan {
   int radix[20];
 };
 
+// Column transforms in registers (col_fft): length n as ns <= 3 radices of
+// at most 16, 1 << lgT columns and nthr threads per block, nblk blocks.
+// ns = 0: the length has another prime factor than 2, 3, 5, 7, and the
+// pass runs tile by tile through LDS (ffty_tile, fftconv_tile).
+struct ColPlan {
+  int n, ns, r[3], lgT, nthr, nblk, ncol;
+  int lds;   // bytes of dynamic LDS
+};
+
 // Per-axis SPME tables (FP64): g[n] = b2[n]*exp(-k_n^2/(4 alpha^2)) and
 // kk[n] = k_n^2 for n = 0..s/2, so that
 // meshfac(nx,ny,nz) = fac0 * gx*gy*gz / (kkx+kky+kkz)  (Essmann eq. 3.9).
@@ -298,6 +307,7 @@ struct SysDev {
   MFE_DPTR(void) spread_tiles;   // [nbricks][(B+order-1)^3] spreading tiles
   SpmeAxes ax;
   FftPlan plan[3], plan_half;
+  ColPlan cy, cz;        // y and z passes
   MFE_DPTR(const void) tw[3];
   MFE_DPTR(const void) tw_half;
   int fx_rpb, fx_nblk;   // x pass: rows per block, blocks
@@ -431,6 +441,10 @@ struct Group {
   int np_blocks = 0, pair_blocks = 0, list_blocks = 0, bricks = 0, kvec = 0, ncut = 0;
   int mesh_blocks = 0;   // blocks of 256 over the real mesh
   int fx_blocks = 0, fy_x = 0, fy_y = 0, fz_x = 0, fz_y = 0;
+  // the column passes of the replicas that take them: blocks, threads, LDS
+  // (fy_x, fz_x: the others')
+  int cy_blocks = 0, cz_blocks = 0, cy_thr = 0, cz_thr = 0;
+  size_t lds_cy = 0, lds_cz = 0;
   size_t lds_spread = 0, lds_gather = 0, lds_fx = 0, lds_fy = 0, lds_fz = 0;
   size_t lds_pair = 0;
   int pair_npt = 0;         // most types of any replica
@@ -735,6 +749,8 @@ const void *k_fm_spread_ptr();
 void fft_geometry(int prec, const int s[3], int *fx_rpb, int *fx_nblk, int *fy_T,
                   int *fy_nbx, int *fz_T, int *fz_nbx, size_t *lds_fx, size_t *lds_fy,
                   size_t *lds_fz);
+// the column plans of the y and z passes (ns = 0 where none)
+void column_plans(int prec, const int s[3], ColPlan *cy, ColPlan *cz);
 template <typename R, int O>
 const void *k_spread_ptr();
 template <typename R, int O>
