@@ -23,8 +23,8 @@ INCLUDE = os.path.join(ROOT, "include")
 BUILD = os.path.join(PKG, "_build")
 LIB = os.path.join(PKG, "libmfe.so")
 
-HIP_SOURCES = ["mfe_engine.hip", "mfe_kernels.hip", "mfe_fft.hip", "mfe_batch.hip",
-               "mfe_fm.hip"]
+HIP_SOURCES = ["mfe_engine.hip", "mfe_kernels.hip", "mfe_fft.hip", "mfe_fft_rows.hip",
+               "mfe_batch.hip", "mfe_fm.hip"]
 CXX_SOURCES = ["mfe_tables.cpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -64,7 +64,7 @@ def build(verbose: bool = False) -> str:
     for s in CXX_SOURCES:
         jobs.append((os.path.join(CSRC, s), os.path.join(BUILD, s + ".o"), "cxx"))
     from concurrent.futures import ThreadPoolExecutor
-    with ThreadPoolExecutor(max_workers=min(4, len(jobs))) as ex:
+    with ThreadPoolExecutor(max_workers=min(8, len(jobs))) as ex:
         objs = list(ex.map(_compile_one, jobs))
     tmp = LIB + ".tmp"
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp] + objs)

@@ -396,6 +396,7 @@ void mfe_fill_view(const mfe_engine *e, mfe::SysDev &v) {
     mfe::fft_geometry(e->prec, e->s, &v.fx_rpb, &v.fx_nblk, &v.fy_T, &v.fy_nbx, &v.fz_T,
                       &v.fz_nbx, &l0, &l1, &l2);
     mfe::column_plans(e->prec, e->s, &v.cy, &v.cz);
+    v.cx = mfe::row_plan(e->prec, e->s, e->B, e->order);
     v.f_s1 = mfe::make_fastdiv(e->s[0]);
     v.f_s2 = mfe::make_fastdiv(e->s[1]);
     v.f_s3 = mfe::make_fastdiv(e->s[2]);
@@ -503,7 +504,14 @@ int mfe_group_build(mfe_engine *const *eng, int R, const mfe::SysDev *d, hipStre
       g.bricks = std::max(g.bricks, e->nbricks);
       for (int m = 0; m < 3; ++m) g.mc_s[m] = std::max(g.mc_s[m], e->s[m]);
       g.mesh_blocks = std::max(g.mesh_blocks, (e->s[0] * e->s[1] * e->s[2] + 255) / 256);
-      g.fx_blocks = std::max(g.fx_blocks, fx_nblk);
+      const mfe::RowPlan cx = mfe::row_plan(e->prec, e->s, e->B, e->order);
+      if (cx.ns) {
+        g.cx_blocks = std::max(g.cx_blocks, cx.nblk);
+        g.cx_thr = std::max(g.cx_thr, cx.nthr);
+        g.lds_cx = std::max(g.lds_cx, (size_t)cx.lds);
+      } else {
+        g.fx_blocks = std::max(g.fx_blocks, fx_nblk);
+      }
       mfe::ColPlan cy, cz;
       mfe::column_plans(e->prec, e->s, &cy, &cz);
       if (cy.ns) {

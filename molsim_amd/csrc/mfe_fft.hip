@@ -11,9 +11,9 @@
 //                -- the z transform pair is fused around the pointwise
 //                product, so the mesh is not written between them
 //   y inverse, x inverse (c2r)
-// The y and z transforms run in registers with one LDS exchange per radix
-// after the first (col_fft) where the length has no prime factor above 7;
-// the x rows and other lengths are mixed-radix Stockham FFTs staged in LDS.
+// The transforms run in registers with one LDS exchange per radix after the
+// first (col_fft, rows_fwd, rows_inv) where the length has no prime factor
+// above 7; other lengths are mixed-radix Stockham FFTs staged in LDS.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -24,66 +24,7 @@
 namespace mfe {
 namespace {
 
-// The spread mesh at point (x, y, z): the point's value in its own brick's
-// spreading tile plus the low-side halo values of the next brick along each
-// axis (at most 8 tiles), added in a fixed order.  Tiles are the bricks
-// extended by order-1 points below (see k_spread).
-template <typename R>
-__device__ __forceinline__ R spread_point(const SysDev &V, const R *__restrict__ tiles, int x,
-                                          int y, int z) {
-  const SpmeGeom &g = V.sg;
-  const int h = g.order - 1;
-  const int E0 = g.B[0] + h, E1 = g.B[1] + h, E2 = g.B[2] + h;
-  const int bc0 = fdiv(x, g.fB[0]), bc1 = fdiv(y, g.fB[1]), bc2 = fdiv(z, g.fB[2]);
-  const int l0 = x - bc0 * g.B[0], l1 = y - bc1 * g.B[1], l2 = z - bc2 * g.B[2];
-  R acc = R(0);
-  for (int dz = 0; dz < 2; ++dz) {
-    if (dz && l2 < g.B[2] - h) break;
-    const int tz = dz ? (bc2 + 1 == g.nb[2] ? 0 : bc2 + 1) : bc2;
-    const int ez = l2 + h - dz * g.B[2];
-    for (int dy = 0; dy < 2; ++dy) {
-      if (dy && l1 < g.B[1] - h) break;
-      const int ty = dy ? (bc1 + 1 == g.nb[1] ? 0 : bc1 + 1) : bc1;
-      const int ey = l1 + h - dy * g.B[1];
-      for (int dx = 0; dx < 2; ++dx) {
-        if (dx && l0 < g.B[0] - h) break;
-        const int tx = dx ? (bc0 + 1 == g.nb[0] ? 0 : bc0 + 1) : bc0;
-        const int ex = l0 + h - dx * g.B[0];
-        const int t = tx + g.nb[0] * (ty + g.nb[1] * tz);
-        acc += tiles[(size_t)t * (E0 * E1 * E2) + (ez * E1 + ey) * E0 + ex];
-      }
-    }
-  }
-  return acc;
-}
-
 // ------------------------------------------------------------ pass kernels
-// The rows are read from the spreading tiles (the spread mesh is never
-// stored).
-template <typename R>
-__global__ void __launch_bounds__(256) k_fft_x_fwd(const SysDev *__restrict__ sys) {
-  const SysDev &V = sys[blockIdx.z];
-  // neighbouring rows (which read the same spreading tiles) on one XCD
-  const int blk = xcd_block(blockIdx.x, gridDim.x);
-  if (blk >= V.fx_nblk) return;
-  extern __shared__ char smem[];
-  const R *__restrict__ tiles = (const R *)V.spread_tiles;
-  const int nrows = V.sg.s[1] * V.sg.s[2], row0 = blk * V.fx_rpb;
-  fftx_fwd_rows<R>(V, row0, min(V.fx_rpb, nrows - row0), V.fx_rpb, smem,
-                   [&](int x, int y, int z) { return spread_point<R>(V, tiles, x, y, z); });
-}
-
-template <typename R>
-__global__ void __launch_bounds__(256) k_fft_x_inv(const SysDev *__restrict__ sys) {
-  const SysDev &V = sys[blockIdx.z];
-  // neighbouring rows (which the y inverse wrote together) on one XCD
-  const int blk = xcd_block(blockIdx.x, gridDim.x);
-  if (blk >= V.fx_nblk) return;
-  extern __shared__ char smem[];
-  const int nrows = V.sg.s[1] * V.sg.s[2], row0 = blk * V.fx_rpb;
-  fftx_inv_rows<R>(V, row0, min(V.fx_rpb, nrows - row0), V.fx_rpb, smem);
-}
-
 template <typename R>
 __global__ void __launch_bounds__(256) k_fft_y(const SysDev *__restrict__ sys, int inv) {
   const SysDev &V = sys[blockIdx.z];
@@ -262,17 +203,6 @@ inline int tile_width(int hx, int target) {
 }
 
 template <typename R>
-int rows_per_block(int s1) {
-  // two LDS buffers of rows*(s1/2+1) complex values, about 32 KB in all and
-  // at most 16 rows; at FP64 about 48 KB and at most 32 rows (23 rows of 128
-  // points measured faster there than 15, while FP32 is fastest at 16)
-  constexpr bool f64 = sizeof(R) == 8;
-  const int per_row = 2 * (s1 / 2 + 1) * (int)sizeof(cplx<R>);
-  const int rows = ((f64 ? 48 : 32) * 1024) / per_row, cap = f64 ? 32 : 16;
-  return rows < 1 ? 1 : (rows > cap ? cap : rows);
-}
-
-template <typename R>
 int tile_target(int n) {
   const int per_col = 2 * (n + 1) * (int)sizeof(cplx<R>);
   int t = (32 * 1024) / per_col;
@@ -287,15 +217,7 @@ void fft_geometry(int prec, const int s[3], int *fx_rpb, int *fx_nblk, int *fy_T
   const size_t csz = f ? sizeof(cplx<float>) : sizeof(cplx<double>);
   const size_t tsz = f ? sizeof(Twiddle<float>) : sizeof(Twiddle<double>);
   const int hx = s[0] / 2 + 1;
-  int rpb = f ? rows_per_block<float>(s[0]) : rows_per_block<double>(s[0]);
-  // the rows and the twiddles within 64 KB of LDS
-  while (rpb > 1 && 2 * (size_t)rpb * (s[0] / 2 + 1) * csz + (size_t)(s[0] / 2 + s[0]) * tsz >
-                        64 * 1024)
-    --rpb;
-  *fx_rpb = rpb;
-  *fx_nblk = (s[1] * s[2] + rpb - 1) / rpb;
-  // two row buffers, then the half- and full-length twiddles
-  *lds_fx = 2 * (size_t)rpb * (s[0] / 2 + 1) * csz + (size_t)(s[0] / 2 + s[0]) * tsz;
+  fft_row_geometry(prec, s, fx_rpb, fx_nblk, lds_fx);
   const int Ty = tile_width(hx, f ? tile_target<float>(s[1]) : tile_target<double>(s[1]));
   *fy_T = Ty;
   *fy_nbx = (hx + Ty - 1) / Ty;
@@ -306,51 +228,48 @@ void fft_geometry(int prec, const int s[3], int *fx_rpb, int *fx_nblk, int *fy_T
   *lds_fz = 2 * (size_t)Tz * (s[2] + 1) * csz + (size_t)s[2] * tsz;
 }
 
-// n as at most three radices of the column stages: the fewest, then the
-// smallest largest radix; false when n has none
-static bool col_radices(int n, int *ns, int r[3]) {
-  static const int rad[] = {16, 15, 14, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
-  auto one = [&](int m) {
+// n as at most three radices in descending order, the last (smallest) at
+// most `last`: the fewest, then the smallest largest one; false when n has
+// none
+bool fft_radices(int n, int last, int *ns, int r[3]) {
+  static const int rad[] = {2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 14, 15, 16};
+  auto is = [&](int m, int most) {
     for (int a : rad)
-      if (a == m) return true;
+      if (a == m) return m <= most;
     return false;
   };
-  if (one(n)) {
+  if (is(n, last)) {
     *ns = 1;
     r[0] = n;
     return true;
   }
-  int best = 0;
   for (int a : rad)
-    if (n % a == 0 && one(n / a) && n / a <= a && (!best || a < best)) {
-      best = a;
+    if (n % a == 0 && is(n / a, std::min(a, last))) {
       *ns = 2;
       r[0] = a;
       r[1] = n / a;
+      return true;
     }
-  if (best) return true;
   for (int a : rad)
     for (int b : rad)
-      if (b <= a && n % (a * b) == 0 && one(n / (a * b)) && n / (a * b) <= b &&
-          (!best || a < best)) {
-        best = a;
+      if (b <= a && n % (a * b) == 0 && is(n / (a * b), std::min(b, last))) {
         *ns = 3;
         r[0] = a;
         r[1] = b;
         r[2] = n / (a * b);
+        return true;
       }
-  return best != 0;
+  return false;
 }
 
 // Columns per block: 128 bytes of a row (16 FP32, 8 FP64), fewer where the
 // buffer (two for three stages) and the tables would pass 64 KB.  Threads
 // for one butterfly each of the smaller radix, at most 16 x 16, so that a
 // two-stage convolution exchanges within one buffer.
-constexpr size_t kColLds = 64 * 1024 - 256;  // beside conv_partials' static LDS
 static void column_plan(int n, int ncol, size_t csz, size_t tsz, bool conv,
                         ColPlan *p) {
   *p = ColPlan{};
-  if (!col_radices(n, &p->ns, p->r)) return;
+  if (!fft_radices(n, 16, &p->ns, p->r)) return;
   const int nbuf = p->ns == 3 ? 2 : 1;
   const size_t tab = (size_t)n * tsz + (conv ? 2 * (size_t)(n / 2 + 1) * sizeof(double) : 0);
   int lgT = csz == 8 ? 4 : 3;
@@ -378,20 +297,6 @@ void column_plans(int prec, const int s[3], ColPlan *cy, ColPlan *cz) {
   column_plan(s[2], s[1] * hx, csz, tsz, true, cz);
 }
 
-void fft_x_forward(const Group &g) {
-  const dim3 gr(g.fx_blocks, 1, g.R);
-  if (g.prec == MFE_PREC_MIXED)
-    hipLaunchKernelGGL(k_fft_x_fwd<float>, gr, dim3(256), g.lds_fx, g.stream, g.d);
-  else
-    hipLaunchKernelGGL(k_fft_x_fwd<double>, gr, dim3(256), g.lds_fx, g.stream, g.d);
-}
-void fft_x_inverse(const Group &g) {
-  const dim3 gr(g.fx_blocks, 1, g.R);
-  if (g.prec == MFE_PREC_MIXED)
-    hipLaunchKernelGGL(k_fft_x_inv<float>, gr, dim3(256), g.lds_fx, g.stream, g.d);
-  else
-    hipLaunchKernelGGL(k_fft_x_inv<double>, gr, dim3(256), g.lds_fx, g.stream, g.d);
-}
 void fft_y(const Group &g, int inverse) {
 #define MFE_Y(T)                                                                              \
   do {                                                                                        \

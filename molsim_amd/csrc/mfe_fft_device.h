@@ -2,7 +2,7 @@
 // (Src/energy.F90:6525-6587): complex arithmetic with compensated FP32
 // twiddles, the LDS-staged mixed-radix Stockham transform, and the passes
 // over one block's rows or tiles of one replica's mesh.  The pass kernels
-// (mfe_fft.hip) run one pass over many blocks; the persistent batched step
+// (mfe_fft.hip, mfe_fft_rows.hip) run one pass over many blocks; the persistent batched step
 // (mfe_kernels.hip) runs all passes of a replica in one workgroup.
 #pragma once
 
@@ -538,6 +538,204 @@ __device__ __forceinline__ void col_conv(const ColPlan &p, int nt, cplx<R> *A, c
   any_stage<R, true, ST_MID>(p.r[1], n, lgT, nt, p.r[2], tw, get(A), put(B));
   __syncthreads();
   any_stage<R, true, ST_LAST>(p.r[0], n, lgT, nt, p.r[2] * p.r[1], tw, get(B), wr);
+}
+
+// --------------------------------------------------- x rows in registers
+// The r2c and c2r transforms of rows of s1 = 2m reals through a complex
+// transform of length m (fftx_fwd_rows has the formulas), with the radices
+// of col_fft: butterfly j of row c, j fastest over the threads.  The pass
+// that combines Z[k] with Z[m-k] takes the butterflies j and Ns - j of the
+// forward transform's last stage (the inverse's first) in one thread, whose
+// outputs (inputs) j + q Ns and m - (j + q Ns) then pair up in registers.
+// Both ends of that pair of stages take the plan's smallest radix, at most
+// 8 (two butterflies are held at once); the inverse runs the radices in
+// reverse order.
+//
+// Outputs of butterfly j (nb butterflies in all) are Z[j + q nb]; with j2 = nb - j the partner of
+// element q is element RAD-1-q of the sequence j2 + i nb.  For j = 0 that
+// sequence is nb, 2 nb, ..., m (Z[m] = Z[0]).
+#define MFE_FOR_RADIX8(r, CALL) \
+  switch (r) {                  \
+    case 2: CALL(2); break;     \
+    case 3: CALL(3); break;     \
+    case 4: CALL(4); break;     \
+    case 5: CALL(5); break;     \
+    case 6: CALL(6); break;     \
+    case 7: CALL(7); break;     \
+    default: CALL(8); break;    \
+  }
+template <typename R, int RAD>
+__device__ __forceinline__ void r2c_stage(const RowPlan &p, int nr, const Twiddle<R> *twh,
+                                          const Twiddle<R> *twf, const cplx<R> *in,
+                                          cplx<R> *__restrict__ out) {
+  const int m = p.m, nb = m / RAD, np = nb / 2 + 1, hx = m + 1;
+  for (int t = threadIdx.x; t < nr * np; t += blockDim.x) {
+    const int c = fdiv(t, p.f_pair), j = t - c * np;
+    const bool self = j == 0 || 2 * j == nb;
+    const cplx<R> *row = in + c * p.ld;
+    cplx<R> v[RAD], u[RAD];
+    auto butterfly = [&](cplx<R> *w, int jj) {
+#pragma unroll
+      for (int q = 0; q < RAD; ++q) w[q] = row[jj + q * nb];
+      if (nb > 1) {
+#pragma unroll
+        for (int q = 1; q < RAD; ++q) w[q] = twmul(w[q], twh[jj * q], false);
+      }
+      reg_dft<R, RAD, false>(w);
+    };
+    butterfly(v, j);
+    if (!self) {
+      butterfly(u, nb - j);
+    } else {
+#pragma unroll
+      for (int q = 0; q < RAD; ++q) u[q] = j == 0 ? v[(q + 1) % RAD] : v[q];
+    }
+    cplx<R> *orow = out + (size_t)c * hx;
+    auto put = [&](cplx<R> zk, cplx<R> zmk, int k) {
+      const cplx<R> zm = conjc(zmk);
+      const cplx<R> ev = {(zk.x + zm.x) * R(0.5), (zk.y + zm.y) * R(0.5)};
+      const cplx<R> d = csub(zk, zm);
+      const cplx<R> od = {d.y * R(0.5), -d.x * R(0.5)};
+      orow[k] = cadd(ev, twmul(od, twf[k], false));
+    };
+#pragma unroll
+    for (int q = 0; q < RAD; ++q) put(v[q], u[RAD - 1 - q], j + q * nb);
+    if (!self) {
+#pragma unroll
+      for (int q = 0; q < RAD; ++q) put(u[q], v[RAD - 1 - q], nb - j + q * nb);
+    }
+    if (j == 0) put(v[0], v[0], m);
+  }
+}
+
+// the inverse's first stage: X of a row from global memory, Z and its
+// butterflies j and nb - j, written to positions j RAD + q by wr(pos, c, v)
+template <typename R, int RAD, typename Wr>
+__device__ __forceinline__ void c2r_stage(const RowPlan &p, int nr, const Twiddle<R> *twf,
+                                          const cplx<R> *__restrict__ in, Wr wr) {
+  const int m = p.m, nb = m / RAD, np = nb / 2 + 1, hx = m + 1;
+  for (int t = threadIdx.x; t < nr * np; t += blockDim.x) {
+    const int c = fdiv(t, p.f_pair), j = t - c * np;
+    const bool self = j == 0 || 2 * j == nb;
+    const cplx<R> *row = in + (size_t)c * hx;
+    cplx<R> x[RAD], y[RAD];
+#pragma unroll
+    for (int q = 0; q < RAD; ++q) {
+      x[q] = row[j + q * nb];
+      y[q] = row[nb - j + q * nb];
+    }
+    if (j == 0) {
+      // Re(X[0]) and Re(X[m]) only
+      x[0].y = R(0);
+      y[RAD - 1].y = R(0);
+    }
+    auto pre = [&](cplx<R> xk, cplx<R> xmk, int k) -> cplx<R> {
+      const cplx<R> xm = conjc(xmk);
+      const cplx<R> A = cadd(xk, xm), D = csub(xk, xm);
+      const cplx<R> Dw = twmul(D, twf[k], true);
+      return {A.x - Dw.y, A.y + Dw.x};
+    };
+    cplx<R> z[RAD];
+#pragma unroll
+    for (int q = 0; q < RAD; ++q) z[q] = pre(x[q], y[RAD - 1 - q], j + q * nb);
+    reg_dft<R, RAD, true>(z);
+#pragma unroll
+    for (int q = 0; q < RAD; ++q) wr(j * RAD + q, c, z[q]);
+    if (!self) {
+#pragma unroll
+      for (int q = 0; q < RAD; ++q) z[q] = pre(y[q], x[RAD - 1 - q], nb - j + q * nb);
+      reg_dft<R, RAD, true>(z);
+#pragma unroll
+      for (int q = 0; q < RAD; ++q) wr((nb - j) * RAD + q, c, z[q]);
+    }
+  }
+}
+
+// a plain stage of the rows: as col_stage with j fastest (st: the stage's
+// place in the plan, whose butterflies per row are p.f_nb[st].d)
+template <typename R, int RAD, bool INV, int POS, typename Rd, typename Wr>
+__device__ __forceinline__ void row_stage(const RowPlan &p, int nr, int st, int Ns,
+                                          const Twiddle<R> *tw, Rd rd, Wr wr) {
+  const int n = p.m, nb = n / RAD, step = POS == ST_FIRST ? 1 : Ns;
+  for (int t = threadIdx.x; t < nr * nb; t += blockDim.x) {
+    const int c = fdiv(t, p.f_nb[st]), j = t - c * nb;
+    cplx<R> v[RAD];
+#pragma unroll
+    for (int q = 0; q < RAD; ++q) v[q] = rd(j + q * nb, c);
+    int base;
+    stage_twiddle<R, RAD, INV, POS>(v, j, n, Ns, base, tw);
+    reg_dft<R, RAD, INV>(v);
+#pragma unroll
+    for (int q = 0; q < RAD; ++q) wr(base + q * step, c, v[q]);
+  }
+}
+template <typename R, bool INV, int POS, typename Rd, typename Wr>
+__device__ __forceinline__ void any_row_stage(const RowPlan &p, int nr, int st, int Ns,
+                                              const Twiddle<R> *tw, Rd rd, Wr wr) {
+#define MFE_CALL(RAD) row_stage<R, RAD, INV, POS>(p, nr, st, Ns, tw, rd, wr)
+  MFE_FOR_RADIX(p.r[st], MFE_CALL)
+#undef MFE_CALL
+}
+
+// forward: nr rows of reals in A (row c at 2 c ld), transformed into out
+// ([nr][m + 1]); B a second buffer of the same size
+template <typename R>
+__device__ __forceinline__ void rows_fwd(const RowPlan &p, int nr, cplx<R> *A, cplx<R> *B,
+                                         const Twiddle<R> *twh, const Twiddle<R> *twf,
+                                         cplx<R> *__restrict__ out) {
+  const int ld = p.ld;
+  auto get = [=](const cplx<R> *b) { return [=](int pos, int c) { return b[c * ld + pos]; }; };
+  auto put = [=](cplx<R> *b) {
+    return [=](int pos, int c, cplx<R> v) { b[c * ld + pos] = v; };
+  };
+  int Ns = 1;
+  if (p.ns >= 2) {
+    any_row_stage<R, false, ST_FIRST>(p, nr, 0, 1, twh, get(A), put(B));
+    __syncthreads();
+    cplx<R> *x = A;
+    A = B;
+    B = x;
+    Ns = p.r[0];
+  }
+  if (p.ns == 3) {
+    any_row_stage<R, false, ST_MID>(p, nr, 1, Ns, twh, get(A), put(B));
+    __syncthreads();
+    A = B;
+  }
+#define MFE_CALL(RAD) r2c_stage<R, RAD>(p, nr, twh, twf, A, out)
+  MFE_FOR_RADIX8(p.r[p.ns - 1], MFE_CALL)
+#undef MFE_CALL
+}
+
+// inverse: nr rows of in ([nr][m + 1]) into reals, written as pairs by
+// wr(k, c, {x[2k], x[2k+1]})
+template <typename R, typename Wr>
+__device__ __forceinline__ void rows_inv(const RowPlan &p, int nr, cplx<R> *A, cplx<R> *B,
+                                         const Twiddle<R> *twh, const Twiddle<R> *twf,
+                                         const cplx<R> *__restrict__ in, Wr wr) {
+  const int ld = p.ld;
+  auto get = [=](const cplx<R> *b) { return [=](int pos, int c) { return b[c * ld + pos]; }; };
+  auto put = [=](cplx<R> *b) {
+    return [=](int pos, int c, cplx<R> v) { b[c * ld + pos] = v; };
+  };
+  if (p.ns == 1) {
+#define MFE_CALL(RAD) c2r_stage<R, RAD>(p, nr, twf, in, wr)
+    MFE_FOR_RADIX8(p.r[0], MFE_CALL)
+#undef MFE_CALL
+    return;
+  }
+#define MFE_CALL(RAD) c2r_stage<R, RAD>(p, nr, twf, in, put(A))
+  MFE_FOR_RADIX8(p.r[p.ns - 1], MFE_CALL)
+#undef MFE_CALL
+  __syncthreads();
+  int Ns = p.r[p.ns - 1];
+  if (p.ns == 3) {
+    any_row_stage<R, true, ST_MID>(p, nr, 1, Ns, twh, get(A), put(B));
+    __syncthreads();
+    A = B;
+    Ns *= p.r[1];
+  }
+  any_row_stage<R, true, ST_LAST>(p, nr, 0, Ns, twh, get(A), wr);
 }
 
 // ----------------------------------------------------------------- x pass

@@ -193,6 +193,32 @@ struct ColPlan {
   int lds;   // bytes of dynamic LDS
 };
 
+// Division by a divisor d fixed at set-up: q = (n * ceil(2^32 / d)) >> 32,
+// exact for 0 <= n with n * d < 2^32 (the error term n * e / 2^32, e < d,
+// stays below 1/d).  One 64-bit multiply instead of the ~25 instructions
+// of a run-time integer division.
+struct FastDiv {
+  unsigned long long m;
+  int d;
+};
+inline FastDiv make_fastdiv(int d) {
+  return FastDiv{((1ull << 32) + (unsigned long long)d - 1) / (unsigned long long)d, d};
+}
+__host__ __device__ __forceinline__ int fdiv(int n, const FastDiv &f) {
+  return (int)(((unsigned long long)(unsigned)n * f.m) >> 32);
+}
+
+// Row transforms in registers (rows_fwd, rows_inv): half length m = s1/2 as
+// ns <= 3 radices, nr rows and nthr threads per block, LDS rows of ld
+// complex values; ns = 0 as in ColPlan (the rows then go through LDS,
+// fftx_fwd_rows and fftx_inv_rows).
+struct RowPlan {
+  int m, ns, r[3], nr, nthr, nblk, ld;
+  int lds;               // bytes of dynamic LDS
+  FastDiv f_nb[3];       // butterflies per row of each stage, m / r
+  FastDiv f_pair;        // pairs of butterflies per row of the last radix
+};
+
 // Per-axis SPME tables (FP64): g[n] = b2[n]*exp(-k_n^2/(4 alpha^2)) and
 // kk[n] = k_n^2 for n = 0..s/2, so that
 // meshfac(nx,ny,nz) = fac0 * gx*gy*gz / (kkx+kky+kkz)  (Essmann eq. 3.9).
@@ -212,22 +238,6 @@ struct PairParams {
   int lewald, lljcut;
 };
 
-// SPME mesh geometry: mesh s, spreading bricks B (nb per axis), dkdr = s/L.
-// Division by a divisor d fixed at set-up: q = (n * ceil(2^32 / d)) >> 32,
-// exact for 0 <= n with n * d < 2^32 (the error term n * e / 2^32, e < d,
-// stays below 1/d).  One 64-bit multiply instead of the ~25 instructions
-// of a run-time integer division.
-struct FastDiv {
-  unsigned long long m;
-  int d;
-};
-inline FastDiv make_fastdiv(int d) {
-  return FastDiv{((1ull << 32) + (unsigned long long)d - 1) / (unsigned long long)d, d};
-}
-__host__ __device__ __forceinline__ int fdiv(int n, const FastDiv &f) {
-  return (int)(((unsigned long long)(unsigned)n * f.m) >> 32);
-}
-
 // Blocks are dispatched to the 8 XCDs round-robin (block b on XCD b % 8),
 // each XCD with its own L2.  This maps them to logical blocks so that each
 // XCD takes one contiguous range, whose data (positions of a slab of the
@@ -238,6 +248,7 @@ __device__ __forceinline__ int xcd_block(int b, int nblk) {
   return x < r ? x * (q + 1) + k : r * (q + 1) + (x - r) * q + k;
 }
 
+// SPME mesh geometry: mesh s, spreading bricks B (nb per axis), dkdr = s/L.
 struct SpmeGeom {
   int s[3], B[3], nb[3], order;
   double dkdr[3];
@@ -308,6 +319,7 @@ struct SysDev {
   SpmeAxes ax;
   FftPlan plan[3], plan_half;
   ColPlan cy, cz;        // y and z passes
+  RowPlan cx;            // x passes
   MFE_DPTR(const void) tw[3];
   MFE_DPTR(const void) tw_half;
   int fx_rpb, fx_nblk;   // x pass: rows per block, blocks
@@ -443,8 +455,8 @@ struct Group {
   int fx_blocks = 0, fy_x = 0, fy_y = 0, fz_x = 0, fz_y = 0;
   // the column passes of the replicas that take them: blocks, threads, LDS
   // (fy_x, fz_x: the others')
-  int cy_blocks = 0, cz_blocks = 0, cy_thr = 0, cz_thr = 0;
-  size_t lds_cy = 0, lds_cz = 0;
+  int cx_blocks = 0, cy_blocks = 0, cz_blocks = 0, cx_thr = 0, cy_thr = 0, cz_thr = 0;
+  size_t lds_cx = 0, lds_cy = 0, lds_cz = 0;
   size_t lds_spread = 0, lds_gather = 0, lds_fx = 0, lds_fy = 0, lds_fz = 0;
   size_t lds_pair = 0;
   int pair_npt = 0;         // most types of any replica
@@ -745,12 +757,18 @@ void launch_fm_acc(const Group &g, const double *part, int nblk, int ncol, int c
 template <typename R, int O>
 const void *k_fm_spread_ptr();
 
-// per-replica launch geometry of the FFT passes (mfe_fft.hip)
+// n as at most three radices in descending order, the last at most `last`
+bool fft_radices(int n, int last, int *ns, int r[3]);
+// dynamic LDS of a transform's block beside its static arrays
+constexpr size_t kColLds = 64 * 1024 - 256;
+// per-replica launch geometry of the FFT passes (mfe_fft.hip, mfe_fft_rows.hip)
+void fft_row_geometry(int prec, const int s[3], int *fx_rpb, int *fx_nblk, size_t *lds_fx);
 void fft_geometry(int prec, const int s[3], int *fx_rpb, int *fx_nblk, int *fy_T,
                   int *fy_nbx, int *fz_T, int *fz_nbx, size_t *lds_fx, size_t *lds_fy,
                   size_t *lds_fz);
-// the column plans of the y and z passes (ns = 0 where none)
+// the plans of the x, y and z passes in registers (ns = 0 where none)
 void column_plans(int prec, const int s[3], ColPlan *cy, ColPlan *cz);
+RowPlan row_plan(int prec, const int s[3], const int B[3], int order);
 template <typename R, int O>
 const void *k_spread_ptr();
 template <typename R, int O>

@@ -1313,7 +1313,7 @@ __global__ void k_spme_clear(const SysDev *__restrict__ sys) {
 // order-1 points on the low side of each axis, then writes the tile to a
 // scratch array.  The forward x FFT reads each mesh point as its own
 // brick's tile value plus the low-side halos of the next bricks (at most 8
-// tiles) in a fixed order (spread_point in mfe_fft.hip).  Work is handed
+// tiles) in a fixed order (spread_point in mfe_fft_rows.hip).  Work is handed
 // out as (particle, stencil plane) items, order planes per particle; each
 // item computes the particle's B-splines in registers (no staging, no
 // barrier between particles) and loads the record of its next item before
