@@ -29,32 +29,6 @@ __device__ __forceinline__ double pbcr2(double &dx, double &dy, double &dz,
   return r2;
 }
 
-// Block-wide sum (max) in a fixed order: a shuffle tree inside each
-// wavefront, then the wavefront results in wavefront order.  Every thread
-// gets the result; sh needs one slot per wavefront.
-template <typename T>
-__device__ __forceinline__ T block_sum(T v, T *sh) {
-  for (int w = 32; w > 0; w >>= 1) v += __shfl_down(v, w, 64);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) sh[wave] = v;
-  __syncthreads();
-  T r = sh[0];
-  for (int k = 1; k < (int)(blockDim.x >> 6); ++k) r += sh[k];
-  return r;
-}
-
-__device__ __forceinline__ double block_max(double v, double *sh) {
-  for (int w = 32; w > 0; w >>= 1) v = fmax(v, __shfl_down(v, w, 64));
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) sh[wave] = v;
-  __syncthreads();
-  double r = sh[0];
-  for (int k = 1; k < (int)(blockDim.x >> 6); ++k) r = fmax(r, sh[k]);
-  return r;
-}
-
 // The partner value of an FP64 register in a lane quad, by DPP (no LDS):
 // kXor1 swaps lanes 0<->1 and 2<->3, kXor2 swaps 0<->2 and 1<->3 -- the
 // exchanges of __shfl_xor(x, 1 or 2) within a quad.  Every lane of the
@@ -86,26 +60,63 @@ __device__ __forceinline__ double wave_sum(double x) {
   return (read_lane(x, 0) + read_lane(x, 16)) + (read_lane(x, 32) + read_lane(x, 48));
 }
 
-// ------------------------------------------------- spline pair term
-// Uniform cubic B-spline on knots r0 + k/dinv: on interval i (fraction f)
-// the weights of coefficients i..i+3 are (1-f)^3/6, (3f^3-6f^2+4)/6,
-// (-3f^3+3f^2+3f+1)/6, f^3/6 (de Boor, A Practical Guide to Splines, ch. IX),
-// and their derivatives in f.
-__device__ __forceinline__ bool knot_weights(double r, double r0, double dinv, int nknot,
-                                             int &i, double w[4], double dw[4]) {
-  const double x = (r - r0) * dinv;
-  if (!(x >= 0.0) || !(x < (double)(nknot - 3))) return false;
-  i = (int)x;
-  const double f = x - i, f2 = f * f, f3 = f2 * f, g = 1.0 - f;
-  w[0] = g * g * g / 6.0;
-  w[1] = (3.0 * f3 - 6.0 * f2 + 4.0) / 6.0;
-  w[2] = (-3.0 * f3 + 3.0 * f2 + 3.0 * f + 1.0) / 6.0;
-  w[3] = f3 / 6.0;
-  dw[0] = -0.5 * g * g;
-  dw[1] = 1.5 * f2 - 2.0 * f;
-  dw[2] = -1.5 * f2 + f + 0.5;
-  dw[3] = 0.5 * f2;
-  return true;
+// Block-wide sum (max) in a fixed order: wave_sum (a shuffle tree) inside
+// each wavefront, then the wavefront results in wavefront order.  Every thread
+// gets the result; sh needs one slot per wavefront.
+__device__ __forceinline__ double block_sum(double v, double *sh) {
+  v = wave_sum(v);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __syncthreads();
+  if (lane == 0) sh[wave] = v;
+  __syncthreads();
+  double r = sh[0];
+  for (int k = 1; k < (int)(blockDim.x >> 6); ++k) r += sh[k];
+  return r;
+}
+
+__device__ __forceinline__ double block_max(double v, double *sh) {
+  for (int w = 32; w > 0; w >>= 1) v = fmax(v, __shfl_down(v, w, 64));
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __syncthreads();
+  if (lane == 0) sh[wave] = v;
+  __syncthreads();
+  double r = sh[0];
+  for (int k = 1; k < (int)(blockDim.x >> 6); ++k) r = fmax(r, sh[k]);
+  return r;
+}
+
+// out[c] (+)= sum over rows b of part[b * ncol + c], c < cols, in a fixed
+// order: a block of 1024 threads takes 16 columns (128 bytes of a row) in 64
+// slices of rows, eight loads in flight per thread, then the slices in order.
+// 391 columns of 1032 rows: 6 us (a thread per column walked the rows one
+// load after another: 63-101 us).  Grid: (cols + 15) / 16 blocks.
+constexpr int kSumCols = 16, kSumThreads = 1024;
+__device__ __forceinline__ void column_sums(const double *__restrict__ part, int rows, int ncol,
+                                            int cols, double *__restrict__ out, bool add) {
+  constexpr int kSlices = kSumThreads / kSumCols, kU = 8;
+  __shared__ double sh[kSlices][kSumCols];
+  const int cl = threadIdx.x % kSumCols, sl = threadIdx.x / kSumCols;
+  const int c = blockIdx.x * kSumCols + cl;
+  double s = 0.0;
+  if (c < cols) {
+    for (int b0 = sl; b0 < rows; b0 += kU * kSlices) {
+      double v[kU];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        const int b = b0 + u * kSlices;
+        v[u] = b < rows ? part[(size_t)b * ncol + c] : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < kU; ++u) s += v[u];
+    }
+  }
+  sh[sl][cl] = s;
+  __syncthreads();
+  if (sl == 0 && c < cols) {
+    double t = 0.0;
+    for (int k = 0; k < kSlices; ++k) t += sh[k][cl];
+    out[c] = add ? out[c] + t : t;
+  }
 }
 
 struct KahanF {
@@ -140,6 +151,28 @@ __device__ __forceinline__ R div_small(R a) {
     const double r = __builtin_fma(-q, double(D), a);
     return __builtin_fma(r, inv, q);
   }
+}
+
+// ------------------------------------------------- spline pair term
+// Uniform cubic B-spline on knots r0 + k/dinv: on interval i (fraction f)
+// the weights of coefficients i..i+3 are (1-f)^3/6, (3f^3-6f^2+4)/6,
+// (-3f^3+3f^2+3f+1)/6, f^3/6 (de Boor, A Practical Guide to Splines, ch. IX),
+// and their derivatives in f.
+__device__ __forceinline__ bool knot_weights(double r, double r0, double dinv, int nknot,
+                                             int &i, double w[4], double dw[4]) {
+  const double x = (r - r0) * dinv;
+  if (!(x >= 0.0) || !(x < (double)(nknot - 3))) return false;
+  i = (int)x;
+  const double f = x - i, f2 = f * f, f3 = f2 * f, g = 1.0 - f;
+  w[0] = div_small<double, 6>(g * g * g);
+  w[1] = div_small<double, 6>(3.0 * f3 - 6.0 * f2 + 4.0);
+  w[2] = div_small<double, 6>(-3.0 * f3 + 3.0 * f2 + 3.0 * f + 1.0);
+  w[3] = div_small<double, 6>(f3);
+  dw[0] = -0.5 * g * g;
+  dw[1] = 1.5 * f2 - 2.0 * f;
+  dw[2] = -1.5 * f2 + f + 0.5;
+  dw[3] = 0.5 * f2;
+  return true;
 }
 
 // stages n = N..ORDER of the Schoenberg recursion (compile-time n, so the

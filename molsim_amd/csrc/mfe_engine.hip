@@ -1910,7 +1910,7 @@ int mfe_adjoint(mfe_engine *e, double *dE_dq, double *dE_dzat, double *dE_dsigat
   return guarded(e, [&]() -> int {
     MFE_HIP_TRY(hipSetDevice(e->device));
     const int ncol = 1 + 2 * e->npt + e->nptpt * e->nknot;
-    const int nb = (e->np + 255) / 256;
+    const int nb = mfe::adjoint_blocks(e->np);
     if (!e->adj_phi || e->adj_cap < nb * ncol) {
       dalloc(e->phi_rec, (size_t)e->max_np);
       dalloc(e->adj_phi, (size_t)e->max_np);

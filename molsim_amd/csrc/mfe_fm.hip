@@ -43,6 +43,7 @@ namespace {
 
 // lanes sharing one particle's list in the model pair kernel
 constexpr int kFmLanes = 4;
+constexpr int kFmBatch = 4;  // list entries a lane loads together
 constexpr int kFmBlock = 256;
 
 template <typename R>
@@ -75,6 +76,9 @@ __device__ __forceinline__ double quad_sum(double x) {
 // where g = f_coul / (q_i q_j efp) -- each pair is seen from both ends, so
 // the per-type terms carry half of the pair's share each time.  Block
 // partials [dsig(npt), deps(npt), dc(nptpt*nknot)] at part[blk * ncol].
+// Bound by the loads of the partners and the model's special functions;
+// 66000 particles with 117 partners, FP32: forces 103 -> 82 us, gradients
+// 117 -> 104 with four entries of a lane in flight together.
 template <typename R, bool BWD>
 __global__ void __launch_bounds__(kFmBlock) k_fm_pair(const SysDev *__restrict__ sys,
                                                       double *__restrict__ part, int ncol) {
@@ -85,11 +89,20 @@ __global__ void __launch_bounds__(kFmBlock) k_fm_pair(const SysDev *__restrict__
   extern __shared__ double sk[];
   __shared__ double sh[kFmBlock / 64];
   const int nk = V.nptpt * V.nknot;
-  if (BWD) {
-    for (int k = threadIdx.x; k < nk; k += blockDim.x) sk[k] = 0.0;
-    __syncthreads();
-  }
+  // the types' parameters and pair indices in LDS (read per entry by the
+  // partner's type)
+  __shared__ R zat_s[MFE_MAX_TYPES], sig_s[MFE_MAX_TYPES], eps_s[MFE_MAX_TYPES];
+  __shared__ int pidx_s[MFE_MAX_TYPES * MFE_MAX_TYPES];
   const PairParams &pp = V.pp;
+  for (int k = threadIdx.x; k < V.npt; k += blockDim.x) {
+    zat_s[k] = (R)pp.zat[k];
+    sig_s[k] = (R)pp.sigat[k];
+    eps_s[k] = (R)pp.epsat[k];
+  }
+  for (int k = threadIdx.x; k < V.npt * V.npt; k += blockDim.x) pidx_s[k] = V.tab.pairidx[k];
+  if (BWD)
+    for (int k = threadIdx.x; k < nk; k += blockDim.x) sk[k] = 0.0;
+  __syncthreads();
   const TableDev &t = V.tab;
   const Box b = V.box;
   const int lane = threadIdx.x % kFmLanes;
@@ -103,7 +116,7 @@ __global__ void __launch_bounds__(kFmBlock) k_fm_pair(const SysDev *__restrict__
   if (act) {
     const double xi = V.ro_s[3 * tt], yi = V.ro_s[3 * tt + 1], zi = V.ro_s[3 * tt + 2];
     ti = V.type_s[tt];
-    const R qi = (R)pp.zat[ti], si = (R)pp.sigat[ti], ei = (R)pp.epsat[ti];
+    const R qi = zat_s[ti], si = sig_s[ti], ei = eps_s[ti];
     R rxi = 0, ryi = 0, rzi = 0;
     if (BWD) {
       rxi = (R)V.fm_res_s[3 * tt];
@@ -111,66 +124,94 @@ __global__ void __launch_bounds__(kFmBlock) k_fm_pair(const SysDev *__restrict__
       rzi = (R)V.fm_res_s[3 * tt + 2];
     }
     const int n = V.nn[tt];
-    for (int k = lane; k < n; k += kFmLanes) {
-      const int pj = (int)((unsigned)V.nbr[(size_t)k * np + tt] & kNbrIdxMask);
-      double dx = xi - V.ro_s[3 * pj], dy = yi - V.ro_s[3 * pj + 1], dz = zi - V.ro_s[3 * pj + 2];
-      const double r2d = pbcr2(dx, dy, dz, b);
-      if (V.nlsem == 0 ? (r2d > t.rcut2) : !(r2d < t.rcut2)) continue;
-      const int tj = V.type_s[pj];
-      const R r2 = (R)r2d, r = sqrt(r2);
-      const R dxr = (R)dx, dyr = (R)dy, dzr = (R)dz;
-      const R qj = (R)pp.zat[tj];
-      // Coulomb: f = q_i q_j efp g(r)
-      R g;
-      if (pp.lewald) {
-        const R ar = alpha * r;
-        g = (erfc_r<R>(ar) / r + two_a_pi * exp_r<R>(-ar * ar)) / r2;
-      } else {
-        g = R(1) / (r * r2);
+    // kFmBatch entries' indices, then their positions, in flight together
+    // (rows clamped into the list; past its end the particle itself)
+    for (int k0 = lane; k0 < n; k0 += kFmBatch * kFmLanes) {
+      int pjs[kFmBatch], tjs[kFmBatch];
+      double xs[kFmBatch], ys[kFmBatch], zs[kFmBatch];
+#pragma unroll
+      for (int u = 0; u < kFmBatch; ++u) {
+        const int k = k0 + u * kFmLanes;
+        const int e = (int)((unsigned)V.nbr[(size_t)min(k, n - 1) * np + tt] & kNbrIdxMask);
+        pjs[u] = k < n ? e : tt;
       }
-      R f = qi * qj * efp * g;
-      // Lennard-Jones inside the WCA cut
-      const R sig = R(0.5) * (si + (R)pp.sigat[tj]);
-      const R ej = (R)pp.epsat[tj];
-      const R eps = sqrt(ei * ej);
-      R fs = 0, fe = 0;
-      if (!pp.lljcut || r < (R)pp.ljrcut * sig) {
-        const R x = sig / r, x2 = x * x, s6 = x2 * x2 * x2, s12 = s6 * s6;
-        fe = R(24) * (R(2) * s12 - s6) / r2;      // df/deps_ij
-        f += eps * fe;
-        fs = R(144) * eps * (R(4) * s12 - s6) / (sig * r2);  // df/dsig_ij
+#pragma unroll
+      for (int u = 0; u < kFmBatch; ++u) {
+        xs[u] = V.ro_s[3 * pjs[u]];
+        ys[u] = V.ro_s[3 * pjs[u] + 1];
+        zs[u] = V.ro_s[3 * pjs[u] + 2];
+        tjs[u] = V.type_s[pjs[u]];
       }
-      // spline term (FP64: few pairs, exact weights)
-      int ki = 0;
-      double w4[4], dw4[4];
-      bool kn = false;
-      int pidx = 0;
-      if (V.nknot) {
-        kn = knot_weights((double)r2d > 0.0 ? sqrt(r2d) : 0.0, V.knot_r0, V.knot_dinv, V.nknot,
-                          ki, w4, dw4);
-        if (kn) {
-          pidx = t.pairidx[ti * t.npt + tj];
-          if (!BWD) {
-            const double *c = V.knot_c + (size_t)pidx * V.nknot + ki;
-            const double dup =
-                (c[0] * dw4[0] + c[1] * dw4[1] + c[2] * dw4[2] + c[3] * dw4[3]) * V.knot_dinv;
-            f += (R)(-dup / sqrt(r2d));
-          }
+      R rxs[kFmBatch], rys[kFmBatch], rzs[kFmBatch];
+      if (BWD) {
+#pragma unroll
+        for (int u = 0; u < kFmBatch; ++u) {
+          rxs[u] = (R)V.fm_res_s[3 * pjs[u]];
+          rys[u] = (R)V.fm_res_s[3 * pjs[u] + 1];
+          rzs[u] = (R)V.fm_res_s[3 * pjs[u] + 2];
         }
       }
-      if (!BWD) {
-        fx += (double)(f * dxr);
-        fy += (double)(f * dyr);
-        fz += (double)(f * dzr);
-      } else {
-        const R w = (rxi - (R)V.fm_res_s[3 * pj]) * dxr + (ryi - (R)V.fm_res_s[3 * pj + 1]) * dyr +
-                    (rzi - (R)V.fm_res_s[3 * pj + 2]) * dzr;
-        dq += (double)(R(2) * efp * qj * g * w);
-        gs += (double)(w * fs);
-        if (eps > R(0)) ge += (double)(w * fe * ej / eps);
-        if (kn) {
-          const double wr = (double)w * V.knot_dinv / sqrt(r2d);
-          for (int m = 0; m < 4; ++m) atomicAdd(&sk[pidx * V.nknot + ki + m], -wr * dw4[m]);
+#pragma unroll
+      for (int u = 0; u < kFmBatch; ++u) {
+        if (k0 + u * kFmLanes >= n) break;
+        double dx = xi - xs[u], dy = yi - ys[u], dz = zi - zs[u];
+        const double r2d = pbcr2(dx, dy, dz, b);
+        if (V.nlsem == 0 ? (r2d > t.rcut2) : !(r2d < t.rcut2)) continue;
+        const int tj = tjs[u];
+        const R r2 = (R)r2d, r = sqrt(r2);
+        const R dxr = (R)dx, dyr = (R)dy, dzr = (R)dz;
+        const R qj = zat_s[tj];
+        // Coulomb: f = q_i q_j efp g(r)
+        R g;
+        if (pp.lewald) {
+          const R ar = alpha * r;
+          g = (erfc_r<R>(ar) / r + two_a_pi * exp_r<R>(-ar * ar)) / r2;
+        } else {
+          g = R(1) / (r * r2);
+        }
+        R f = qi * qj * efp * g;
+        // Lennard-Jones inside the WCA cut
+        const R sig = R(0.5) * (si + sig_s[tj]);
+        const R ej = eps_s[tj];
+        const R eps = sqrt(ei * ej);
+        R fs = 0, fe = 0;
+        if (!pp.lljcut || r < (R)pp.ljrcut * sig) {
+          const R x = sig / r, x2 = x * x, s6 = x2 * x2 * x2, s12 = s6 * s6;
+          fe = R(24) * (R(2) * s12 - s6) / r2;      // df/deps_ij
+          f += eps * fe;
+          fs = R(144) * eps * (R(4) * s12 - s6) / (sig * r2);  // df/dsig_ij
+        }
+        // spline term (FP64: few pairs, exact weights)
+        int ki = 0;
+        double w4[4], dw4[4];
+        bool kn = false;
+        int pidx = 0;
+        if (V.nknot) {
+          kn = knot_weights((double)r2d > 0.0 ? sqrt(r2d) : 0.0, V.knot_r0, V.knot_dinv, V.nknot,
+                            ki, w4, dw4);
+          if (kn) {
+            pidx = pidx_s[ti * V.npt + tj];
+            if (!BWD) {
+              const double *c = V.knot_c + (size_t)pidx * V.nknot + ki;
+              const double dup =
+                  (c[0] * dw4[0] + c[1] * dw4[1] + c[2] * dw4[2] + c[3] * dw4[3]) * V.knot_dinv;
+              f += (R)(-dup / sqrt(r2d));
+            }
+          }
+        }
+        if (!BWD) {
+          fx += (double)(f * dxr);
+          fy += (double)(f * dyr);
+          fz += (double)(f * dzr);
+        } else {
+          const R w = (rxi - rxs[u]) * dxr + (ryi - rys[u]) * dyr + (rzi - rzs[u]) * dzr;
+          dq += (double)(R(2) * efp * qj * g * w);
+          gs += (double)(w * fs);
+          if (eps > R(0)) ge += (double)(w * fe * ej / eps);
+          if (kn) {
+            const double wr = (double)w * V.knot_dinv / sqrt(r2d);
+            for (int m = 0; m < 4; ++m) atomicAdd(&sk[pidx * V.nknot + ki + m], -wr * dw4[m]);
+          }
         }
       }
     }
@@ -363,14 +404,11 @@ __global__ void __launch_bounds__(kFmBlock) k_fm_q(const SysDev *__restrict__ sy
   }
 }
 
-// acc[off + c] += sum over blocks of part[b * ncol + c] (fixed order)
-__global__ void __launch_bounds__(kFmBlock) k_fm_acc(const double *__restrict__ part, int nblk,
-                                                     int ncol, int cols, double *__restrict__ acc) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
-  double s = 0.0;
-  for (int b2 = 0; b2 < nblk; ++b2) s += part[(size_t)b2 * ncol + c];
-  acc[c] += s;
+// acc[c] += sum over blocks of part[b * ncol + c] (fixed order)
+__global__ void __launch_bounds__(kSumThreads) k_fm_acc(const double *__restrict__ part, int nblk,
+                                                        int ncol, int cols,
+                                                        double *__restrict__ acc) {
+  column_sums(part, nblk, ncol, cols, acc, true);
 }
 
 inline dim3 grid1(int x, const Group &g) { return dim3(x > 0 ? x : 1, 1, g.R); }
@@ -437,7 +475,7 @@ void launch_fm_q(const Group &g, const double *rpart, double *qr, double *part) 
 void launch_fm_acc(const Group &g, const double *part, int nblk, int ncol, int cols,
                    double *acc) {
   if (cols <= 0) return;
-  hipLaunchKernelGGL(k_fm_acc, dim3((cols + kFmBlock - 1) / kFmBlock), dim3(kFmBlock), 0,
+  hipLaunchKernelGGL(k_fm_acc, dim3((cols + kSumCols - 1) / kSumCols), dim3(kSumThreads), 0,
                      g.stream, part, nblk, ncol, cols, acc);
 }
 

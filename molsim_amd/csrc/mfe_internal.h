@@ -679,6 +679,7 @@ void launch_spme(const Group &g, bool energy, int first_stage, int last_stage,
                  int gather_mode = GM_FORCE, const FinArgs *fin = nullptr);
 // adjoint passes: real-space pair sums, per-particle dE/dq, column sums
 void launch_adjoint(const Group &g, int ncol, double *out);
+int adjoint_blocks(int np);  // rows of its partials
 void launch_std_ewald(const Group &g);
 void launch_bonds(const Group &g);
 void launch_surf(const Group &g);

@@ -2341,61 +2341,98 @@ __global__ void __launch_bounds__(kReduceThreads) k_reduce(const SysDev *__restr
 //   dE/dc[p][k]    1/2 spline weight of coefficient k
 // and 1/2 of the pair's model energy.  Per-block column partials:
 // [E, dsig(npt), deps(npt), dc(nptpt*nknot)].
+//
+// Four lanes share a particle's list, each with the indices and then the
+// positions of four entries in flight: a thread per particle, one entry at
+// a time, left the FP64 units to a wavefront per SIMD (66000 particles, 117
+// partners: 322 -> 130 us, now bound by FP64 issue: erfc, roots, divisions).
+constexpr int kAdjLanes = 4;
+constexpr int kAdjPer = kBlock / kAdjLanes;  // particles per block
 __global__ void __launch_bounds__(kBlock) k_adjoint(const SysDev *__restrict__ sys) {
   const SysDev &V = sys[blockIdx.z];
-  if ((int)blockIdx.x >= V.nblk_np) return;
+  const int np = V.np;
+  if ((int)blockIdx.x * kAdjPer >= np) return;
   extern __shared__ double sk[];
   __shared__ double sh[kBlock];
   const int nk = V.nptpt * V.nknot;
+  // the types' parameters and pair indices in LDS (read per entry by the
+  // partner's type)
+  __shared__ double zat_s[MFE_MAX_TYPES], sig_s[MFE_MAX_TYPES], eps_s[MFE_MAX_TYPES];
+  __shared__ int pidx_s[MFE_MAX_TYPES * MFE_MAX_TYPES];
+  const PairParams &pp = V.pp;
+  const TableDev &t = V.tab;
+  for (int k = threadIdx.x; k < V.npt; k += blockDim.x) {
+    zat_s[k] = pp.zat[k];
+    sig_s[k] = pp.sigat[k];
+    eps_s[k] = pp.epsat[k];
+  }
+  for (int k = threadIdx.x; k < t.npt * t.npt; k += blockDim.x) pidx_s[k] = t.pairidx[k];
   for (int k = threadIdx.x; k < nk; k += blockDim.x) sk[k] = 0.0;
   __syncthreads();
-  const PairParams &pp = V.pp;
-  const TableDev t = V.tab;
   const Box b = V.box;
-  const int np = V.np;
-  const int tt = blockIdx.x * blockDim.x + threadIdx.x;
-  double eu = 0.0, gs = 0.0, ge = 0.0;
+  const int lane = threadIdx.x % kAdjLanes;
+  const int tt = blockIdx.x * kAdjPer + threadIdx.x / kAdjLanes;
+  const bool act = tt < np;
+  double eu = 0.0, gs = 0.0, ge = 0.0, phi = 0.0;
   int ti = -1;
-  if (tt < np) {
-    const int i = V.c_sorted[tt];
+  if (act) {
     const double xi = V.ro_s[3 * tt], yi = V.ro_s[3 * tt + 1], zi = V.ro_s[3 * tt + 2];
     ti = V.type_s[tt];
-    const double qi = pp.zat[ti];
-    double phi = 0.0;
+    const double qi = zat_s[ti];
     const int n = V.nn[tt];
-    for (int k = 0; k < n; ++k) {
-      const int pj = (int)((unsigned)V.nbr[(size_t)k * np + tt] & kNbrIdxMask);
-      double dx = xi - V.ro_s[3 * pj], dy = yi - V.ro_s[3 * pj + 1], dz = zi - V.ro_s[3 * pj + 2];
-      const double r2 = pbcr2(dx, dy, dz, b);
-      if (V.nlsem == 0 ? (r2 > t.rcut2) : !(r2 < t.rcut2)) continue;
-      const int tj = V.type_s[pj];
-      const double r = sqrt(r2);
-      const double qj = pp.zat[tj];
-      const double c0 = pp.lewald ? erfc(pp.alpha * r) : 1.0;
-      phi += qj * pp.efp * c0 / r;
-      eu += 0.5 * qi * qj * pp.efp * c0 / r;
-      const double sig = 0.5 * (pp.sigat[ti] + pp.sigat[tj]);
-      const double eps = sqrt(pp.epsat[ti] * pp.epsat[tj]);
-      if (!pp.lljcut || r < pp.ljrcut * sig) {
-        const double x = sig / r, x2 = x * x, s6 = x2 * x2 * x2, s12 = s6 * s6;
-        const double sh_ = pp.lljcut ? pp.ljushift : 0.0;
-        eu += 0.5 * (4.0 * eps * (s12 - s6) + sh_ * eps);
-        gs += 0.5 * 4.0 * eps * (12.0 * s12 - 6.0 * s6) / sig;
-        if (eps > 0.0) ge += (4.0 * (s12 - s6) + sh_) * pp.epsat[tj] / (2.0 * eps);
+    for (int k0 = lane; k0 < n; k0 += kPairBatch * kAdjLanes) {
+      int pjs[kPairBatch], tjs[kPairBatch];
+      double xs[kPairBatch], ys[kPairBatch], zs[kPairBatch];
+#pragma unroll
+      for (int u = 0; u < kPairBatch; ++u) {
+        // rows clamped into the list; past its end the particle itself
+        const int k = k0 + u * kAdjLanes;
+        const int e = (int)((unsigned)V.nbr[(size_t)min(k, n - 1) * np + tt] & kNbrIdxMask);
+        pjs[u] = k < n ? e : tt;
       }
-      if (V.nknot) {
-        int ki;
-        double w[4], dw[4];
-        if (knot_weights(r, V.knot_r0, V.knot_dinv, V.nknot, ki, w, dw)) {
-          const int pidx = t.pairidx[ti * t.npt + tj];
-          const double *c = V.knot_c + (size_t)pidx * V.nknot + ki;
-          eu += 0.5 * (c[0] * w[0] + c[1] * w[1] + c[2] * w[2] + c[3] * w[3]);
-          for (int m = 0; m < 4; ++m) atomicAdd(&sk[pidx * V.nknot + ki + m], 0.5 * w[m]);
+#pragma unroll
+      for (int u = 0; u < kPairBatch; ++u) {
+        xs[u] = V.ro_s[3 * pjs[u]];
+        ys[u] = V.ro_s[3 * pjs[u] + 1];
+        zs[u] = V.ro_s[3 * pjs[u] + 2];
+        tjs[u] = V.type_s[pjs[u]];
+      }
+#pragma unroll
+      for (int u = 0; u < kPairBatch; ++u) {
+        if (k0 + u * kAdjLanes >= n) break;
+        double dx = xi - xs[u], dy = yi - ys[u], dz = zi - zs[u];
+        const double r2 = pbcr2(dx, dy, dz, b);
+        if (V.nlsem == 0 ? (r2 > t.rcut2) : !(r2 < t.rcut2)) continue;
+        const int tj = tjs[u];
+        const double r = sqrt(r2);
+        const double qj = zat_s[tj];
+        const double c0 = pp.lewald ? erfc(pp.alpha * r) : 1.0;
+        phi += qj * pp.efp * c0 / r;
+        eu += 0.5 * qi * qj * pp.efp * c0 / r;
+        const double sig = 0.5 * (sig_s[ti] + sig_s[tj]);
+        const double eps = sqrt(eps_s[ti] * eps_s[tj]);
+        if (!pp.lljcut || r < pp.ljrcut * sig) {
+          const double x = sig / r, x2 = x * x, s6 = x2 * x2 * x2, s12 = s6 * s6;
+          const double sh_ = pp.lljcut ? pp.ljushift : 0.0;
+          eu += 0.5 * (4.0 * eps * (s12 - s6) + sh_ * eps);
+          gs += 0.5 * 4.0 * eps * (12.0 * s12 - 6.0 * s6) / sig;
+          if (eps > 0.0) ge += (4.0 * (s12 - s6) + sh_) * eps_s[tj] / (2.0 * eps);
+        }
+        if (V.nknot) {
+          int ki;
+          double w[4], dw[4];
+          if (knot_weights(r, V.knot_r0, V.knot_dinv, V.nknot, ki, w, dw)) {
+            const int pidx = pidx_s[ti * t.npt + tj];
+            const double *c = V.knot_c + (size_t)pidx * V.nknot + ki;
+            eu += 0.5 * (c[0] * w[0] + c[1] * w[1] + c[2] * w[2] + c[3] * w[3]);
+            for (int m = 0; m < 4; ++m) atomicAdd(&sk[pidx * V.nknot + ki + m], 0.5 * w[m]);
+          }
         }
       }
     }
-    V.adj_phi[i] = phi;
   }
+  phi = lane_sum(phi, kAdjLanes);
+  if (act && lane == 0) V.adj_phi[V.c_sorted[tt]] = phi;
   double *out = V.adj_part + (size_t)blockIdx.x * V.adj_ncol;
   const double se = block_sum(eu, sh);
   if (threadIdx.x == 0) out[0] = se;
@@ -2431,15 +2468,12 @@ __global__ void __launch_bounds__(kBlock) k_adjoint_q(const SysDev *__restrict__
   V.adj_dq[i] = d;
 }
 
-// column sums of the adjoint partials in block order
-__global__ void __launch_bounds__(kBlock) k_adjoint_sum(const SysDev *__restrict__ sys,
-                                                        double *out) {
+// column sums of the adjoint partials in a fixed order
+__global__ void __launch_bounds__(kSumThreads) k_adjoint_sum(const SysDev *__restrict__ sys,
+                                                             double *out) {
   const SysDev &V = sys[blockIdx.z];
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= V.adj_ncol) return;
-  double s = 0.0;
-  for (int b2 = 0; b2 < V.nblk_np; ++b2) s += V.adj_part[(size_t)b2 * V.adj_ncol + c];
-  out[(size_t)blockIdx.z * V.adj_ncol + c] = s;
+  column_sums(V.adj_part, (V.np + kAdjPer - 1) / kAdjPer, V.adj_ncol, V.adj_ncol,
+              out + (size_t)blockIdx.z * V.adj_ncol, false);
 }
 
 // ------------------------------------------------- counter-based noise
@@ -3786,11 +3820,13 @@ void launch_collect(const Group &g, int *fl, double *en, int nen) {
 void launch_adjoint(const Group &g, int ncol, double *out) {
   // LDS of the knot accumulators: the largest replica's nptpt*nknot doubles
   const size_t lds = (size_t)std::max(ncol - 1, 1) * sizeof(double);
-  hipLaunchKernelGGL(k_adjoint, grid(g.np_blocks, g), dim3(kBlock), lds, g.stream, g.d);
+  hipLaunchKernelGGL(k_adjoint, grid(g.np_blocks * kAdjLanes, g), dim3(kBlock), lds, g.stream,
+                     g.d);
   hipLaunchKernelGGL(k_adjoint_q, grid(g.np_blocks, g), dim3(kBlock), 0, g.stream, g.d);
-  hipLaunchKernelGGL(k_adjoint_sum, grid(nblocks(ncol), g), dim3(kBlock), 0, g.stream, g.d,
-                     out);
+  hipLaunchKernelGGL(k_adjoint_sum, grid((ncol + kSumCols - 1) / kSumCols, g),
+                     dim3(kSumThreads), 0, g.stream, g.d, out);
 }
+int adjoint_blocks(int np) { return (np + kAdjPer - 1) / kAdjPer; }
 
 void launch_set_positions(const Group &g, const double *ro_new) {
   hipLaunchKernelGGL(k_set_positions, grid(g.np_blocks, g), dim3(kBlock), 0, g.stream, g.d,
