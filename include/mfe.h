@@ -384,11 +384,11 @@ int mfe_fm_loss_grad(mfe_engine *e, double *loss, double *dL_dzat,
 /* No reference counterpart: MOLSIM runs one system per process.  A batch
    drives nrep engines, each set up as above (own box, particles, tables,
    list, mesh), as one system: every stage of UTotal and VelVer is one
-   launch over all replicas; BD steps take one persistent launch where the
-   replicas allow it (mfe_batch_step_bd).  The replicas must share device,
-   precision, Ewald kind and SPME order; box, N, mesh, tables and cutoffs
-   are per replica.  Each replica computes exactly what its engine computes
-   alone.  Results stay in the engines (mfe_download_forces,
+   launch over all replicas; BD steps of large batches take one persistent
+   launch where the replicas allow it (mfe_batch_step_bd).  The replicas
+   must share device, precision, Ewald kind and SPME order; box, N, mesh,
+   tables and cutoffs are per replica.  Each replica computes exactly what
+   its engine computes alone.  Results stay in the engines (mfe_download_forces,
    mfe_download_state, mfe_get_energy) or come back together through
    mfe_batch_get_energies.  The engines must outlive the batch; a set-up
    call on an engine is picked up at the batch's next call.  On an error
@@ -406,16 +406,20 @@ int mfe_batch_compute(mfe_batch *b, uint32_t flags);
 int mfe_batch_step_md(mfe_batch *b, int32_t nsteps, double tstep, uint32_t flags);
 /* nsteps of BDStep + NList with each replica's device noise stream and
    factors (mfe_set_bd).  Mixed-precision SPME replicas without chains,
-   surface term or spline knots are advanced in one persistent launch: workgroups take replicas from a
-   queue (costliest first) and run all nsteps of a replica with workgroup
-   barriers only -- every stage of BDStep, UTotal and the gated SetVListMD.
-   A replica's result there depends on that replica alone.  Other batches
-   replay one captured graph per step.  As in mfe_step_bd, replicas whose
-   forces are not those of their current positions are evaluated first. */
+   surface term or spline knots can be advanced in one persistent launch:
+   workgroups take replicas from a queue (costliest first) and run all
+   nsteps of a replica with workgroup barriers only -- every stage of
+   BDStep, UTotal and the gated SetVListMD.  A replica's result there
+   depends on that replica alone.  Batches of at least two replicas per
+   compute unit take it, others replay one captured graph per step, unless
+   mfe_batch_set_persistent says otherwise.  As in mfe_step_bd, replicas
+   whose forces are not those of their current positions are evaluated
+   first. */
 int mfe_batch_step_bd(mfe_batch *b, int32_t nsteps, uint32_t flags);
-/* No reference counterpart: whether mfe_batch_step_bd may take the
-   persistent launch (on = 1, the default) or always replays the per-stage
-   graph (on = 0); and whether it would take it for this batch now. */
+/* No reference counterpart: mfe_batch_step_bd takes the persistent launch
+   wherever the replicas allow it (on = 1) or always replays the per-stage
+   graph (on = 0); without a call the number of replicas decides.  And
+   whether it would take the persistent launch for this batch now. */
 int mfe_batch_set_persistent(mfe_batch *b, int32_t on);
 int32_t mfe_batch_uses_persistent(mfe_batch *b);
 /* energies of the last UTotal of every replica: out[nrep] */

@@ -34,7 +34,7 @@ struct mfe_batch {
   int failed = -1;
   // persistent BD: replica order (costliest first), queue counter, and
   // the captured graph of the launch (queue reset + kernel) for pgraph_key
-  bool persist = true;
+  int persist = -1;  // mfe_batch_set_persistent: 0, 1, or -1 where not called
   int *d_order = nullptr, *d_queue = nullptr;
   hipGraphExec_t pgraph = nullptr;
   long long pgraph_key = -1;
@@ -244,8 +244,20 @@ int mfe_batch_compute(mfe_batch *b, uint32_t flags) {
 // no chains, surface term or spline knots, whose LDS needs fit a CU.
 namespace {
 
+//
+// Where the caller has not said, batches of fewer than two replicas per CU
+// replay the per-stage graph: a replica's persistent step takes a CU's time
+// however many CUs stand idle, and the per-stage launches spread every
+// replica over the chip.  Per BD step, persistent against per-stage: 8
+// replicas of up to 4000 ions (rc 18 A, meshes 18-36) 812 / 83 us, 96: 935 /
+// 288, 384: 1191 / 911; 96 of up to 1000 ions 254 / 157; 512 at rc 20 A and
+// meshes 16-48 1604 / 1169, 1024: 2241 / 2337.  The schedules cross between
+// two and four replicas per CU, depending on their sizes; from two on the
+// persistent launch stays the default, whose results do not depend on the
+// batch a replica is in, and the autotuner times both.
 bool persist_eligible(const mfe_batch *b, size_t *lds) {
-  if (!b->persist) return false;
+  if (b->persist == 0) return false;
+  if (b->persist < 0 && (int)b->eng.size() < 2 * std::max(b->eng[0]->ncu, 1)) return false;
   const mfe::Group &g = b->grp;
   if (g.prec != MFE_PREC_MIXED || g.ewald != MFE_EWALD_SPME || g.chains || g.surf ||
       g.knots || g.order < 3 || g.order > 8)
@@ -359,7 +371,7 @@ int mfe_batch_step_bd(mfe_batch *b, int32_t nsteps, uint32_t flags) {
 
 int mfe_batch_set_persistent(mfe_batch *b, int32_t on) {
   if (!b) return MFE_E_BAD_PARAM;
-  b->persist = on != 0;
+  b->persist = on != 0 ? 1 : 0;
   return MFE_OK;
 }
 

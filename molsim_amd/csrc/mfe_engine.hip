@@ -283,7 +283,7 @@ void set_cell_geom(mfe_engine *e) {
 int list_lsh_for(const mfe_engine *e) {
   const double row = 3.0 * e->np / std::max(e->cg.ncells, 1);
   if (row < 8.0) return 0;
-  return row >= 48.0 && e->np <= 32768 ? 4 : (e->np <= 262144 ? 2 : 0);
+  return row >= 20.0 && e->np <= 32768 ? 4 : (e->np <= 262144 ? 2 : 0);
 }
 
 int auto_maxnn(const mfe_engine *e) {
@@ -540,11 +540,18 @@ int mfe_group_build(mfe_engine *const *eng, int R, const mfe::SysDev *d, hipStre
       g.lds_gather = std::max(g.lds_gather, gext);
     }
   }
-  // the fused pair + gather launch: its block holds both kernels' static
-  // LDS (~6.5 KB) and the larger dynamic need, within 64 KB
+  // The fused pair + gather launch: its block holds both kernels' static
+  // LDS (~6.5 KB) and the larger dynamic need, within 64 KB.  It saves a
+  // launch and lets the pair waves fill what the gather leaves idle (200k
+  // ions 40 us against 26 + 22, 8 replicas of 2250 ions 19.5 against 22); a
+  // batch that fills the chip several times over is faster with the pair
+  // launch beside the SPME stages on the second stream (96 replicas 163 us
+  // fused, 87 + 44 apart).
+  constexpr long long kFuseBlocks = 2048;
   g.fuse_pg = g.prec == MFE_PREC_MIXED && g.ewald == MFE_EWALD_SPME && !g.chains && !g.surf &&
               !g.knots && !g.pair_any64 && g.pair_cf_lds &&
-              std::max(g.lds_pair, g.lds_gather) <= mfe::kPairLdsBudget;
+              std::max(g.lds_pair, g.lds_gather) <= mfe::kPairLdsBudget &&
+              (R == 1 || (long long)R * (g.pair_blocks + g.bricks) <= kFuseBlocks);
   return MFE_OK;
 }
 

@@ -621,7 +621,9 @@ class Batch:
         self._check(self.L.mfe_batch_step_bd(self.h, int(nsteps), flags), "mfe_batch_step_bd")
 
     def set_persistent(self, on=True):
-        """Let step_bd take the persistent launch where eligible (default)."""
+        """Let step_bd take the persistent launch where eligible (on) or
+        always the per-stage graph (off); by default the number of replicas
+        decides."""
         self._check(self.L.mfe_batch_set_persistent(self.h, 1 if on else 0),
                     "mfe_batch_set_persistent")
 
