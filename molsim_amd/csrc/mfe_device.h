@@ -255,6 +255,19 @@ struct SpreadAcc<double> {
 
 constexpr int kMaxOrder = 8;
 
+// the spreading tile (z planes of SpmeGeom::plane values) written to global
+// memory without the padding
+template <typename R>
+__device__ __forceinline__ void store_tile(const SpmeGeom &g, int E0, int E1, int E2,
+                                           const typename SpreadAcc<R>::T *tile,
+                                           R *__restrict__ out) {
+  const int pad = g.plane - E0 * E1;
+  for (int k = threadIdx.x; k < E0 * E1 * E2; k += blockDim.x) {
+    const int z = pad ? fdiv(fdiv(k, g.fE[0]), g.fE[1]) : 0;
+    out[k] = SpreadAcc<R>::get(tile[k + z * pad]);
+  }
+}
+
 // one particle record in brick order: fraction (x, y, z) and charge
 template <typename R>
 struct Rec4 {

@@ -369,6 +369,7 @@ void mfe_fill_view(const mfe_engine *e, mfe::SysDev &v) {
       v.sg.dkdr[m] = e->s[m] / e->box.L[m];
     }
     v.sg.order = e->order;
+    v.sg.plane = e->spread_plane;
     for (int m = 0; m < 3; ++m) {
       v.sg.fB[m] = mfe::make_fastdiv(e->B[m]);
       v.sg.fE[m] = mfe::make_fastdiv(e->B[m] + e->order - 1);
@@ -1092,20 +1093,31 @@ int mfe_set_ewald(mfe_engine *e, int32_t kind, double alpha, int32_t order,
         e->plan[m] = make_plan(e->s[m]);
         if (!plan_ok(e->plan[m])) return fail(e, MFE_E_BAD_PARAM, "mesh has a prime factor > 32");
       }
-      // bricks of the spreading and gather blocks: B divides s; 16 when s
-      // allows (fewer halo points per brick), else the smallest divisor >= 8
-      size_t ext = 1;
+      // bricks of the spreading and gather blocks: B divides s, the largest
+      // divisor from 16 down to 8 (fewer halo points per brick and fewer,
+      // fuller blocks: 120^3, 100k ions, order 4, B = 8 / 15: spreading 17.2
+      // / 7.8 us, gather 27 / 12, binning 15 / 9.5; 70^3, 20005 ions, B = 10
+      // / 14: no difference), else the smallest divisor above
+      size_t ext = 1, planes = 1;
       for (int m = 0; m < 3; ++m) {
-        int b = (e->s[m] % 16 == 0) ? 16 : smallest_divisor_at_least(e->s[m], 8);
+        int b = 0;
+        for (int d = 16; d >= 8 && !b; --d)
+          if (e->s[m] % d == 0) b = d;
+        if (!b) b = smallest_divisor_at_least(e->s[m], 17);
         if (b > 16) b = smallest_divisor_at_least(e->s[m], order - 1);
         e->B[m] = b;
         e->nb[m] = e->s[m] / b;
         ext *= (size_t)(b + order - 1);
+        if (m == 1) planes = ext;
       }
       e->nbricks = e->nb[0] * e->nb[1] * e->nb[2];
       const size_t rsz = e->prec == MFE_PREC_MIXED ? 4 : 8;
-      // spreading tile: 64-bit fixed point (mixed) or FP64 per extended point
-      e->spread_lds = (int)(ext * 8);
+      // spreading tile: 64-bit fixed point (mixed) or FP64 per extended point,
+      // z planes of an odd number of values where the CU's LDS holds them
+      // (SpmeGeom::plane)
+      const size_t E2 = (size_t)(e->B[2] + order - 1);
+      e->spread_plane = (int)((planes | 1) * E2 * 8 <= 160 * 1024 ? planes | 1 : planes);
+      e->spread_lds = (int)(e->spread_plane * E2 * 8);
       const size_t gext = ext * rsz;
       const int lds_need = (int)std::max<size_t>((size_t)e->spread_lds, gext);
       if ((size_t)lds_need > 160 * 1024)

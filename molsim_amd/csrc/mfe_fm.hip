@@ -315,9 +315,9 @@ __global__ void __launch_bounds__(1024) k_fm_spread(const SysDev *__restrict__ s
   const int o0 = bx * g.B[0] - (ORDER - 1), o1 = by * g.B[1] - (ORDER - 1),
             o2 = bz * g.B[2] - (ORDER - 1);
   const int E0 = g.B[0] + ORDER - 1, E1 = g.B[1] + ORDER - 1, E2 = g.B[2] + ORDER - 1;
-  const int ntile = E0 * E1 * E2;
+  const int ntile = E0 * E1 * E2, plane = g.plane;
   const int first = bstart[blockIdx.x], items = (bstart[blockIdx.x + 1] - first) * ORDER;
-  for (int k = threadIdx.x; k < ntile; k += blockDim.x) tile[k] = Acc(0);
+  for (int k = threadIdx.x; k < plane * E2; k += blockDim.x) tile[k] = Acc(0);
   __syncthreads();
   for (int r = threadIdx.x; r < items; r += blockDim.x) {
     const int rec = first + r / ORDER;
@@ -339,20 +339,20 @@ __global__ void __launch_bounds__(1024) k_fm_spread(const SysDev *__restrict__ s
     const int lx = (code & 1023) - o0;
     const int ly = ((code >> 10) & 1023) - o1;
     const int lz = ((code >> 20) & 1023) - o2;
-    Acc *plane = tile + (lz - iz) * E1 * E0;
+    Acc *zp = tile + (lz - iz) * plane;
 #pragma unroll
     for (int jy = 0; jy < ORDER; ++jy) {
       // point (jx, jy, iz): dx[jx] * A + wx[jx] * Bc
       const R A = v.x * wy[jy] * wzi;
       const R Bc = v.y * dy[jy] * wzi + v.z * wy[jy] * dzi;
-      Acc *row = plane + (ly - jy) * E0 + lx;
+      Acc *row = zp + (ly - jy) * E0 + lx;
 #pragma unroll
       for (int j = 0; j < ORDER; ++j) SpreadAcc<R>::add(&row[-j], dx[j] * A + wx[j] * Bc);
     }
   }
   __syncthreads();
   R *__restrict__ out = (R *)V.spread_tiles + (size_t)blockIdx.x * ntile;
-  for (int k = threadIdx.x; k < ntile; k += blockDim.x) out[k] = SpreadAcc<R>::get(tile[k]);
+  store_tile<R>(g, E0, E1, E2, tile, out);
 }
 
 // the sum q r of the residual partials (the surface term needs it whole)

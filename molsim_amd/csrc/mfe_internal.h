@@ -251,6 +251,11 @@ __device__ __forceinline__ int xcd_block(int b, int nblk) {
 // SPME mesh geometry: mesh s, spreading bricks B (nb per axis), dkdr = s/L.
 struct SpmeGeom {
   int s[3], B[3], nb[3], order;
+  // values per z plane of a spreading tile in LDS: odd (one more than the
+  // plane's points where those are even), so that the stencil planes of one
+  // particle, which neighbouring lanes add, start in different banks: planes
+  // of 20 x 20 values (bricks of 15, order 6) fall into two
+  int plane;
   double dkdr[3];
   FastDiv fB[3];   // the brick edges B
   FastDiv fE[3];   // the extended tile edges B + order - 1
@@ -589,7 +594,7 @@ struct mfe_engine {
   void *tw[3] = {nullptr, nullptr, nullptr};     // twiddles of length s[a]
   void *tw_half = nullptr;                       // twiddles of length s1/2
   mfe::FftPlan plan[3]{}, plan_half{};
-  int spread_lds = 0;
+  int spread_lds = 0, spread_plane = 0;
   // standard Ewald
   int ncut = 0, ncut_cube = 0, nkvec = 0;
   double *k_vec = nullptr;   // [nkvec][4]: kx, ky, kz (2*pi*n/L), kfac

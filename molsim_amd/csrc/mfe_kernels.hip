@@ -1342,7 +1342,7 @@ __global__ void __launch_bounds__(kSpreadThreads) k_spread(const SysDev *__restr
   const int o0 = bx * g.B[0] - (ORDER - 1), o1 = by * g.B[1] - (ORDER - 1),
             o2 = bz * g.B[2] - (ORDER - 1);
   const int E0 = g.B[0] + ORDER - 1, E1 = g.B[1] + ORDER - 1, E2 = g.B[2] + ORDER - 1;
-  const int ntile = E0 * E1 * E2;
+  const int ntile = E0 * E1 * E2, plane = g.plane;
   const int first = bstart[blockIdx.x], items = (bstart[blockIdx.x + 1] - first) * ORDER;
   int r = threadIdx.x;
   Rec4<R> f{};
@@ -1352,7 +1352,7 @@ __global__ void __launch_bounds__(kSpreadThreads) k_spread(const SysDev *__restr
     f = load_rec(frac + 4 * rec);
     code = meta[rec].x;
   }
-  for (int k = threadIdx.x; k < ntile; k += kSpreadThreads) tile[k] = Acc(0);
+  for (int k = threadIdx.x; k < plane * E2; k += kSpreadThreads) tile[k] = Acc(0);
   __syncthreads();
   for (; r < items; r += kSpreadThreads) {
     const int rn = r + kSpreadThreads;
@@ -1376,11 +1376,11 @@ __global__ void __launch_bounds__(kSpreadThreads) k_spread(const SysDev *__restr
     const int ly = ((code >> 10) & 1023) - o1;
     const int lz = ((code >> 20) & 1023) - o2;
     const R qz = f.q * wzi;
-    Acc *plane = tile + (lz - iz) * E1 * E0;
+    Acc *zp = tile + (lz - iz) * plane;
 #pragma unroll
     for (int jy = 0; jy < ORDER; ++jy) {
       const R qyz = qz * wy[jy];
-      Acc *row = plane + (ly - jy) * E0 + lx;
+      Acc *row = zp + (ly - jy) * E0 + lx;
 #pragma unroll
       for (int j = 0; j < ORDER; ++j) SpreadAcc<R>::add(&row[-j], qyz * wx[j]);
     }
@@ -1389,7 +1389,7 @@ __global__ void __launch_bounds__(kSpreadThreads) k_spread(const SysDev *__restr
   }
   __syncthreads();
   R *__restrict__ out = (R *)V.spread_tiles + (size_t)blockIdx.x * ntile;
-  for (int k = threadIdx.x; k < ntile; k += kSpreadThreads) out[k] = SpreadAcc<R>::get(tile[k]);
+  store_tile<R>(g, E0, E1, E2, tile, out);
 }
 
 // per-lane stencil sums: compensated FP32 on the mixed path, plain FP64
