@@ -151,11 +151,10 @@ void free_all(mfe_engine *e) {
   dfree(e->mesh_r); dfree(e->mesh_c); dfree(e->b_count); dfree(e->b_start); dfree(e->b_done);
   dfree(e->b_id); dfree(e->b_slot); dfree(e->rec_frac); dfree(e->rec_meta);
   dfree(e->spread_tiles);
-  dfree(e->mc_ia); dfree(e->mc_rtm); dfree(e->mc_out);
+  dfree(e->mc_ia); dfree(e->mc_rtm); dfree(e->mc_old); dfree(e->mc_part);
   if (e->mc_spec) (void)hipFree(e->mc_spec);
   e->mc_spec = nullptr;
   e->mc_spec_bytes = 0;
-  dfree(e->mc_fac);
   if (e->h_mc) (void)hipHostFree(e->h_mc);
   e->h_mc = nullptr;
   e->h_mc_bytes = 0;
@@ -311,6 +310,21 @@ int read_flags(mfe_engine *e) {
   MFE_HIP_TRY(hipMemcpyAsync(e->h_flags, e->flags, 3 * sizeof(int), hipMemcpyDeviceToHost, e->stream));
   MFE_HIP_TRY(hipStreamSynchronize(e->stream));
   return mfe_map_flag_error(e, e->h_flags[0]);
+}
+
+// NList's skin test after new positions and, where it fires, the rebuild;
+// returns the flagged error, if any (waits for the stream)
+int skin_and_rebuild(mfe_engine *e) {
+  const mfe::Group &G = e->grp;
+  mfe::launch_skin(G);
+  if (!mfe::launch_finalize_rebuild(G, 0u, false, -1, 0.0, false, e->h_flags)) {
+    mfe::launch_reduce(G, 0u, true, false);
+    mfe::launch_nlist_rebuild(G, true);
+    return read_flags(e);
+  }
+  MFE_HIP_TRY(hipGetLastError());
+  MFE_HIP_TRY(hipStreamSynchronize(e->stream));
+  return e->h_flags[1] ? read_flags(e) : mfe_map_flag_error(e, e->h_flags[0]);
 }
 
 inline int nblocks256(int n) { return (n + 255) / 256; }
@@ -1321,10 +1335,7 @@ int mfe_upload_positions(mfe_engine *e, const double *ro) {
       upload(e->ro_stage, ro, 3 * (size_t)e->np, e->stream);
       sync_view(e);
       mfe::launch_set_positions(e->grp, e->ro_stage);
-      mfe::launch_skin(e->grp);
-      mfe::launch_reduce(e->grp, 0u, true, false);
-      mfe::launch_nlist_rebuild(e->grp, true);
-      return read_flags(e);
+      return skin_and_rebuild(e);
     }
     upload(e->ro, ro, 3 * (size_t)e->np, e->stream);
     MFE_HIP_TRY(hipStreamSynchronize(e->stream));
@@ -1434,17 +1445,20 @@ int mc_prepare(mfe_engine *e, int natm, const int32_t *ianatm, const double *rtm
   return MFE_OK;
 }
 
-// device room for natm moved particles and the four results
+// bytes of the results at the start of the pinned memory: pair change and
+// overlap, or the parts of the reciprocal change
+constexpr size_t kMcResultBytes = 8 * (size_t)mfe::kMcRecBlocks;
+
+// device and pinned room for a move of natm particles
 void mc_buffers(mfe_engine *e, int natm) {
   if (e->mc_cap < natm) {
     dalloc(e->mc_ia, (size_t)natm);
     dalloc(e->mc_rtm, 3 * (size_t)natm);
     e->mc_cap = natm;
   }
-  // [reciprocal change, 0, du_twob, overlap, block partials]
-  if (!e->mc_out) dalloc(e->mc_out, 4 + 2 * (size_t)mfe::kMcPairBlocks);
-  // pinned staging: 4 results, then the indices, then the positions
-  const size_t bytes = 32 + ((size_t)natm * sizeof(int) + 7) / 8 * 8 + 24 * (size_t)natm;
+  if (!e->mc_part) dalloc(e->mc_part, 2 * (size_t)mfe::kMcPairBlocks);
+  const size_t bytes = kMcResultBytes + ((size_t)natm * sizeof(int) + 7) / 8 * 8 +
+                       24 * (size_t)natm;
   if (e->h_mc_bytes < bytes) {
     if (e->h_mc) MFE_HIP_TRY(hipHostFree(e->h_mc));
     e->h_mc = nullptr;
@@ -1454,60 +1468,50 @@ void mc_buffers(mfe_engine *e, int natm) {
   }
 }
 
-// the move's indices and positions in the pinned staging (device-
-// accessible host memory: a kernel that reads them a few times takes them
-// from there directly)
-void mc_stage(mfe_engine *e, const std::vector<int> &ia, const double *rtm, int **hi_out,
-              double **hr_out) {
+// the move in the kernels' form; one that the arguments cannot hold goes to
+// the device through the pinned staging (asynchronous copies; every MC call
+// ends with a synchronization before the staging is written again)
+mfe::McMove mc_move(mfe_engine *e, const std::vector<int> &ia, const double *rtm) {
+  mfe::McMove mv;
   const size_t natm = ia.size();
-  int *hi = reinterpret_cast<int *>(e->h_mc + 32);
-  double *hr = reinterpret_cast<double *>(e->h_mc + 32 + (natm * sizeof(int) + 7) / 8 * 8);
+  mv.natm = (int)natm;
+  mv.ia = e->mc_ia;
+  mv.rtm = e->mc_rtm;
+  if (natm <= (size_t)mfe::kMcArg) {
+    std::copy(ia.begin(), ia.end(), mv.ia_v);
+    std::copy(rtm, rtm + 3 * natm, mv.rtm_v);
+    return mv;
+  }
+  int *hi = reinterpret_cast<int *>(e->h_mc + kMcResultBytes);
+  double *hr =
+      reinterpret_cast<double *>(e->h_mc + kMcResultBytes + (natm * sizeof(int) + 7) / 8 * 8);
   std::memcpy(hi, ia.data(), natm * sizeof(int));
   std::memcpy(hr, rtm, 3 * natm * sizeof(double));
-  *hi_out = hi;
-  *hr_out = hr;
+  upload(e->mc_ia, hi, natm, e->stream);
+  upload(e->mc_rtm, hr, 3 * natm, e->stream);
+  return mv;
 }
 
-// the move's indices and positions to the device through the pinned
-// staging (asynchronous copies; every MC call ends with a synchronization
-// before the staging is written again), for kernels that read them often
-void mc_upload(mfe_engine *e, const std::vector<int> &ia, const double *rtm) {
-  int *hi;
-  double *hr;
-  mc_stage(e, ia, rtm, &hi, &hr);
-  upload(e->mc_ia, hi, ia.size(), e->stream);
-  upload(e->mc_rtm, hr, 3 * ia.size(), e->stream);
-}
+// the results, which the last kernel of a trial writes to pinned memory
+// (valid once the stream is synchronized)
+double *mc_results(mfe_engine *e) { return reinterpret_cast<double *>(e->h_mc); }
 
-// the results slots of the pinned staging, which the last kernel of a
-// trial writes directly
-double *mc_result_slots(mfe_engine *e) { return reinterpret_cast<double *>(e->h_mc); }
-
-// n results from the staging's result slots (waits for the stream)
-void mc_results(mfe_engine *e, int n, double *out) {
-  MFE_HIP_TRY(hipStreamSynchronize(e->stream));
-  const double *h = mc_result_slots(e);
-  for (int k = 0; k < n; ++k) out[k] = h[k];
-}
-
-// the kept spectrum (the complex mesh's size) and the stencil factors of
-// natm moved particles; a new spectrum buffer is not a valid one
+// the kept spectrum (the complex mesh's size, FP64 values on both precision
+// paths; a new buffer is not a valid one) and room for the positions of
+// natm moved particles
 void mc_spectrum_buffers(mfe_engine *e, int natm) {
-  // FP64 values on both precision paths
+  if (e->mc_old_cap < natm) {
+    dalloc(e->mc_old, 3 * (size_t)natm);
+    e->mc_old_cap = natm;
+  }
   const size_t bytes = (size_t)e->hx * e->s[1] * e->s[2] * 16;
-  if (e->mc_spec_bytes != bytes) {
-    if (e->mc_spec) MFE_HIP_TRY(hipFree(e->mc_spec));
-    e->mc_spec = nullptr;
-    e->mc_spec_bytes = 0;
-    e->mc_cached = false;
-    MFE_HIP_TRY(hipMalloc(&e->mc_spec, bytes));
-    e->mc_spec_bytes = bytes;
-  }
-  const size_t nfac = 2 * 2 * (size_t)natm * (e->s[0] + e->s[1] + e->s[2]);
-  if (e->mc_fac_cap < nfac) {
-    dalloc(e->mc_fac, nfac);
-    e->mc_fac_cap = nfac;
-  }
+  if (e->mc_spec_bytes == bytes) return;
+  if (e->mc_spec) MFE_HIP_TRY(hipFree(e->mc_spec));
+  e->mc_spec = nullptr;
+  e->mc_spec_bytes = 0;
+  e->mc_cached = false;
+  MFE_HIP_TRY(hipMalloc(&e->mc_spec, bytes));
+  e->mc_spec_bytes = bytes;
 }
 
 }  // namespace
@@ -1526,24 +1530,11 @@ int mfe_mc_delta_pair(mfe_engine *e, int32_t natm, const int32_t *ianatm, const 
   return guarded(e, [&]() -> int {
     MFE_HIP_TRY(hipSetDevice(e->device));
     mc_buffers(e, natm);
-    // small moves straight from the pinned staging (the kernel stages them
-    // in LDS), larger ones through device copies
-    int *hi;
-    double *hr;
-    mc_stage(e, ia, rtm, &hi, &hr);
-    const int *mia = hi;
-    const double *mrtm = hr;
-    if (natm > mfe::kMcStage) {
-      upload(e->mc_ia, hi, (size_t)natm, e->stream);
-      upload(e->mc_rtm, hr, 3 * (size_t)natm, e->stream);
-      mia = e->mc_ia;
-      mrtm = e->mc_rtm;
-    }
+    const mfe::McMove mv = mc_move(e, ia, rtm);
     sync_view(e);
-    mfe::launch_mc_pair(e->grp, natm, mia, mrtm, mc_result_slots(e), e->mc_out + 4,
-                        e->nlkind == MFE_NL_CELL);
-    double h[2];
-    mc_results(e, 2, h);
+    double *h = mc_results(e);
+    mfe::launch_mc_pair(e->grp, mv, h, e->mc_part, e->nlkind == MFE_NL_CELL);
+    MFE_HIP_TRY(hipStreamSynchronize(e->stream));
     *overlap = h[1] != 0.0 ? 1 : 0;
     *du_twob = *overlap ? 0.0 : h[0];
     return MFE_OK;
@@ -1632,11 +1623,20 @@ int mfe_mc_delta_pair_noalloc(mfe_engine *e, int32_t natm, const int32_t *ianatm
     double *d_rtm = reinterpret_cast<double *>(sp + kNaRtmOff);
     double *d_out = reinterpret_cast<double *>(sp + kNaOutOff);
     double *d_part = reinterpret_cast<double *>(sp + kNaPartOff);
-    MFE_HIP_TRY(hipMemcpyAsync(d_ia, ia, natm * sizeof(int), hipMemcpyHostToDevice, e->stream));
-    MFE_HIP_TRY(hipMemcpyAsync(d_rtm, rtm, 3 * (size_t)natm * sizeof(double),
-                               hipMemcpyHostToDevice, e->stream));
+    mfe::McMove mv;
+    mv.natm = natm;
+    mv.ia = d_ia;
+    mv.rtm = d_rtm;
+    if (natm <= mfe::kMcArg) {
+      std::copy(ia, ia + natm, mv.ia_v);
+      std::copy(rtm, rtm + 3 * (size_t)natm, mv.rtm_v);
+    } else {
+      MFE_HIP_TRY(hipMemcpyAsync(d_ia, ia, natm * sizeof(int), hipMemcpyHostToDevice, e->stream));
+      MFE_HIP_TRY(hipMemcpyAsync(d_rtm, rtm, 3 * (size_t)natm * sizeof(double),
+                                 hipMemcpyHostToDevice, e->stream));
+    }
     sync_view(e);
-    mfe::launch_mc_pair(e->grp, natm, d_ia, d_rtm, d_out, d_part, e->nlkind == MFE_NL_CELL);
+    mfe::launch_mc_pair(e->grp, mv, d_out, d_part, e->nlkind == MFE_NL_CELL);
     double h[2];
     MFE_HIP_TRY(hipMemcpyAsync(h, d_out, sizeof(h), hipMemcpyDeviceToHost, e->stream));
     MFE_HIP_TRY(hipStreamSynchronize(e->stream));
@@ -1667,9 +1667,7 @@ int mfe_mc_delta_rec(mfe_engine *e, int32_t natm, const int32_t *ianatm, const d
     MFE_HIP_TRY(hipSetDevice(e->device));
     mc_buffers(e, natm);
     mc_spectrum_buffers(e, natm);
-    int *hi;
-    double *hr;
-    mc_stage(e, ia, rtm, &hi, &hr);
+    const mfe::McMove mv = mc_move(e, ia, rtm);
     sync_view(e);
     const mfe::Group &G = e->grp;
     if (!(reuse_current && e->mc_cached)) {
@@ -1680,12 +1678,12 @@ int mfe_mc_delta_rec(mfe_engine *e, int32_t natm, const int32_t *ianatm, const d
       mfe::launch_spme(G, true, SP_BIN, SP_FFTY);
       mfe::fft_z_forward(G, e->mc_spec);
     }
-    // the trial's stencil factors, then the energy change over the spectrum
-    mfe::launch_mc_kfac(G, natm, hi, hr, e->mc_fac);
-    mfe::launch_mc_kdelta(G, natm, e->mc_fac, e->mc_spec, false, e->mc_out + 4,
-                          mc_result_slots(e));
+    // the energy change over the spectrum, the blocks' parts added in order
+    double *part = mc_results(e);
+    const int nb = mfe::launch_mc_rec(G, mv, e->mc_spec, e->mc_old, part);
+    MFE_HIP_TRY(hipStreamSynchronize(e->stream));
     double h = 0.0;
-    mc_results(e, 1, &h);
+    for (int b = 0; b < nb; ++b) h += part[b];
     e->mc_cached = true;
     e->mc_last_ia = ia;
     e->mc_last_rtm.assign(rtm, rtm + 3 * (size_t)natm);
@@ -1725,34 +1723,21 @@ int mfe_mc_accept(mfe_engine *e, int32_t natm, const int32_t *ianatm, const doub
   return guarded(e, [&]() -> int {
     MFE_HIP_TRY(hipSetDevice(e->device));
     mc_buffers(e, natm);
-    // small moves straight from the pinned staging, larger ones through
-    // device copies
-    const bool small = natm <= mfe::kMcStage;
-    int *hi = nullptr;
-    double *hr = nullptr;
-    if (small) mc_stage(e, ia, rtm, &hi, &hr);
-    else mc_upload(e, ia, rtm);
+    const mfe::McMove mv = mc_move(e, ia, rtm);
     sync_view(e);
     const mfe::Group &G = e->grp;
-    if (keep) {
-      // the trial's change added to the kept spectrum (its stencil factors
-      // are those of the last trial, this move)
-      mfe::launch_mc_kdelta(G, natm, e->mc_fac, e->mc_spec, true, nullptr, nullptr);
-    }
-    // the accepted positions, then NList(iSimulationStep) as after an upload
-    if (small) {
-      mfe::launch_set_positions_moved(G, natm, hi, hr);
-    } else {
+    // the trial's change added to the kept spectrum, and the accepted
+    // positions, then NList(iSimulationStep) as after an upload
+    const bool small = natm <= mfe::kMcArg;
+    mfe::launch_mc_accept(G, mv, small, keep ? e->mc_spec : nullptr, e->mc_old);
+    if (!small) {
       if (!e->ro_stage) dalloc(e->ro_stage, 3 * (size_t)e->max_np);
       MFE_HIP_TRY(hipMemcpyAsync(e->ro_stage, e->ro, 3 * (size_t)e->np * sizeof(double),
                                  hipMemcpyDeviceToDevice, e->stream));
       mfe::launch_mc_place(G, natm, e->mc_ia, e->mc_rtm, e->ro_stage);
       mfe::launch_set_positions(G, e->ro_stage);
     }
-    mfe::launch_skin(G);
-    mfe::launch_reduce(G, 0u, true, false);
-    mfe::launch_nlist_rebuild(G, true);
-    int r = read_flags(e);
+    int r = skin_and_rebuild(e);
     if (r) return r;
     e->mc_cached = keep;
     return MFE_OK;

@@ -563,21 +563,18 @@ struct mfe_engine {
   void *mesh_r = nullptr;    // real mesh [s3][s2][s1]
   void *mesh_c = nullptr;    // complex mesh [s3][s2][hx]
   int *b_count = nullptr, *b_start = nullptr, *b_id = nullptr, *b_slot = nullptr;
-  // Monte Carlo trial moves: moved particles, their trial positions, and the
-  // two reciprocal energies (current, trial)
+  // Monte Carlo trial moves: the moved particles, trial and current
+  // positions on the device (the first two for moves of more than kMcArg),
+  // and the pair part's block partials
   int *mc_ia = nullptr;
-  double *mc_rtm = nullptr, *mc_out = nullptr;
-  int mc_cap = 0;
-  // the current configuration's spreading tiles and (in mc_out[0]) its
-  // E_rec, kept for callers whose positions have not changed since
-  // MC trial moves: the kept spectrum (forward transform of the current
-  // configuration's mesh, valid while mc_cached) and the stencil factors
+  double *mc_rtm = nullptr, *mc_old = nullptr, *mc_part = nullptr;
+  int mc_cap = 0, mc_old_cap = 0;
+  // the kept spectrum (forward transform of the current configuration's
+  // mesh, valid while mc_cached)
   void *mc_spec = nullptr;
   size_t mc_spec_bytes = 0;
-  double *mc_fac = nullptr;
-  size_t mc_fac_cap = 0;
-  // pinned host staging of a move (indices, positions) and its results, so
-  // the copies of an MC call run asynchronously on the stream
+  // pinned host memory: the results of a trial, then the staging of a move
+  // of more than kMcArg particles, so its copies run on the stream
   char *h_mc = nullptr;
   size_t h_mc_bytes = 0;
   bool mc_cached = false;
@@ -696,9 +693,10 @@ void launch_reduce_finalize(const Group &g, unsigned flags, bool skin, bool bd, 
                             double dt, bool split = false);
 // launch_reduce_finalize (with the skin test) followed by the gated
 // rebuild, in one launch; false (nothing launched) when the group cannot
-// take it (several replicas, or no grid barrier state)
+// take it (several replicas, or no grid barrier state).  mode < 0 leaves the
+// finalize out; hflags (pinned): see k_finalize_rebuild
 bool launch_finalize_rebuild(const Group &g, unsigned flags, bool bd, int mode, double dt,
-                             bool split);
+                             bool split, int *hflags = nullptr);
 // the pair forces and the gather (into force_rec) in one launch
 void launch_pair_gather(const Group &g, bool energy, bool skin);
 void launch_move(const Group &g, double dt, int bd);
@@ -708,14 +706,28 @@ void launch_sort_pos(const Group &g);
 // of the positions)
 void launch_mc_place(const Group &g, int natm, const int *ia, const double *rtm,
                      double *ro_stage);
-// Monte Carlo trial move, reciprocal part (k_mc_kfac, k_mc_kdelta): the
-// stencil factors of the natm moved particles (current and trial
-// positions) into fac[natm][2][s1 + s2 + s3] (double2), then one pass over
-// the kept spectrum spec: the energy change (without EpsiFourPi) into
-// out[0] over part[2 * kMcPairBlocks], or (apply) spec += D.  One replica.
-void launch_mc_kfac(const Group &g, int natm, const int *ia, const double *rtm, void *fac);
-void launch_mc_kdelta(const Group &g, int natm, const void *fac, void *spec, bool apply,
-                      double *part, double *out);
+// A Monte Carlo trial move as its kernels take it: up to kMcArg moved
+// particles in the kernel arguments (no copy to the device, and no kernel
+// waits for a read of host memory), more of them from device memory.
+constexpr int kMcArg = 64;
+struct McMove {
+  int natm;
+  int ia_v[kMcArg];
+  double rtm_v[3 * kMcArg];
+  const int *ia;      // natm > kMcArg
+  const double *rtm;
+};
+// most blocks (and parts of the sum) of a trial's pass over the spectrum
+constexpr int kMcRecBlocks = 1024;
+// Monte Carlo trial move, reciprocal part (mc_rec_body): the energy change
+// (without EpsiFourPi) over the kept spectrum spec as part[b] of each of the
+// returned number of blocks (device-visible memory), the moved particles'
+// current positions into old[3 natm].  One replica.
+int launch_mc_rec(const Group &g, const McMove &mv, void *spec, double *old, double *part);
+// an accepted move, the last that launch_mc_rec was given: place (at most
+// kMcArg particles): launch_set_positions with it in place; with spec also
+// spec += its change
+void launch_mc_accept(const Group &g, const McMove &mv, bool place, void *spec, double *old);
 // the z forward transform of the complex mesh into out (no Green function)
 void fft_z_forward(const Group &g, void *out);
 // Monte Carlo trial move, pair part: out[0] the two-body energy change,
@@ -724,16 +736,9 @@ void fft_z_forward(const Group &g, void *out);
 // kMcPairBlocks blocks whose partials part[2 * kMcPairBlocks] are summed
 // in a fixed order; else the Verlet-list partners in one block
 constexpr int kMcPairBlocks = 512;
-// moves of up to this many particles: k_mc_pair stages them in LDS and may
-// read them from host memory
-constexpr int kMcStage = 64;
-void launch_mc_pair(const Group &g, int natm, const int *ia, const double *rtm, double *out,
-                    double *part, bool all);
+void launch_mc_pair(const Group &g, const McMove &mv, double *out, double *part, bool all);
 void launch_skin(const Group &g);
 void launch_set_positions(const Group &g, const double *ro_new);
-// the same with the current positions, the natm <= kMcStage particles ia
-// moved to rtm (device or pinned host memory)
-void launch_set_positions_moved(const Group &g, int natm, const int *ia, const double *rtm);
 void launch_collect(const Group &g, int *flags, double *en, int nen);
 // persistent batched BD (mfe_kernels.hip): nsteps BDSteps of every replica
 // in one launch, a workgroup per replica at a time, replicas taken from a

@@ -1679,171 +1679,273 @@ __global__ void __launch_bounds__(256) k_mc_place(int natm, const int *__restric
 // transform per trial, and no difference of two large energies.  Weights
 // and charge are rounded as the spreading rounds them (the fraction and q
 // to R, the B-spline in R), so D takes out the stencil the mesh holds up
-// to the rounding of the spreading's products.
+// to the rounding of the spreading's products.  One replica, fewer than
+// 2^31 points, kx fastest.
 //
-// The factor tables, fac[(a * 2 + n) * (s1 + s2 + s3) + off_m + k] for
-// moved particle a (n = 0 its current position, 1 the trial one), axis m
-// and wavenumber k, the charge folded into the x factor.
+// A block takes tiles of kMcTile consecutive spectrum points (four per
+// thread, their D in registers) and forms the factors that the tile needs
+// in LDS: x factors c(kx) with the charge folded in, and per mesh row
+// (ky, kz) the product of its y and z factors, each for the current (n = 0)
+// and the trial (1) position of up to `chunk` moved particles at a time.
+// The roots exp(-2 pi i p / s) of all axes come first, one per thread, so a
+// factor is ORDER products with table values at exactly reduced phases.
+// apply == false writes the block's part of the energy change to
+// part[block] (the host adds the parts in block order) and block 0 keeps
+// the current positions in `old`; apply == true adds D to F for the move
+// just tried, from those.
+// A trial costs one launch, bound by the latencies of roots, factors and
+// spectrum: 8.6 us for one particle in an 80^3 mesh.  The factor tables, the
+// pass and the sum as kernels of their own took 7.5, 4.6 and 3.8 us (the
+// call 31 us, now 24.5).  Two points per thread and twice the blocks
+// measured 8.8 us.
+constexpr int kMcPoints = 4;
+constexpr int kMcTile = 256 * kMcPoints;
+// mesh rows that a tile can touch
+__host__ __device__ inline int mc_rows(int hx) { return (kMcTile - 1) / hx + 2; }
+
+__device__ __forceinline__ int mc_ia(const McMove &mv, int a) {
+  return mv.natm <= kMcArg ? mv.ia_v[a] : mv.ia[a];
+}
+__device__ __forceinline__ double mc_rtm(const McMove &mv, int k) {
+  return mv.natm <= kMcArg ? mv.rtm_v[k] : mv.rtm[k];
+}
+
 template <typename R, int ORDER>
-__global__ void __launch_bounds__(256) k_mc_kfac(const SysDev *__restrict__ sys, int natm,
-                                                 const int *__restrict__ ia,
-                                                 const double *__restrict__ rtm,
-                                                 double2 *__restrict__ fac) {
-  const SysDev &V = sys[blockIdx.z];
-  const SpmeGeom g = V.sg;
-  const int s0 = g.s[0], s1 = g.s[1], s2 = g.s[2], ns = s0 + s1 + s2;
-  const int total = natm * 2 * ns;
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < total; t += gridDim.x * blockDim.x) {
-    const int row = t / ns, k0 = t - row * ns;
-    const int a = row >> 1, trial = row & 1;
-    const int m = k0 < s0 ? 0 : (k0 < s0 + s1 ? 1 : 2);
-    const int k = k0 - (m == 0 ? 0 : (m == 1 ? s0 : s0 + s1));
-    const int i = ia[a];
-    int mm[3];
-    double fr[3];
-    mesh_coords(trial ? rtm + 3 * a : V.ro + 3 * i, g, mm, fr);
+__device__ __forceinline__ void mc_rec_body(const SysDev &V, const McMove &mv, int chunk,
+                                            double2 *__restrict__ F, double *__restrict__ old,
+                                            bool apply, double *__restrict__ part, int blk,
+                                            int nblk) {
+  extern __shared__ __align__(16) unsigned char mc_lds[];
+  const SpmeGeom &g = V.sg;
+  const SpmeAxes &ax = V.ax;
+  const int s0 = g.s[0], s1 = g.s[1], s2 = g.s[2], hx = V.hx;
+  const unsigned n = (unsigned)hx * s1 * s2;
+  const int rows = mc_rows(hx);
+  double2 *root = reinterpret_cast<double2 *>(mc_lds);        // [s0 + s1 + s2]
+  double2 *fx = root + s0 + s1 + s2;                          // [2 chunk][hx]
+  double2 *fr = fx + 2 * chunk * hx;                          // [2 chunk][rows]
+  for (int k = threadIdx.x; k < s0 + s1 + s2; k += blockDim.x) {
+    const int m = k < s0 ? 0 : (k < s0 + s1 ? 1 : 2);
+    const int ph = k - (m == 0 ? 0 : (m == 1 ? s0 : s0 + s1));
+    double sn, cs;
+    sincospi(-2.0 * (double)ph / (double)(m == 0 ? s0 : (m == 1 ? s1 : s2)), &sn, &cs);
+    root[k] = make_double2(cs, sn);
+  }
+  if (!apply && blk == 0)
+    for (int k = threadIdx.x; k < 3 * mv.natm; k += blockDim.x)
+      old[k] = V.ro[3 * mc_ia(mv, k / 3) + k % 3];
+  // the factor of an axis of sm points (its roots at rt) at wavenumber k
+  auto factor = [&](double x, double dk, int sm, const double2 *rt, int k) -> double2 {
+    const double u = dk * x;
+    const double f = floor(u);
+    int pt = (int)f % sm;
+    pt += pt < 0 ? sm : 0;
     R w[ORDER];
-    bspline<R, ORDER>((R)fr[m], w, nullptr);
-    const int sm = g.s[m];
+    bspline<R, ORDER>((R)(u - f), w, nullptr);
+    // the phase k (pt - j) reduced to [0, s): pt, k < s < 2^15
+    int ph = (int)(((unsigned)k * (unsigned)pt) % (unsigned)sm);
     double re = 0.0, im = 0.0;
 #pragma unroll
     for (int j = 0; j < ORDER; ++j) {
-      int pt = (mm[m] - j) % sm;
-      pt += pt < 0 ? sm : 0;
-      // the phase k pt / s reduced exactly
-      const int ph = (int)(((long long)k * pt) % sm);
-      double sn, cs;
-      sincospi(-2.0 * (double)ph / (double)sm, &sn, &cs);
-      re += (double)w[j] * cs;
-      im += (double)w[j] * sn;
+      const double2 c = rt[ph];
+      re += (double)w[j] * c.x;
+      im += (double)w[j] * c.y;
+      ph -= k;
+      ph += ph < 0 ? sm : 0;
     }
-    if (m == 0) {
-      const double q = (double)(R)V.q[i];
-      re *= q;
-      im *= q;
-    }
-    fac[t] = make_double2(re, im);
-  }
-}
-
-// One pass over the kept spectrum F (the complex mesh's layout, kx
-// fastest, fewer than 2^31 points): apply == 1 adds D to F (an accepted
-// move); apply == 0 writes this block's part of the energy change to
-// part[2 * blockIdx.x] (and 0 to part[2 * blockIdx.x + 1]), summed by
-// k_mc_pair_sum in a fixed order.  The grid is fixed, so each thread's
-// points and the sums' order are too.  One replica (an engine's MC move).
-template <typename R>
-__global__ void __launch_bounds__(256) k_mc_kdelta(const SysDev *__restrict__ sys, int natm,
-                                                   const double2 *__restrict__ fac, void *spec,
-                                                   int apply, double *__restrict__ part) {
-  const SysDev &V = sys[0];
-  const SpmeGeom g = V.sg;
-  const SpmeAxes &ax = V.ax;
-  const int s0 = g.s[0], s1 = g.s[1], s2 = g.s[2], hx = V.hx, ns = s0 + s1 + s2;
-  cplx<R> *__restrict__ F = (cplx<R> *)spec;
-  const unsigned n = (unsigned)hx * s1 * s2;
+    return make_double2(re, im);
+  };
   double acc = 0.0;
-  for (unsigned e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x) {
-    const unsigned r = e / (unsigned)hx;
-    const int kx = (int)(e - r * (unsigned)hx);
-    const unsigned kzu = r / (unsigned)s1;
-    const int ky = (int)(r - kzu * (unsigned)s1), kz = (int)kzu;
-    double dr = 0.0, di = 0.0;
-    for (int a = 0; a < natm; ++a) {
+  for (unsigned e0 = (unsigned)blk * kMcTile; e0 < n; e0 += (unsigned)nblk * kMcTile) {
+    const unsigned r0 = e0 / (unsigned)hx;
+    const unsigned r1 = (min(e0 + kMcTile, n) - 1) / (unsigned)hx;
+    const int nr = (int)(r1 - r0) + 1, ne = hx + nr;
+    double2 v[kMcPoints];
+    double dr[kMcPoints], di[kMcPoints];
 #pragma unroll
-      for (int trial = 0; trial < 2; ++trial) {
-        const double2 *f = fac + (size_t)(2 * a + trial) * ns;
-        const double2 cx = f[kx], cy = f[s0 + ky], cz = f[s0 + s1 + kz];
-        const double pr = cx.x * cy.x - cx.y * cy.y, pi = cx.x * cy.y + cx.y * cy.x;
-        const double tr = pr * cz.x - pi * cz.y, ti = pr * cz.y + pi * cz.x;
-        dr += trial ? tr : -tr;
-        di += trial ? ti : -ti;
+    for (int u = 0; u < kMcPoints; ++u) {
+      v[u] = F[min(e0 + u * 256 + threadIdx.x, n - 1)];
+      dr[u] = 0.0;
+      di[u] = 0.0;
+    }
+    for (int a0 = 0; a0 < mv.natm; a0 += chunk) {
+      const int na = min(chunk, mv.natm - a0);
+      // the roots are written, the last chunk's factors read
+      __syncthreads();
+      for (int t = threadIdx.x; t < 2 * na * ne; t += blockDim.x) {
+        const int row = t / ne, k = t - row * ne;
+        const int a = a0 + (row >> 1), i = mc_ia(mv, a);
+        double r[3];
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+          r[m] = (row & 1) ? mc_rtm(mv, 3 * a + m) : (apply ? old[3 * a + m] : V.ro[3 * i + m]);
+        if (k < hx) {
+          const double2 c = factor(r[0], g.dkdr[0], s0, root, k);
+          const double q = (double)(R)V.q[i];
+          fx[row * hx + k] = make_double2(c.x * q, c.y * q);
+        } else {
+          const unsigned rr = r0 + (unsigned)(k - hx), kz = rr / (unsigned)s1;
+          const double2 cy = factor(r[1], g.dkdr[1], s1, root + s0,
+                                    (int)(rr - kz * (unsigned)s1));
+          const double2 cz = factor(r[2], g.dkdr[2], s2, root + s0 + s1, (int)kz);
+          fr[row * rows + k - hx] =
+              make_double2(cy.x * cz.x - cy.y * cz.y, cy.x * cz.y + cy.y * cz.x);
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < kMcPoints; ++u) {
+        const unsigned e = min(e0 + u * 256 + threadIdx.x, n - 1), r = e / (unsigned)hx;
+        const int kx = (int)(e - r * (unsigned)hx), kr = (int)(r - r0);
+        for (int a = 0; a < 2 * na; a += 2) {
+          const double2 x0 = fx[a * hx + kx], y0 = fr[a * rows + kr];
+          const double2 x1 = fx[(a + 1) * hx + kx], y1 = fr[(a + 1) * rows + kr];
+          dr[u] += (x1.x * y1.x - x1.y * y1.y) - (x0.x * y0.x - x0.y * y0.y);
+          di[u] += (x1.x * y1.y + x1.y * y1.x) - (x0.x * y0.y + x0.y * y0.x);
+        }
       }
     }
-    const cplx<R> v = F[e];
-    if (apply) {
-      F[e] = {(R)((double)v.x + dr), (R)((double)v.y + di)};
-    } else {
-      const int nx = kx, ny = min(ky, s1 - ky), nz = min(kz, s2 - kz);
-      const double m2 = ax.kk[0][nx] + ax.kk[1][ny] + ax.kk[2][nz];
+#pragma unroll
+    for (int u = 0; u < kMcPoints; ++u) {
+      const unsigned e = e0 + u * 256 + threadIdx.x;
+      if (e >= n) continue;
+      if (apply) {
+        F[e] = make_double2(v[u].x + dr[u], v[u].y + di[u]);
+        continue;
+      }
+      const unsigned r = e / (unsigned)hx, kzu = r / (unsigned)s1;
+      const int kx = (int)(e - r * (unsigned)hx), ky = (int)(r - kzu * (unsigned)s1);
+      const int ny = min(ky, s1 - ky), nz = min((int)kzu, s2 - (int)kzu);
+      const double m2 = ax.kk[0][kx] + ax.kk[1][ny] + ax.kk[2][nz];
       if (m2 > 0.0) {
-        const double mf = ax.fac0 * ax.g[0][nx] * ax.g[1][ny] * ax.g[2][nz] / m2;
-        const double wt = (nx == 0 || 2 * nx == s0) ? 0.5 : 1.0;
-        acc += wt * mf * (2.0 * ((double)v.x * dr + (double)v.y * di) + (dr * dr + di * di));
+        const double mf = ax.fac0 * ax.g[0][kx] * ax.g[1][ny] * ax.g[2][nz] / m2;
+        const double wt = (kx == 0 || 2 * kx == s0) ? 0.5 : 1.0;
+        acc += wt * mf * (2.0 * (v[u].x * dr[u] + v[u].y * di[u]) +
+                          (dr[u] * dr[u] + di[u] * di[u]));
       }
     }
   }
   if (apply) return;
   __shared__ double sh[256 / 64];
   const double t = block_sum(acc, sh);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = t;
-    part[2 * blockIdx.x + 1] = 0.0;
-  }
+  if (threadIdx.x == 0) part[blk] = t;
+}
+
+template <typename R, int ORDER>
+__global__ void __launch_bounds__(256) k_mc_rec(const SysDev *__restrict__ sys, const McMove mv,
+                                                int chunk, double2 *spec, double *old,
+                                                double *part) {
+  mc_rec_body<R, ORDER>(sys[0], mv, chunk, spec, old, false, part, (int)blockIdx.x,
+                        (int)gridDim.x);
 }
 
 // UTwoBodyANew/UTwoBodyAOld (Src/denergy.F90:289-495) for a trial move of
 // natm particles: each moved particle against its list partners that stay
 // (u at the trial position minus u at the current one), plus the pairs of
 // moved particles among themselves, each once (both trial minus both
-// current, as its lptmdutwob branch).  The table is walked as the
-// reference walks ubuf, from the pair's first interval to the first with
-// r2 >= zlow, in FP64 on both precision paths.  A trial pair inside the
-// hard core or below r2umin is an overlap (its goto 400).  One block,
-// lanes over list entries, a fixed-order sum.
-__device__ __forceinline__ double mc_pair_u(const SysDev &V, int ti, int tj, double dx,
-                                            double dy, double dz, int &ovl) {
+// current, as its lptmdutwob branch), in FP64 on both precision paths.  A
+// trial pair inside the hard core or below r2umin is an overlap (its goto
+// 400).  One block and a list of tens of partners: the time is the chain
+// of dependent loads, so the pair records are staged in LDS while the
+// particle's own data arrive, a lane's first list entry is loaded with the
+// list's length, and both positions of a pair are looked up together, by
+// the bin of r2 (the interval the reference's walk from the pair's first
+// interval to the first with r2 >= zlow stops at): 6.8 us with 9 partners,
+// 9.3 with that walk, the two positions in turn and the move in host memory.
+// One pair: u(d[0]) - u(d[1]), trial less current.
+__device__ __forceinline__ double mc_pair_du(const SysDev &V, const PairRec *rec_s,
+                                             const int *pidx_s, int ti, int tj,
+                                             double (&d)[2][3], int &ovl) {
   const TableDev &t = V.tab;
-  const double r2 = pbcr2(dx, dy, dz, V.box);
-  const bool in = V.nlsem == 0 ? !(r2 > t.rcut2) : (r2 < t.rcut2);
-  if (!in) return 0.0;
-  const int p = t.pairidx[ti * t.npt + tj];
-  if (r2 < t.r2atat[p] || r2 < t.r2umin[p]) {
-    ovl = 1;
-    return 0.0;
+  const int p = pidx_s[ti * t.npt + tj], nbin = t.nbin;
+  const PairRec R = rec_s[p];
+  const unsigned short *bins = reinterpret_cast<const unsigned short *>((const uint4 *)t.img) +
+                               (size_t)p * nbin;
+  const double *zl = (const double *)t.zlow + R.off;
+  double r2[2], r2c[2], z0[2], z1[2], zv[2], u[2];
+  int bk[2], iv[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    r2[s] = pbcr2(d[s][0], d[s][1], d[s][2], V.box);
+    r2c[s] = fmax(r2[s], R.lo);
+    const float sf = __builtin_amdgcn_rcpf((float)r2c[s]);
+    bk[s] = bins[(int)fminf(fmaxf((sf - R.s_lo) * R.s_inv, 0.0f), (float)(nbin - 1))];
   }
-  const int o = t.off[p], n = t.nint[p];
-  int k = 0;
-  while (k < n - 1 && r2 < t.zlow[o + k]) ++k;
-  const double *c = t.coef + (size_t)(o + k) * kCoefStride;
-  const double d = r2 - t.zlow[o + k];
-  return c[0] + d * (c[1] + d * (c[2] + d * (c[3] + d * (c[4] + d * c[5]))));
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int kb = bk[s] & (kSlowBin - 1);
+    z0[s] = zl[kb];
+    z1[s] = zl[min(kb + 1, R.nint - 1)];
+  }
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int kb = bk[s] & (kSlowBin - 1);
+    if (bk[s] & kSlowBin) {
+      iv[s] = find_interval([&](int k) -> double { return zl[k]; }, R.nint, r2c[s], kb);
+      zv[s] = zl[iv[s]];
+    } else {
+      const bool at = r2c[s] >= z0[s];
+      iv[s] = at ? kb : min(kb + 1, R.nint - 1);
+      zv[s] = at ? z0[s] : z1[s];
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const double2 *q = reinterpret_cast<const double2 *>((const double *)t.coef) +
+                       (size_t)(kCoefStride / 2) * (R.off + iv[s]);
+    const double2 a = q[0], b = q[1], c = q[2];
+    const double x = r2[s] - zv[s];
+    u[s] = a.x + x * (a.y + x * (b.x + x * (b.y + x * (c.x + x * c.y))));
+    const bool in = V.nlsem == 0 ? !(r2[s] > t.rcut2) : (r2[s] < t.rcut2);
+    const bool ov = in && (r2[s] < R.r2at || r2[s] < R.r2um);
+    if (s == 0) ovl |= ov ? 1 : 0;
+    if (!in || ov) u[s] = 0.0;
+  }
+  return u[0] - u[1];
 }
 
-__global__ void __launch_bounds__(256) k_mc_pair(const SysDev *__restrict__ sys, int natm,
-                                                const int *__restrict__ ia_in,
-                                                const double *__restrict__ rtm_in,
+__global__ void __launch_bounds__(256) k_mc_pair(const SysDev *__restrict__ sys, const McMove mv,
                                                 double *__restrict__ out,
                                                 double *__restrict__ part) {
   const SysDev &V = sys[blockIdx.z];
-  // up to kMcStage moved particles are copied into LDS once per block, so
-  // the move may come from host memory (the pinned staging) and the loops
-  // below read it from LDS
-  __shared__ int ia_s[kMcStage];
-  __shared__ double rtm_s[3 * kMcStage];
-  const bool staged = natm <= kMcStage;
+  // up to kMcArg moved particles are in the arguments and copied into LDS
+  // once per block, more are read from device memory
+  __shared__ int ia_s[kMcArg];
+  __shared__ double rtm_s[3 * kMcArg];
+  __shared__ PairRec rec_s[MFE_MAX_PAIRS];
+  __shared__ int pidx_s[MFE_MAX_TYPES * MFE_MAX_TYPES];
+  const TableDev &tab = V.tab;
+  const int natm = mv.natm;
+  const bool staged = natm <= kMcArg;
+  for (int k = threadIdx.x; k < tab.nptpt; k += blockDim.x) rec_s[k] = tab.rec[k];
+  for (int k = threadIdx.x; k < tab.npt * tab.npt; k += blockDim.x) pidx_s[k] = tab.pairidx[k];
   if (staged) {
-    for (int k = threadIdx.x; k < natm; k += blockDim.x) ia_s[k] = ia_in[k];
-    for (int k = threadIdx.x; k < 3 * natm; k += blockDim.x) rtm_s[k] = rtm_in[k];
+    for (int k = threadIdx.x; k < natm; k += blockDim.x) ia_s[k] = mv.ia_v[k];
+    for (int k = threadIdx.x; k < 3 * natm; k += blockDim.x) rtm_s[k] = mv.rtm_v[k];
   }
   __syncthreads();
-  const int *ia = staged ? ia_s : ia_in;
-  const double *rtm = staged ? rtm_s : rtm_in;
+  const int *ia = staged ? ia_s : mv.ia;
+  const double *rtm = staged ? rtm_s : mv.rtm;
   const int np = V.np;
-  const int stride = gridDim.x * blockDim.x;
   // cell-list semantics (UTwoBodyANew/OldCellList, Src/denergy.F90:728-928):
   // every particle within rcut of the old or new position, as the cells
   // around each position hold them; Verlet list (UTwoBodyANew/Old): the
-  // moved particle's list partners
-  const bool all = V.nlsem == 1;
+  // moved particle's list partners, on all of the block's lanes for one
+  // moved particle, else a wavefront per moved particle
+  const bool all = V.nlsem == 1, whole = all || natm == 1;
+  const int l0 = all ? (int)(blockIdx.x * blockDim.x + threadIdx.x)
+                     : (whole ? (int)threadIdx.x : (int)(threadIdx.x & 63));
+  const int nl = all ? (int)(gridDim.x * blockDim.x) : (whole ? (int)blockDim.x : 64);
+  const int a1 = whole ? 1 : (int)(blockDim.x >> 6);
   double acc = 0.0;
-  int ovl = 0, ovl_old = 0;
-  for (int a = 0; a < natm; ++a) {
+  int ovl = 0;
+  for (int a = whole ? 0 : (int)(threadIdx.x >> 6); a < natm; a += a1) {
     const int i = ia[a], t = V.c_pos[i], ti = V.type[i];
     const double xo = V.ro[3 * i], yo = V.ro[3 * i + 1], zo = V.ro[3 * i + 2];
     const double xn = rtm[3 * a], yn = rtm[3 * a + 1], zn = rtm[3 * a + 2];
     const int n = all ? np : V.nn[t];
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += stride) {
+    const int first = all ? 0 : V.nbr[(size_t)min(l0, V.maxnn - 1) * np + t];
+    for (int k = l0; k < n; k += nl) {
       int jp, tj;
       double xj, yj, zj;
       if (all) {
@@ -1853,7 +1955,8 @@ __global__ void __launch_bounds__(256) k_mc_pair(const SysDev *__restrict__ sys,
         yj = V.ro[3 * k + 1];
         zj = V.ro[3 * k + 2];
       } else {
-        const int j = (int)((unsigned)V.nbr[(size_t)k * np + t] & kNbrIdxMask);  // cell-ordered slot
+        const int e = k == l0 ? first : V.nbr[(size_t)k * np + t];
+        const int j = (int)((unsigned)e & kNbrIdxMask);  // cell-ordered slot
         jp = V.c_sorted[j];
         tj = V.type_s[j];
         xj = V.ro_s[3 * j];
@@ -1863,19 +1966,22 @@ __global__ void __launch_bounds__(256) k_mc_pair(const SysDev *__restrict__ sys,
       bool moved = false;
       for (int b = 0; b < natm; ++b) moved |= ia[b] == jp;
       if (moved) continue;
-      acc += mc_pair_u(V, ti, tj, xn - xj, yn - yj, zn - zj, ovl) -
-             mc_pair_u(V, ti, tj, xo - xj, yo - yj, zo - zj, ovl_old);
+      double d[2][3] = {{xn - xj, yn - yj, zn - zj}, {xo - xj, yo - yj, zo - zj}};
+      acc += mc_pair_du(V, rec_s, pidx_s, ti, tj, d, ovl);
     }
   }
   for (int q = blockIdx.x == 0 ? (int)threadIdx.x : natm * natm; q < natm * natm;
        q += blockDim.x) {
     const int a = q / natm, b = q - a * natm;
     if (b <= a) continue;
-    const int i = ia[a], j = ia[b], ti = V.type[i], tj = V.type[j];
-    acc += mc_pair_u(V, ti, tj, rtm[3 * a] - rtm[3 * b], rtm[3 * a + 1] - rtm[3 * b + 1],
-                     rtm[3 * a + 2] - rtm[3 * b + 2], ovl) -
-           mc_pair_u(V, ti, tj, V.ro[3 * i] - V.ro[3 * j], V.ro[3 * i + 1] - V.ro[3 * j + 1],
-                     V.ro[3 * i + 2] - V.ro[3 * j + 2], ovl_old);
+    const int i = ia[a], j = ia[b];
+    double d[2][3];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      d[0][m] = rtm[3 * a + m] - rtm[3 * b + m];
+      d[1][m] = V.ro[3 * i + m] - V.ro[3 * j + m];
+    }
+    acc += mc_pair_du(V, rec_s, pidx_s, V.type[i], V.type[j], d, ovl);
   }
   __shared__ double red[256 / 64];
   for (int w = 32; w > 0; w >>= 1) acc += __shfl_down(acc, w, 64);
@@ -2619,23 +2725,12 @@ __global__ void __launch_bounds__(kBlock) k_move(const SysDev *__restrict__ sys,
 // minimum image of new - old (one shift per axis, as PBCr2), so the skin
 // test that follows decides whether the list is rebuilt.  The new
 // positions are ro_new (a host upload), or, with ro_new null, the current
-// ones with the natm <= kMcStage particles ia moved to rtm (an accepted MC
-// move, staged in LDS, so it may come from host memory).
-__global__ void __launch_bounds__(kBlock) k_set_positions(const SysDev *__restrict__ sys,
-                                                          const double *__restrict__ ro_new,
-                                                          int natm, const int *__restrict__ ia,
-                                                          const double *__restrict__ rtm) {
+// ones with the move's particles (at most kMcArg) at their new places.
+__device__ __forceinline__ void set_positions_body(const SysDev &V,
+                                                   const double *__restrict__ ro_new,
+                                                   const McMove *mv) {
 #pragma clang fp contract(off)
-  const SysDev &V = sys[blockIdx.z];
-  if ((int)blockIdx.x >= V.nblk_np) return;
   __shared__ double sh[kBlock];
-  __shared__ int ia_s[kMcStage];
-  __shared__ double rtm_s[3 * kMcStage];
-  if (!ro_new) {
-    for (int k = threadIdx.x; k < natm; k += blockDim.x) ia_s[k] = ia[k];
-    for (int k = threadIdx.x; k < 3 * natm; k += blockDim.x) rtm_s[k] = rtm[k];
-    __syncthreads();
-  }
   const Box b = V.box;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   double r2 = 0.0;
@@ -2655,10 +2750,10 @@ __global__ void __launch_bounds__(kBlock) k_set_positions(const SysDev *__restri
     } else {
 #pragma unroll
       for (int m = 0; m < 3; ++m) xn[m] = xo[m];
-      for (int a = 0; a < natm; ++a)
-        if (ia_s[a] == i) {
+      for (int a = 0; a < mv->natm; ++a)
+        if (mv->ia_v[a] == i) {
 #pragma unroll
-          for (int m = 0; m < 3; ++m) xn[m] = rtm_s[3 * a + m];
+          for (int m = 0; m < 3; ++m) xn[m] = mv->rtm_v[3 * a + m];
         }
     }
 #pragma unroll
@@ -2682,6 +2777,29 @@ __global__ void __launch_bounds__(kBlock) k_set_positions(const SysDev *__restri
   }
   const double mx = block_max(r2, sh);
   if (threadIdx.x == 0) V.part[V.off_move + blockIdx.x] = mx;
+}
+
+__global__ void __launch_bounds__(kBlock) k_set_positions(const SysDev *__restrict__ sys,
+                                                          const double *__restrict__ ro_new) {
+  const SysDev &V = sys[blockIdx.z];
+  if ((int)blockIdx.x < V.nblk_np) set_positions_body(V, ro_new, nullptr);
+}
+
+// An accepted move: the first nset blocks (V.nblk_np, or none where the
+// positions are set apart) place a move of up to kMcArg particles and update
+// the displacements, the others add the trial's change to the kept spectrum
+// (none where no spectrum is kept).  That change is taken from `old`, the
+// positions before the move, so the two parts are independent: 9.3 us in one
+// launch (50000 particles, 80^3 mesh), 4.6 and 5.9 us in two.
+template <typename R, int ORDER>
+__global__ void __launch_bounds__(kBlock) k_mc_accept(const SysDev *__restrict__ sys,
+                                                      const McMove mv, int nset, int chunk,
+                                                      double2 *spec, double *old) {
+  if ((int)blockIdx.x < nset)
+    set_positions_body(sys[0], nullptr, &mv);
+  else
+    mc_rec_body<R, ORDER>(sys[0], mv, chunk, spec, old, true, nullptr, (int)blockIdx.x - nset,
+                          (int)gridDim.x - nset);
 }
 
 // NList's r2max2 (Src/nlist.F90:602-608) is the largest r2 that is not a
@@ -2825,9 +2943,13 @@ __global__ void __launch_bounds__(kReduceThreads) k_reduce_finalize(const SysDev
 // so the rebuild's first phase needs no barrier after it.  One
 // 1024-thread block per CU, all resident, as the rebuild's grid barriers
 // require.
+// mode < 0: no finalize (new positions from the host or an accepted MC
+// move).  hflags, if given, is pinned host memory for the flags as they
+// stand when the test did not fire, which spares the host a copy; where
+// hflags[1] says that it fired, the host reads them after the rebuild.
 __global__ void __launch_bounds__(kReduceThreads) k_finalize_rebuild(
     const SysDev *__restrict__ sys, int energy, int bd, int mode, double dt, int split,
-    unsigned *bar, int spin) {
+    unsigned *bar, int spin, int *hflags) {
   const SysDev &V = sys[0];
   const int nb = V.nblk_np;
   const double *pmove = V.part + V.off_move, *pcand = V.part + V.off_skin;
@@ -2840,7 +2962,7 @@ __global__ void __launch_bounds__(kReduceThreads) k_finalize_rebuild(
   }
   if (blockIdx.x == 0) {
     ph_reduce(V, energy, 1, bd);
-  } else {
+  } else if (mode >= 0) {
     const double es[3] = {0.0, 0.0, 0.0};
     const int stride = ((int)gridDim.x - 1) * kReduceThreads;
     for (int i = ((int)blockIdx.x - 1) * kReduceThreads + (int)threadIdx.x; i < V.np;
@@ -2862,7 +2984,13 @@ __global__ void __launch_bounds__(kReduceThreads) k_finalize_rebuild(
     M1 = fmax(M1, mx_s[0][w]);
     M2 = fmax(M2, mx_s[1][w]);
   }
-  if (!(sqrt(M1) + sqrt(M2) > V.drnlist)) return;
+  const bool fired = sqrt(M1) + sqrt(M2) > V.drnlist;
+  if (hflags && blockIdx.x == 0 && threadIdx.x == 0) {
+    hflags[0] = V.flags[0];
+    hflags[1] = fired ? 1 : 0;
+    hflags[2] = V.flags[2];
+  }
+  if (!fired) return;
   // after a failed rebuild earlier in the call the list stays void
   if (__hip_atomic_load(&V.flags[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ERR_SYNC)
     return;
@@ -3536,43 +3664,76 @@ void launch_mc_place(const Group &g, int natm, const int *ia, const double *rtm,
                      ro_stage);
 }
 
-void launch_mc_kfac(const Group &g, int natm, const int *ia, const double *rtm, void *fac) {
-  const int total = natm * 2 * (g.mc_s[0] + g.mc_s[1] + g.mc_s[2]);
-  const dim3 gr(std::max(1, std::min((total + 255) / 256, 1024)), 1, g.R);
-#define MFE_MC(R, O)                                                                         \
-  case O:                                                                                    \
-    hipLaunchKernelGGL((k_mc_kfac<R, O>), gr, dim3(256), 0, g.stream, g.d, natm, ia, rtm,     \
-                       (double2 *)fac);                                                      \
-    break;
-  if (g.prec == MFE_PREC_MIXED) {
-    switch (g.order) { MFE_MC(float, 3) MFE_MC(float, 4) MFE_MC(float, 5) MFE_MC(float, 6)
-                       MFE_MC(float, 7) MFE_MC(float, 8) }
-  } else {
-    switch (g.order) { MFE_MC(double, 3) MFE_MC(double, 4) MFE_MC(double, 5) MFE_MC(double, 6)
-                       MFE_MC(double, 7) MFE_MC(double, 8) }
+// moved particles whose factors a block holds at a time: up to eight, as
+// many as 32 KB of LDS take beside the roots
+static int mc_chunk(const Group &g, int natm) {
+  const int hx = g.mc_s[0] / 2 + 1;
+  const size_t per = 2 * (size_t)(hx + mc_rows(hx)) * sizeof(double2);
+  return (int)std::max<size_t>(1, std::min<size_t>({(size_t)natm, 8, (32 * 1024) / per}));
+}
+static size_t mc_lds_bytes(const Group &g, int chunk) {
+  const int hx = g.mc_s[0] / 2 + 1;
+  return ((size_t)(g.mc_s[0] + g.mc_s[1] + g.mc_s[2]) +
+          2 * (size_t)chunk * (hx + mc_rows(hx))) * sizeof(double2);
+}
+static int mc_rec_blocks(const Group &g) {
+  const size_t n = (size_t)(g.mc_s[0] / 2 + 1) * g.mc_s[1] * g.mc_s[2];
+  return (int)std::min<size_t>((n + kMcTile - 1) / kMcTile, kMcRecBlocks);
+}
+
+// dynamic LDS above the default limit (meshes of about 1000 points along
+// each axis)
+static void mc_allow_lds(const void *kernel, size_t lds) {
+  if (lds > 60 * 1024)
+    (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+}
+
+// the instance of the engine's precision and spline order
+#define MFE_MC_CASES(T)                                                          \
+  switch (g.order) {                                                             \
+    MFE_MC(T, 3) MFE_MC(T, 4) MFE_MC(T, 5) MFE_MC(T, 6) MFE_MC(T, 7) MFE_MC(T, 8) \
   }
+
+int launch_mc_rec(const Group &g, const McMove &mv, void *spec, double *old, double *part) {
+  const int nb = mc_rec_blocks(g), chunk = mc_chunk(g, mv.natm);
+  const size_t lds = mc_lds_bytes(g, chunk);
+#define MFE_MC(T, O)                                                                       \
+  case O:                                                                                  \
+    mc_allow_lds((const void *)k_mc_rec<T, O>, lds);                                       \
+    hipLaunchKernelGGL((k_mc_rec<T, O>), dim3(nb), dim3(256), lds, g.stream, g.d, mv,      \
+                       chunk, (double2 *)spec, old, part);                                 \
+    break;
+  if (g.prec == MFE_PREC_MIXED) { MFE_MC_CASES(float) }
+  else { MFE_MC_CASES(double) }
+#undef MFE_MC
+  return nb;
+}
+
+void launch_mc_accept(const Group &g, const McMove &mv, bool place, void *spec, double *old) {
+  const int nset = place ? g.np_blocks : 0, nb = nset + (spec ? mc_rec_blocks(g) : 0);
+  if (!nb) return;
+  const int chunk = spec ? mc_chunk(g, mv.natm) : 1;
+  const size_t lds = spec ? mc_lds_bytes(g, chunk) : 0;
+#define MFE_MC(T, O)                                                                       \
+  case O:                                                                                  \
+    mc_allow_lds((const void *)k_mc_accept<T, O>, lds);                                    \
+    hipLaunchKernelGGL((k_mc_accept<T, O>), dim3(nb), dim3(kBlock), lds, g.stream, g.d,    \
+                       mv, nset, chunk, (double2 *)spec, old);                             \
+    return;
+  if (spec && g.prec == MFE_PREC_MIXED) { MFE_MC_CASES(float) }
+  else if (spec) { MFE_MC_CASES(double) }
+  // without a spectrum any instance places the move
+  switch (4) { MFE_MC(double, 4) }
 #undef MFE_MC
 }
+#undef MFE_MC_CASES
 
-void launch_mc_kdelta(const Group &g, int natm, const void *fac, void *spec, bool apply,
-                      double *part, double *out) {
-  // the kept spectrum is FP64 on both precision paths
-  const dim3 gr(kMcPairBlocks);
-  hipLaunchKernelGGL(k_mc_kdelta<double>, gr, dim3(256), 0, g.stream, g.d, natm,
-                     (const double2 *)fac, spec, apply ? 1 : 0, part);
-  if (!apply)
-    hipLaunchKernelGGL(k_mc_pair_sum, dim3(1), dim3(64), 0, g.stream, part, kMcPairBlocks, out);
-}
-
-void launch_mc_pair(const Group &g, int natm, const int *ia, const double *rtm, double *out,
-                    double *part, bool all) {
+void launch_mc_pair(const Group &g, const McMove &mv, double *out, double *part, bool all) {
   if (!all) {
-    hipLaunchKernelGGL(k_mc_pair, grid(1, g), dim3(256), 0, g.stream, g.d, natm, ia, rtm, out,
-                       part);
+    hipLaunchKernelGGL(k_mc_pair, grid(1, g), dim3(256), 0, g.stream, g.d, mv, out, part);
     return;
   }
-  hipLaunchKernelGGL(k_mc_pair, dim3(kMcPairBlocks), dim3(256), 0, g.stream, g.d, natm, ia, rtm,
-                     out, part);
+  hipLaunchKernelGGL(k_mc_pair, dim3(kMcPairBlocks), dim3(256), 0, g.stream, g.d, mv, out, part);
   hipLaunchKernelGGL(k_mc_pair_sum, dim3(1), dim3(64), 0, g.stream, part, kMcPairBlocks, out);
 }
 
@@ -3725,12 +3886,12 @@ void launch_reduce_finalize(const Group &g, unsigned flags, bool skin, bool bd, 
 }
 
 bool launch_finalize_rebuild(const Group &g, unsigned flags, bool bd, int mode, double dt,
-                             bool split) {
+                             bool split, int *hflags) {
   if (!(g.R == 1 && g.rebuild_bar && g.flags && g.ncu > 1)) return false;
   const int energy = (flags & (MFE_ENERGY | MFE_VIRIAL)) ? 1 : 0;
   hipLaunchKernelGGL(k_finalize_rebuild, dim3(g.ncu), dim3(kReduceThreads), 0, g.stream, g.d,
                      energy, bd ? 1 : 0, mode, dt, split ? 1 : 0, g.rebuild_bar,
-                     g.sync_spin >= 0 ? g.sync_spin : kGridSpin);
+                     g.sync_spin >= 0 ? g.sync_spin : kGridSpin, hflags);
   return true;
 }
 
@@ -3830,12 +3991,7 @@ int adjoint_blocks(int np) { return (np + kAdjPer - 1) / kAdjPer; }
 
 void launch_set_positions(const Group &g, const double *ro_new) {
   hipLaunchKernelGGL(k_set_positions, grid(g.np_blocks, g), dim3(kBlock), 0, g.stream, g.d,
-                     ro_new, 0, (const int *)nullptr, (const double *)nullptr);
-}
-
-void launch_set_positions_moved(const Group &g, int natm, const int *ia, const double *rtm) {
-  hipLaunchKernelGGL(k_set_positions, grid(g.np_blocks, g), dim3(kBlock), 0, g.stream, g.d,
-                     (const double *)nullptr, natm, ia, rtm);
+                     ro_new);
 }
 
 void launch_skin(const Group &g) {
