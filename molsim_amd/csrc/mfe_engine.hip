@@ -166,7 +166,7 @@ void free_all(mfe_engine *e) {
   dfree(e->bd_fac1); dfree(e->bd_fac2); dfree(e->bd_noise); dfree(e->d_sys);
   dfree(e->ro_stage);
   dfree(e->knot_c); dfree(e->phi_rec); dfree(e->adj_phi); dfree(e->adj_dq);
-  dfree(e->adj_part); dfree(e->adj_out);
+  dfree(e->adj_part); dfree(e->adj_out); dfree(e->adj_dro);
   dfree(e->fm_ro); dfree(e->fm_tgt); dfree(e->fm_fld); dfree(e->fm_res); dfree(e->fm_res_s);
   dfree(e->fm_vec); dfree(e->fm_part); dfree(e->fm_acc); dfree(e->fm_qr);
   if (e->h_en) (void)hipHostFree(e->h_en);
@@ -1914,14 +1914,16 @@ int mfe_adjoint(mfe_engine *e, double *dE_dq, double *dE_dzat, double *dE_dsigat
   return guarded(e, [&]() -> int {
     MFE_HIP_TRY(hipSetDevice(e->device));
     const int ncol = 1 + 2 * e->npt + e->nptpt * e->nknot;
-    const int nb = mfe::adjoint_blocks(e->np);
-    if (!e->adj_phi || e->adj_cap < nb * ncol) {
+    const int npart = mfe::adjoint_blocks(e->np) * ncol + nblocks256(e->np) * e->npt;
+    if (!e->adj_phi || e->adj_cap < npart || e->adj_out_cap < ncol + e->npt) {
       dalloc(e->phi_rec, (size_t)e->max_np);
       dalloc(e->adj_phi, (size_t)e->max_np);
       dalloc(e->adj_dq, (size_t)e->max_np);
-      dalloc(e->adj_part, (size_t)nb * ncol);
-      dalloc(e->adj_out, (size_t)ncol);
-      e->adj_cap = nb * ncol;
+      dalloc(e->adj_dro, 3 * (size_t)e->max_np);
+      dalloc(e->adj_part, (size_t)npart);
+      dalloc(e->adj_out, (size_t)(ncol + e->npt));
+      e->adj_cap = npart;
+      e->adj_out_cap = ncol + e->npt;
       touch(e);
     }
     sync_view(e);
@@ -1933,27 +1935,24 @@ int mfe_adjoint(mfe_engine *e, double *dE_dq, double *dE_dzat, double *dE_dsigat
     if (G.surf) mfe::launch_surf(G);
     mfe::launch_reduce(G, f, false, false);
     mfe::launch_finalize(G, 0, 0.0);
-    mfe::launch_adjoint(G, ncol, e->adj_out);
-    std::vector<double> out(ncol), dq(e->np), fo(3 * (size_t)e->np);
-    MFE_HIP_TRY(hipMemcpyAsync(out.data(), e->adj_out, ncol * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-    MFE_HIP_TRY(hipMemcpyAsync(dq.data(), e->adj_dq, e->np * sizeof(double), hipMemcpyDeviceToHost, e->stream));
-    MFE_HIP_TRY(hipMemcpyAsync(fo.data(), e->forceo, fo.size() * sizeof(double), hipMemcpyDeviceToHost, e->stream));
+    mfe::launch_adjoint(G, e->np, e->npt, ncol, e->adj_part, e->adj_out, e->adj_dro);
+    std::vector<double> out(ncol + e->npt);
+    MFE_HIP_TRY(hipMemcpyAsync(out.data(), e->adj_out, out.size() * sizeof(double),
+                               hipMemcpyDeviceToHost, e->stream));
     fetch_energy(e);
     int r = read_flags(e);
     if (r) return r;
-    if (dE_dq) std::copy(dq.begin(), dq.end(), dE_dq);
-    if (dE_dzat) {
-      for (int t = 0; t < e->npt; ++t) dE_dzat[t] = 0.0;
-      for (int i = 0; i < e->np; ++i) dE_dzat[e->h_type[i]] += dq[i];
-    }
+    if (dE_dq)
+      MFE_HIP_TRY(hipMemcpyAsync(dE_dq, e->adj_dq, e->np * sizeof(double),
+                                 hipMemcpyDeviceToHost, e->stream));
+    if (dE_dro)
+      MFE_HIP_TRY(hipMemcpyAsync(dE_dro, e->adj_dro, 3 * (size_t)e->np * sizeof(double),
+                                 hipMemcpyDeviceToHost, e->stream));
+    MFE_HIP_TRY(hipStreamSynchronize(e->stream));
+    if (dE_dzat) std::copy(out.begin() + ncol, out.end(), dE_dzat);
     if (dE_dsigat) for (int t = 0; t < e->npt; ++t) dE_dsigat[t] = out[1 + t];
     if (dE_depsat) for (int t = 0; t < e->npt; ++t) dE_depsat[t] = out[1 + e->npt + t];
-    if (dE_dknot) std::copy(out.begin() + 1 + 2 * e->npt, out.end(), dE_dknot);
-    if (dE_dro) {
-      // position adjoint: dE/dr = -force (UTotal's force before the unit scaling)
-      const double ffac = e->h_sys.ffac;
-      for (size_t k = 0; k < fo.size(); ++k) dE_dro[k] = -fo[k] / ffac;
-    }
+    if (dE_dknot) std::copy(out.begin() + 1 + 2 * e->npt, out.begin() + ncol, dE_dknot);
     // the model energy: exact pair sum + reciprocal (with self/surface) + bonds
     if (energy) *energy = out[0] + e->h_en[2] + e->h_en[3];
     return MFE_OK;

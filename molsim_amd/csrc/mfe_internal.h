@@ -624,8 +624,8 @@ struct mfe_engine {
   mfe::PairParams pp{};
   bool have_pp = false;
   double *phi_rec = nullptr, *adj_phi = nullptr, *adj_dq = nullptr;
-  double *adj_part = nullptr, *adj_out = nullptr;
-  int adj_cap = 0;
+  double *adj_part = nullptr, *adj_out = nullptr, *adj_dro = nullptr;
+  int adj_cap = 0, adj_out_cap = 0;
   // force matching: device-resident frames (positions, target forces), the
   // model forces' reciprocal field, residuals, residual spreading weights,
   // block partials and the accumulated loss and gradient
@@ -679,8 +679,11 @@ struct FinArgs {
 enum { GM_FORCE = 0, GM_POT = 1, GM_FIELD = 2, GM_POTONLY = 3, GM_FORCE_REC = 4 };
 void launch_spme(const Group &g, bool energy, int first_stage, int last_stage,
                  int gather_mode = GM_FORCE, const FinArgs *fin = nullptr);
-// adjoint passes: real-space pair sums, per-particle dE/dq, column sums
-void launch_adjoint(const Group &g, int ncol, double *out);
+// adjoint passes of one engine: real-space pair sums, per-particle dE/dq and
+// dE/dr (dro), column sums; part: adjoint_blocks(np) * ncol partials, then
+// npt per 256 particles; out: the ncol sums, then dE/dzat[npt]
+void launch_adjoint(const Group &g, int np, int npt, int ncol, double *part, double *out,
+                    double *dro);
 int adjoint_blocks(int np);  // rows of its partials
 void launch_std_ewald(const Group &g);
 void launch_bonds(const Group &g);
