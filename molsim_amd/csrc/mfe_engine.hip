@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "mfe_internal.h"
+#include "mfe_transfer.h"
 
 using mfe::HipError;
 
@@ -169,6 +170,9 @@ void free_all(mfe_engine *e) {
   dfree(e->adj_part); dfree(e->adj_out); dfree(e->adj_dro);
   dfree(e->fm_ro); dfree(e->fm_tgt); dfree(e->fm_fld); dfree(e->fm_res); dfree(e->fm_res_s);
   dfree(e->fm_vec); dfree(e->fm_part); dfree(e->fm_acc); dfree(e->fm_qr);
+  if (e->ring) e->ring->release();
+  delete e->ring;
+  e->ring = nullptr;
   if (e->h_en) (void)hipHostFree(e->h_en);
   if (e->h_flags) (void)hipHostFree(e->h_flags);
   e->h_en = nullptr;
@@ -759,6 +763,7 @@ int mfe_create(const mfe_config *cfg, mfe_engine **out) {
     MFE_HIP_TRY(hipSetDevice(e->device));
     MFE_HIP_TRY(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
     MFE_HIP_TRY(mfe::side_create(e->side));
+    e->ring = new mfe::DownloadRing();
     hipDeviceProp_t prop;
     MFE_HIP_TRY(hipGetDeviceProperties(&prop, e->device));
     e->ncu = prop.multiProcessorCount;
@@ -1321,11 +1326,8 @@ int mfe_upload_positions(mfe_engine *e, const double *ro) {
   e->forces_current = false;
   e->mc_cached = false;
   if (!e->have_particles || !e->have_box) return fail(e, MFE_E_STATE, "box and particles first");
-  for (int i = 0; i < 3 * e->np; ++i) {
-    const int m = i % 3;
-    if (!(std::fabs(ro[i]) <= e->box.L2[m]))
-      return fail(e, MFE_E_BAD_PARAM, "particle outside the box [-L/2, L/2]");
-  }
+  if (!mfe::in_box(ro, (size_t)e->np, e->box.L2))
+    return fail(e, MFE_E_BAD_PARAM, "particle outside the box [-L/2, L/2]");
   return guarded(e, [&]() -> int {
     MFE_HIP_TRY(hipSetDevice(e->device));
     if (e->list_valid && e->have_positions && e->have_neighbor) {
@@ -1361,10 +1363,11 @@ int mfe_download_state(mfe_engine *e, double *ro, double *rod, double *rodd) {
   if (!e) return MFE_E_BAD_PARAM;
   return guarded(e, [&]() -> int {
     const size_t n = 3 * (size_t)e->np * sizeof(double);
-    if (ro) MFE_HIP_TRY(hipMemcpyAsync(ro, e->ro, n, hipMemcpyDeviceToHost, e->stream));
-    if (rod) MFE_HIP_TRY(hipMemcpyAsync(rod, e->rod, n, hipMemcpyDeviceToHost, e->stream));
-    if (rodd) MFE_HIP_TRY(hipMemcpyAsync(rodd, e->rodd, n, hipMemcpyDeviceToHost, e->stream));
-    MFE_HIP_TRY(hipStreamSynchronize(e->stream));
+    std::vector<mfe::DownloadPart> parts;
+    if (ro) parts.push_back({ro, e->ro, n});
+    if (rod) parts.push_back({rod, e->rod, n});
+    if (rodd) parts.push_back({rodd, e->rodd, n});
+    mfe::download(*e->ring, e->device, parts, e->stream);
     return MFE_OK;
   });
 }
@@ -1373,9 +1376,8 @@ int mfe_download_forces(mfe_engine *e, double *forceo) {
   if (!e || !forceo) return MFE_E_BAD_PARAM;
   if (!e->have_particles) return fail(e, MFE_E_STATE, "mfe_set_particles first");
   return guarded(e, [&]() -> int {
-    MFE_HIP_TRY(hipMemcpyAsync(forceo, e->forceo, 3 * (size_t)e->np * sizeof(double),
-                               hipMemcpyDeviceToHost, e->stream));
-    MFE_HIP_TRY(hipStreamSynchronize(e->stream));
+    mfe::download(*e->ring, e->device, {{forceo, e->forceo, 3 * (size_t)e->np * sizeof(double)}},
+                  e->stream);
     return MFE_OK;
   });
 }
@@ -1410,8 +1412,8 @@ int mfe_compute(mfe_engine *e, uint32_t flags, double *forceo, mfe_energy *energ
     sync_view(e);
     mfe_launch_utotal(e->grp, f, 0, 0.0, false, false);
     if (forceo)
-      MFE_HIP_TRY(hipMemcpyAsync(forceo, e->forceo, 3 * (size_t)e->np * sizeof(double),
-                                 hipMemcpyDeviceToHost, e->stream));
+      mfe::download(*e->ring, e->device,
+                    {{forceo, e->forceo, 3 * (size_t)e->np * sizeof(double)}}, e->stream, false);
     fetch_energy(e);
     int r = read_flags(e);
     if (r) return r;
@@ -1431,12 +1433,16 @@ int mc_prepare(mfe_engine *e, int natm, const int32_t *ianatm, const double *rtm
   if (rc) return rc;
   if (natm > e->np) return fail(e, MFE_E_BAD_PARAM, "natm > np");
   ia.assign(natm, 0);
-  std::vector<char> seen(e->np, 0);
+  // a few particles compared with each other: clearing a mark per particle
+  // of the system cost a one-particle move of 50000 about 2 us
+  const bool few = natm <= 64;
+  std::vector<char> seen(few ? 0 : e->np, 0);
   for (int a = 0; a < natm; ++a) {
     const int i = ianatm[a] - 1;
     if (i < 0 || i >= e->np) return fail(e, MFE_E_BAD_PARAM, "ianatm out of range");
-    if (seen[i]) return fail(e, MFE_E_BAD_PARAM, "ianatm repeats a particle");
-    seen[i] = 1;
+    if (few ? std::find(ia.begin(), ia.begin() + a, i) != ia.begin() + a : seen[i] != 0)
+      return fail(e, MFE_E_BAD_PARAM, "ianatm repeats a particle");
+    if (!few) seen[i] = 1;
     ia[a] = i;
     for (int m = 0; m < 3; ++m)
       if (!std::isfinite(rtm[3 * a + m])) return fail(e, MFE_E_BAD_PARAM, "rtm not finite");
@@ -2033,13 +2039,12 @@ int mfe_model_forces(mfe_engine *e, double *force) {
     fm_buffers(e);
     sync_view(e);
     fm_forward(e);
-    std::vector<double> fo(3 * (size_t)e->np);
-    MFE_HIP_TRY(hipMemcpyAsync(fo.data(), e->forceo, fo.size() * sizeof(double),
-                               hipMemcpyDeviceToHost, e->stream));
     int r = read_flags(e);
     if (r) return r;
+    const size_t n3 = 3 * (size_t)e->np;
+    mfe::download(*e->ring, e->device, {{force, e->forceo, n3 * sizeof(double)}}, e->stream);
     const double inv = 1.0 / e->h_sys.ffac;
-    for (size_t k = 0; k < fo.size(); ++k) force[k] = fo[k] * inv;
+    for (size_t k = 0; k < n3; ++k) force[k] *= inv;
     return MFE_OK;
   });
 }
@@ -2049,12 +2054,10 @@ int mfe_fm_set_frames(mfe_engine *e, int32_t nframes, const double *ro, const do
   e->forces_current = false;
   if (!e->have_particles || !e->have_box) return fail(e, MFE_E_STATE, "box and particles first");
   const size_t n3 = 3 * (size_t)e->np;
-  for (size_t k = 0; k < n3 * nframes; ++k) {
-    const int m = (int)(k % 3);
-    if (!(std::fabs(ro[k]) <= e->box.L2[m]))
-      return fail(e, MFE_E_BAD_PARAM, "frame position outside the box [-L/2, L/2]");
+  if (!mfe::in_box(ro, (size_t)e->np * nframes, e->box.L2))
+    return fail(e, MFE_E_BAD_PARAM, "frame position outside the box [-L/2, L/2]");
+  for (size_t k = 0; k < n3 * nframes; ++k)
     if (!std::isfinite(f_target[k])) return fail(e, MFE_E_BAD_PARAM, "target not finite");
-  }
   return guarded(e, [&]() -> int {
     MFE_HIP_TRY(hipSetDevice(e->device));
     if (nframes != e->fm_nframes || e->fm_frame_np != e->np) {

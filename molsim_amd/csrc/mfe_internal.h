@@ -486,6 +486,10 @@ struct Group {
 }  // namespace mfe
 
 // ------------------------------------------------------------------ engine
+namespace mfe {
+struct DownloadRing;
+}
+
 struct mfe_engine {
   int device = 0;
   int prec = MFE_PREC_MIXED;
@@ -577,6 +581,8 @@ struct mfe_engine {
   // of more than kMcArg particles, so its copies run on the stream
   char *h_mc = nullptr;
   size_t h_mc_bytes = 0;
+  // pinned slots of large downloads (made on the first one)
+  mfe::DownloadRing *ring = nullptr;
   bool mc_cached = false;
   // the move of the last mfe_mc_delta_rec (0-based indices, positions):
   // mfe_mc_accept of the same move keeps its trial mesh and E_rec
