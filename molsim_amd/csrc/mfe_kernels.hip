@@ -508,7 +508,13 @@ __device__ __forceinline__ void rebuild_phases(const SysDev &V, unsigned *bar, i
 __global__ void __launch_bounds__(1024) k_rebuild(const SysDev *__restrict__ sys,
                                                   const int *__restrict__ gate, unsigned *bar,
                                                   int spin) {
-  if (gate[1] == 0 || (gate[0] & ERR_SYNC)) return;
+  // one thread's reading decides for the block (see k_finalize_rebuild)
+  __shared__ int go_s;
+  if (threadIdx.x == 0)
+    go_s = gate[1] != 0 &&
+           !(__hip_atomic_load(&gate[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ERR_SYNC);
+  __syncthreads();
+  if (!go_s) return;
   rebuild_phases(sys[0], bar, spin);
 }
 
@@ -2985,6 +2991,12 @@ __global__ void __launch_bounds__(kReduceThreads) k_finalize_rebuild(
       ph_finalize(V, i, mode, dt, es, split != 0);
   }
   __shared__ double mx_s[2][kReduceThreads / 64];
+  __shared__ int void_s;
+  // one thread's reading decides for the block: a block of this launch may
+  // raise the error meanwhile, and waves that read different values would
+  // part, some into the rebuild without the others
+  if (threadIdx.x == 0)
+    void_s = __hip_atomic_load(&V.flags[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ERR_SYNC;
   for (int w = 32; w > 0; w >>= 1) {
     m1 = fmax(m1, __shfl_xor(m1, w, 64));
     m2 = fmax(m2, __shfl_xor(m2, w, 64));
@@ -3007,8 +3019,7 @@ __global__ void __launch_bounds__(kReduceThreads) k_finalize_rebuild(
   }
   if (!fired) return;
   // after a failed rebuild earlier in the call the list stays void
-  if (__hip_atomic_load(&V.flags[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ERR_SYNC)
-    return;
+  if (void_s) return;
   rebuild_phases(V, bar, spin);
 }
 
