@@ -340,14 +340,18 @@ __global__ void __launch_bounds__(1024) k_fm_spread(const SysDev *__restrict__ s
     const int ly = ((code >> 10) & 1023) - o1;
     const int lz = ((code >> 20) & 1023) - o2;
     Acc *zp = tile + (lz - iz) * plane;
+    constexpr double kScale = kSplineScale<ORDER, 1>;
+    const R vx = SpreadAcc<R>::pre(v.x, kScale), vy = SpreadAcc<R>::pre(v.y, kScale),
+            vz = SpreadAcc<R>::pre(v.z, kScale);
 #pragma unroll
     for (int jy = 0; jy < ORDER; ++jy) {
       // point (jx, jy, iz): dx[jx] * A + wx[jx] * Bc
-      const R A = v.x * wy[jy] * wzi;
-      const R Bc = v.y * dy[jy] * wzi + v.z * wy[jy] * dzi;
+      const R A = vx * wy[jy] * wzi;
+      const R Bc = vy * dy[jy] * wzi + vz * wy[jy] * dzi;
       Acc *row = zp + (ly - jy) * E0 + lx;
 #pragma unroll
-      for (int j = 0; j < ORDER; ++j) SpreadAcc<R>::add(&row[-j], dx[j] * A + wx[j] * Bc);
+      for (int j = 0; j < ORDER; ++j)
+        SpreadAcc<R>::add(&row[-j], dx[j] * A + wx[j] * Bc, kScale);
     }
   }
   __syncthreads();

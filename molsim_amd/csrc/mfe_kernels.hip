@@ -1381,14 +1381,15 @@ __global__ void __launch_bounds__(kSpreadThreads) k_spread(const SysDev *__restr
     const int lx = (code & 1023) - o0;
     const int ly = ((code >> 10) & 1023) - o1;
     const int lz = ((code >> 20) & 1023) - o2;
-    const R qz = f.q * wzi;
+    constexpr double kScale = kSplineScale<ORDER, 0>;
+    const R qz = SpreadAcc<R>::pre(f.q, kScale) * wzi;
     Acc *zp = tile + (lz - iz) * plane;
 #pragma unroll
     for (int jy = 0; jy < ORDER; ++jy) {
       const R qyz = qz * wy[jy];
       Acc *row = zp + (ly - jy) * E0 + lx;
 #pragma unroll
-      for (int j = 0; j < ORDER; ++j) SpreadAcc<R>::add(&row[-j], qyz * wx[j]);
+      for (int j = 0; j < ORDER; ++j) SpreadAcc<R>::add(&row[-j], qyz * wx[j], kScale);
     }
     f = fn;
     code = cn;
@@ -1469,10 +1470,10 @@ __device__ __forceinline__ void gather_body(const SysDev *__restrict__ sys, FinA
   const int o0 = bx * g.B[0], o1 = by * g.B[1], o2 = bz * g.B[2];
   const int E0 = g.B[0] + ORDER - 1, E1 = g.B[1] + ORDER - 1, E2 = g.B[2] + ORDER - 1;
   const int nstage = E0 * E1 * E2;
-  // GL lanes share a particle, lane l summing stencil planes l, l + GL,
-  // ...: two lanes on the FP32 path (no idle lanes at even orders), eight
-  // on the FP64 path (one plane each)
-  constexpr int GL = sizeof(R) == 4 ? 2 : 8;
+  // two lanes share a particle, lane l summing stencil planes l, l + 2, ...
+  // (none idle at even orders), each with the particle's splines: FP64, 200k
+  // ions, order 6, 28.3 us with two lanes, 30.1 with four, 34.9 with eight
+  constexpr int GL = 2;
   constexpr int kGStep = kGatherLanes / GL;
   constexpr int kPlanes = (ORDER + GL - 1) / GL;
   const int first = bstart[bxi], n = bstart[bxi + 1] - first;
@@ -1553,12 +1554,12 @@ __device__ __forceinline__ void gather_body(const SysDev *__restrict__ sys, FinA
         const int iz = l + GL * kz;
         if (iz >= ORDER) break;
         // weights of plane iz, selected among this step's GL planes
-        R vz = v[2][GL * kz], dz = d[2][GL * kz];
+        R vz = v[2][0], dz = d[2][0];
 #pragma unroll
-        for (int k = 1; k < GL; ++k)
-          if (GL * kz + k < ORDER && l == k) {
-            vz = v[2][GL * kz + k];
-            dz = d[2][GL * kz + k];
+        for (int k = 1; k < ORDER; ++k)
+          if (iz == k) {
+            vz = v[2][k];
+            dz = d[2][k];
           }
         const R *plane = tile + (size_t)(lz - iz) * E1 * E0;
 #pragma unroll
@@ -1579,10 +1580,10 @@ __device__ __forceinline__ void gather_body(const SysDev *__restrict__ sys, FinA
           if (MODE == GM_POT || MODE == GM_POTONLY) pacc += (double)sx * (double)(v[1][iy] * vz);
         }
       }
-      ex = acc.get(0);
-      ey = acc.get(1);
-      ez = acc.get(2);
-      ep = pacc;
+      ex = acc.get(0) * kSplineScale<ORDER, 1>;
+      ey = acc.get(1) * kSplineScale<ORDER, 1>;
+      ez = acc.get(2) * kSplineScale<ORDER, 1>;
+      ep = pacc * kSplineScale<ORDER, 0>;
     }
     // the GL lanes of a particle are all in or all out of the loop
     if constexpr (GL == 2) {
@@ -1635,8 +1636,10 @@ __device__ __forceinline__ void gather_body(const SysDev *__restrict__ sys, FinA
   }
 }
 
+// two blocks per CU on the FP64 path up to the order whose tile and
+// registers allow it
 template <typename R, int ORDER, int MODE, bool FIN>
-__global__ void __launch_bounds__(kGatherLanes) k_gather(const SysDev *__restrict__ sys,
+__global__ void __launch_bounds__(kGatherLanes, sizeof(R) == 8 && ORDER <= 6 ? 4 : 1) k_gather(const SysDev *__restrict__ sys,
                                                          FinArgs fa) {
   gather_body<R, ORDER, MODE, FIN>(sys, fa, (int)blockIdx.x);
 }
@@ -1787,7 +1790,8 @@ __device__ __forceinline__ void mc_rec_body(const SysDev &V, const McMove &mv, i
           r[m] = (row & 1) ? mc_rtm(mv, 3 * a + m) : (apply ? old[3 * a + m] : V.ro[3 * i + m]);
         if (k < hx) {
           const double2 c = factor(r[0], g.dkdr[0], s0, root, k);
-          const double q = (double)(R)V.q[i];
+          // the splines' divisors with the charge
+          const double q = (double)(R)V.q[i] * kSplineScale<ORDER, 0>;
           fx[row * hx + k] = make_double2(c.x * q, c.y * q);
         } else {
           const unsigned rr = r0 + (unsigned)(k - hx), kz = rr / (unsigned)s1;
@@ -3379,7 +3383,7 @@ MFE_STAGE void p_spread(const SysDev &V, char *smem, int lds) {
 #pragma unroll
           for (int ix = 0; ix < ORDER; ++ix) {
             const int x = mm[0] - ix < 0 ? mm[0] - ix + s1 : mm[0] - ix;
-            SpreadAcc<float>::add(&row[x], qyz * wx[ix]);
+            SpreadAcc<float>::add(&row[x], qyz * wx[ix], kSplineScale<ORDER, 0>);
           }
         }
       }
@@ -3481,8 +3485,10 @@ MFE_STAGE void p_gather(const SysDev &V, char *smem, int lds) {
       }
     }
     const double qd = (double)(float)V.q[i];
-    const double fld[3] = {-ac.get(0) * g.dkdr[0] * V.efp, -ac.get(1) * g.dkdr[1] * V.efp,
-                           -ac.get(2) * g.dkdr[2] * V.efp};
+    constexpr double kScale = kSplineScale<ORDER, 1>;
+    const double fld[3] = {-(ac.get(0) * kScale) * g.dkdr[0] * V.efp,
+                           -(ac.get(1) * kScale) * g.dkdr[1] * V.efp,
+                           -(ac.get(2) * kScale) * g.dkdr[2] * V.efp};
     double ft[3];
 #pragma unroll
     for (int m = 0; m < 3; ++m) ft[m] = V.force[3 * i + m] + qd * fld[m];
