@@ -673,21 +673,30 @@ bool mfe_launch_utotal(const mfe::Group &g, unsigned flags, int mode, double dt,
     mfe::launch_pair_gather(g, energy, skin);
     return finalize_launch(g, flags, skin, bd, mode, dt, true, rebuild);
   }
-  const bool fork = g.ewald == MFE_EWALD_SPME && g.side.stream;
+  // Bonds and the surface sums follow the pair launch on its stream: they
+  // share no data with the reciprocal stages either, and add to the pair
+  // forces before the gather does (a chain system of 6000 particles: 95 us a
+  // step with the 7 us of the bonds after the gather, 86 so).  The two
+  // branches of the standard Ewald sum are too short for a fork (1000 ions:
+  // 42 us a step, 47 with the structure factors beside the pair launch).
+  const bool spme = g.ewald == MFE_EWALD_SPME;
+  const bool fork = spme && g.side.stream;
+  mfe::Group gp = g;
   int first = SP_BIN;
   if (fork) {
     if (!skin) mfe::launch_sort_pos(g);
     MFE_HIP_TRY(hipEventRecord(g.side.fork, g.stream));
     MFE_HIP_TRY(hipStreamWaitEvent(g.side.stream, g.side.fork, 0));
-    mfe::Group gp = g;
     gp.stream = g.side.stream;
-    mfe::launch_pair(gp, energy, false, skin);
+  }
+  mfe::launch_pair(gp, energy, !fork && !skin, skin);
+  if (g.chains) mfe::launch_bonds(gp);
+  if (g.surf) mfe::launch_surf(gp);
+  if (fork) {
     MFE_HIP_TRY(hipEventRecord(g.side.join, g.side.stream));
     mfe::launch_spme(g, energy, SP_BIN, SP_IFFTX);
     MFE_HIP_TRY(hipStreamWaitEvent(g.stream, g.side.join, 0));
     first = SP_GATHER;
-  } else {
-    mfe::launch_pair(g, energy, !skin, skin);
   }
   // with SPME as the last force stage and no VelVer kick, the gather
   // launch also finalizes each particle (forceo only) and reduces the
@@ -700,10 +709,8 @@ bool mfe_launch_utotal(const mfe::Group &g, unsigned flags, int mode, double dt,
     mfe::launch_spme(g, energy, first, SP_GATHER, mfe::GM_FORCE, &fa);
     return false;
   }
-  if (g.ewald == MFE_EWALD_SPME) mfe::launch_spme(g, energy, first, SP_GATHER);
+  if (spme) mfe::launch_spme(g, energy, first, SP_GATHER);
   else if (g.ewald == MFE_EWALD_STD) mfe::launch_std_ewald(g);
-  if (g.chains) mfe::launch_bonds(g);
-  if (g.surf) mfe::launch_surf(g);
   if (g.surf) {
     // the surface field of the reduction enters the forces
     mfe::launch_reduce(g, flags, skin, bd);
