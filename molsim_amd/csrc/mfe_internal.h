@@ -480,6 +480,7 @@ struct Group {
   // the pair forces and the gather in one launch (launch_pair_gather):
   // mixed SPME without bonds, surface term, spline knots or FP64
   // separations, coefficients in LDS, both LDS needs within the block limit
+  bool fuse_sk = false;
   bool fuse_pg = false;
 };
 
@@ -691,7 +692,11 @@ void launch_spme(const Group &g, bool energy, int first_stage, int last_stage,
 void launch_adjoint(const Group &g, int np, int npt, int ncol, double *part, double *out,
                     double *dro);
 int adjoint_blocks(int np);  // rows of its partials
-void launch_std_ewald(const Group &g);
+// the standard Ewald sum: structure factors, then the forces from them
+void launch_std_factors(const Group &g);
+void launch_std_forces(const Group &g);
+// the pair forces and the structure factors in one launch (Group::fuse_sk)
+void launch_pair_sk(const Group &g, bool energy, bool skin);
 void launch_bonds(const Group &g);
 void launch_surf(const Group &g);
 void launch_reduce(const Group &g, unsigned flags, bool skin, bool bd);

@@ -2059,17 +2059,14 @@ __device__ __forceinline__ double2 phase(double x) {
 // axis: 9.4 us (11.5 with 256 threads, four sincos, eight block sums); bound
 // by the FP64 sincos chain of each thread.
 constexpr int kSkThreads = 512;
-__global__ void __launch_bounds__(kSkThreads) k_ewald_sk(const SysDev *__restrict__ sys,
-                                                         int energy) {
-  const SysDev &V = sys[blockIdx.z];
-  if ((int)blockIdx.x >= V.nkvec) return;
+__device__ __forceinline__ void ewald_sk_body(const SysDev &V, int energy, int kn) {
+  if (kn >= V.nkvec) return;
   const double *__restrict__ ro = V.ro;
   const double *__restrict__ q = V.q;
   const int np = V.np;
   const double *__restrict__ kv = V.k_vec;
   const double alpha2 = V.alpha * V.alpha;
   __shared__ double red[8][kSkThreads / 64];
-  const int kn = blockIdx.x;
   const double kx = kv[4 * kn], ky = kv[4 * kn + 1], kz = kv[4 * kn + 2];
   double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   for (int i = threadIdx.x; i < np; i += kSkThreads) {
@@ -2107,6 +2104,23 @@ __global__ void __launch_bounds__(kSkThreads) k_ewald_sk(const SysDev *__restric
       part[V.nkvec + kn] = -(1.0 - k2 / (2.0 * alpha2)) * term;
     }
   }
+}
+
+__global__ void __launch_bounds__(kSkThreads) k_ewald_sk(const SysDev *__restrict__ sys,
+                                                         int energy) {
+  ewald_sk_body(sys[blockIdx.z], energy, (int)blockIdx.x);
+}
+
+// The mixed path's pair forces and the structure factors in one launch, the
+// pair and skin blocks [0, npb) first: both leave most of the chip idle and
+// share no data (1000 ions, 8 wave numbers per axis: 12 + 9 us in two).
+static_assert(kSkThreads == kPairBlock, "the fused launch runs both bodies in one block size");
+template <int NT, bool POS64>
+__global__ void __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(4)))
+k_pair_sk(const SysDev *__restrict__ sys, int energy, int pgrid, int skin, int npb) {
+  const int b = (int)blockIdx.x;
+  if (b < npb) pair_f_body<NT, true, false, POS64>(sys, energy, pgrid, skin, b);
+  else ewald_sk_body(sys[blockIdx.z], energy, b - npb);
 }
 
 // One wavefront per particle, its lanes over the k-vectors: a thread per
@@ -3885,8 +3899,29 @@ void launch_spme(const Group &g, bool energy, int first, int last, int gmode,
   else spme_stages<double>(g, energy, first, last, gmode, fin);
 }
 
-void launch_std_ewald(const Group &g) {
+void launch_pair_sk(const Group &g, bool energy, bool skin) {
+  const int pgrid = std::max(g.pair_blocks, 1);
+  const int npb = pgrid + (skin ? (g.np_blocks + 1) / 2 : 0);
+  const int e1 = energy ? 1 : 0, s1 = skin ? 1 : 0;
+  const int nt = g.pair_npt <= 3 ? 3 : (g.pair_npt <= 4 ? 4 : 8);
+#define MFE_PSK(NT, P64)                                                                   \
+  hipLaunchKernelGGL((k_pair_sk<NT, P64>), grid(npb + g.kvec, g), dim3(kPairBlock),        \
+                     g.lds_pair, g.stream, g.d, e1, pgrid, s1, npb)
+#define MFE_PSK_NT(P64)          \
+  if (nt == 3) MFE_PSK(3, P64);  \
+  else if (nt == 4) MFE_PSK(4, P64); \
+  else MFE_PSK(8, P64);
+  if (g.pair_any64) { MFE_PSK_NT(true) }
+  else { MFE_PSK_NT(false) }
+#undef MFE_PSK_NT
+#undef MFE_PSK
+}
+
+void launch_std_factors(const Group &g) {
   hipLaunchKernelGGL(k_ewald_sk, grid(g.kvec, g), dim3(kSkThreads), 0, g.stream, g.d, 1);
+}
+
+void launch_std_forces(const Group &g) {
   const dim3 gr = grid((g.np_blocks * kBlock + kEwParticles - 1) / kEwParticles, g);
   const size_t lds = (size_t)kEwParticles * 3 * (g.ncut + 1) * sizeof(double2);
   if (lds <= 64 * 1024)
