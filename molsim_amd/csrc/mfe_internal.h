@@ -480,8 +480,10 @@ struct Group {
   // the pair forces and the gather in one launch (launch_pair_gather):
   // mixed SPME without bonds, surface term, spline knots or FP64
   // separations, coefficients in LDS, both LDS needs within the block limit
-  bool fuse_sk = false;
   bool fuse_pg = false;
+  // the pair forces and the standard Ewald sum's structure factors in one
+  // launch (launch_pair_sk)
+  bool fuse_sk = false;
 };
 
 }  // namespace mfe
