@@ -249,22 +249,33 @@ RowPlan row_plan(int prec, const int s[3], const int B[3], int order) {
   return p;
 }
 
+// The forward pass on the mixed path takes kRowThreads threads whatever the
+// butterflies need, for its tile loads (four points of a thread in flight),
+// where the launch has few blocks: 128^3 16.4 -> 13.1 us, 64^3 8.9 -> 7.0,
+// 70^3 9.8 -> 8.2, 240^3 no change (512 threads: 17.0, 6.6, 7.7 and 94.9
+// against 82.7).  Launches that fill the chip several times over lose by it
+// (a batch of 96 replicas of 36^3 4% of its step); FP64 128^3 19.8 either way.
+constexpr long long kFewRowBlocks = 2048;
 void fft_x_forward(const Group &g) {
-#define MFE_X(T, ROW, LDS_ROWS)                                                               \
+#define MFE_X(T, ROW, LDS_ROWS, THR)                                                          \
   do {                                                                                        \
     if (g.cx_blocks)                                                                          \
-      hipLaunchKernelGGL(ROW<T>, dim3(g.cx_blocks, 1, g.R), dim3(g.cx_thr), g.lds_cx,         \
-                         g.stream, g.d);                                                      \
+      hipLaunchKernelGGL(ROW<T>, dim3(g.cx_blocks, 1, g.R), dim3(THR), g.lds_cx, g.stream,    \
+                         g.d);                                                                \
     if (g.fx_blocks)                                                                          \
       hipLaunchKernelGGL(LDS_ROWS<T>, dim3(g.fx_blocks, 1, g.R), dim3(256), g.lds_fx,         \
                          g.stream, g.d);                                                      \
   } while (0)
-  if (g.prec == MFE_PREC_MIXED) MFE_X(float, k_row_fwd, k_fft_x_fwd);
-  else MFE_X(double, k_row_fwd, k_fft_x_fwd);
+  if (g.prec == MFE_PREC_MIXED) {
+    const bool few = (long long)g.cx_blocks * g.R <= kFewRowBlocks;
+    MFE_X(float, k_row_fwd, k_fft_x_fwd, few ? kRowThreads : g.cx_thr);
+  } else {
+    MFE_X(double, k_row_fwd, k_fft_x_fwd, g.cx_thr);
+  }
 }
 void fft_x_inverse(const Group &g) {
-  if (g.prec == MFE_PREC_MIXED) MFE_X(float, k_row_inv, k_fft_x_inv);
-  else MFE_X(double, k_row_inv, k_fft_x_inv);
+  if (g.prec == MFE_PREC_MIXED) MFE_X(float, k_row_inv, k_fft_x_inv, g.cx_thr);
+  else MFE_X(double, k_row_inv, k_fft_x_inv, g.cx_thr);
 #undef MFE_X
 }
 }  // namespace mfe
