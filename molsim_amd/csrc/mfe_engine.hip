@@ -137,6 +137,21 @@ int smallest_divisor_at_least(int s, int lo) {
   return s;
 }
 
+// Edge of the spreading and gather bricks along an axis of s points: 16
+// where it divides s, else the largest divisor of s from 15 down to 8
+// (large) or the smallest from 8 up, else the smallest that holds a
+// spline's reach.  Large bricks have fewer halo points and fill the blocks
+// better: 120^3, 100k ions, order 4, edges 8 / 15: spreading 17.2 / 7.8 us,
+// gather 27 / 12, binning 15 / 9.5.
+int brick_edge(int s, int order, bool large) {
+  if (s < 8) return s;
+  for (int k = 0; k < 9; ++k) {
+    const int d = large || k == 0 ? 16 - k : 7 + k;
+    if (s % d == 0) return d;
+  }
+  return smallest_divisor_at_least(s, order - 1);
+}
+
 void free_all(mfe_engine *e) {
   e->md_graph.clear();
   dfree(e->ro); dfree(e->rod); dfree(e->rodd); dfree(e->force); dfree(e->forceo);
@@ -1132,22 +1147,20 @@ int mfe_set_ewald(mfe_engine *e, int32_t kind, double alpha, int32_t order,
         e->plan[m] = make_plan(e->s[m]);
         if (!plan_ok(e->plan[m])) return fail(e, MFE_E_BAD_PARAM, "mesh has a prime factor > 32");
       }
-      // bricks of the spreading and gather blocks: B divides s, the largest
-      // divisor from 16 down to 8 (fewer halo points per brick and fewer,
-      // fuller blocks: 120^3, 100k ions, order 4, B = 8 / 15: spreading 17.2
-      // / 7.8 us, gather 27 / 12, binning 15 / 9.5; 70^3, 20005 ions, B = 10
-      // / 14: no difference), else the smallest divisor above
-      size_t ext = 1, planes = 1;
-      for (int m = 0; m < 3; ++m) {
-        int b = 0;
-        for (int d = 16; d >= 8 && !b; --d)
-          if (e->s[m] % d == 0) b = d;
-        if (!b) b = smallest_divisor_at_least(e->s[m], 17);
-        if (b > 16) b = smallest_divisor_at_least(e->s[m], order - 1);
-        e->B[m] = b;
-        e->nb[m] = e->s[m] / b;
-        ext *= (size_t)(b + order - 1);
-        if (m == 1) planes = ext;
+      // bricks of the spreading and gather blocks: the largest edges of
+      // brick_edge whose tile a CU's LDS holds (62 x 62 x 24 at order 6:
+      // edges 31, 31 and 8; with 12 the tile is 172 KB)
+      bool large = true;
+      size_t ext, planes;
+      for (;; large = false) {
+        ext = 1;
+        for (int m = 0; m < 3; ++m) {
+          e->B[m] = brick_edge(e->s[m], order, large);
+          e->nb[m] = e->s[m] / e->B[m];
+          ext *= (size_t)(e->B[m] + order - 1);
+        }
+        planes = ext / (size_t)(e->B[2] + order - 1);
+        if (!large || ext * 8 <= mfe::kCuLds) break;
       }
       e->nbricks = e->nb[0] * e->nb[1] * e->nb[2];
       const size_t rsz = e->prec == MFE_PREC_MIXED ? 4 : 8;
@@ -1155,11 +1168,11 @@ int mfe_set_ewald(mfe_engine *e, int32_t kind, double alpha, int32_t order,
       // z planes of an odd number of values where the CU's LDS holds them
       // (SpmeGeom::plane)
       const size_t E2 = (size_t)(e->B[2] + order - 1);
-      e->spread_plane = (int)((planes | 1) * E2 * 8 <= 160 * 1024 ? planes | 1 : planes);
+      e->spread_plane = (int)((planes | 1) * E2 * 8 <= mfe::kCuLds ? planes | 1 : planes);
       e->spread_lds = (int)(e->spread_plane * E2 * 8);
       const size_t gext = ext * rsz;
       const int lds_need = (int)std::max<size_t>((size_t)e->spread_lds, gext);
-      if ((size_t)lds_need > 160 * 1024)
+      if ((size_t)lds_need > mfe::kCuLds)
         return fail(e, MFE_E_BAD_PARAM, "mesh brick too large for LDS (mesh 2q, q prime > 16?)");
       const size_t M = (size_t)e->s[0] * e->s[1] * e->s[2];
       const size_t Mc = (size_t)e->hx * e->s[1] * e->s[2];

@@ -163,6 +163,8 @@ constexpr int kBarGen = kBarTop + kBarStride;
 constexpr int kBarWords = kBarGen + kBarStride;
 // ranges of the rebuild's scan of the cell counts
 constexpr int kScanBlocks = 256;
+// LDS of a CU, the most that a block can have
+constexpr size_t kCuLds = 160 * 1024;
 // threads per block of the pair kernel and its dynamic LDS budget
 constexpr int kPairBlock = 512;
 // blocks of the persistent pair kernel (two per CU)
