@@ -140,9 +140,7 @@ int smallest_divisor_at_least(int s, int lo) {
 // Edge of the spreading and gather bricks along an axis of s points: 16
 // where it divides s, else the largest divisor of s from 15 down to 8
 // (large) or the smallest from 8 up, else the smallest that holds a
-// spline's reach.  Large bricks have fewer halo points and fill the blocks
-// better: 120^3, 100k ions, order 4, edges 8 / 15: spreading 17.2 / 7.8 us,
-// gather 27 / 12, binning 15 / 9.5.
+// spline's reach.
 int brick_edge(int s, int order, bool large) {
   if (s < 8) return s;
   for (int k = 0; k < 9; ++k) {
@@ -150,6 +148,27 @@ int brick_edge(int s, int order, bool large) {
     if (s % d == 0) return d;
   }
   return smallest_divisor_at_least(s, order - 1);
+}
+
+// Whether the bricks take the large edges.  They have fewer halo points and
+// fill the blocks better where the bricks outnumber the CUs (120^3, 100k
+// ions, order 4, edges 8 / 15: spreading 17.2 / 7.8 us, gather 27 / 12,
+// binning 15 / 9.5), and in a batch (96 replicas of 500 to 4000 ions, order
+// 4: 281 / 250 us a step; order 6: 330 / 289).  A single system of fewer
+// bricks runs on that many CUs: large ones cost it little while they hold
+// few particles (16000 ions on 36^3, order 4: 61.0 / 63.6 us a step; FP64
+// 80.6 / 88.3) and much when crowded (20000 on 24^3, order 6: 74 / 132;
+// FP64 114 / 227, where the block holds the LDS adds longer).  The line, in
+// stencil points of a brick's particles, lies where single systems lose
+// more than batches gain: FP64 4000 ions on 24^3, order 6 (1.08e5 a brick),
+// 80.6 / 104.7; FP32 8000 ions on 30^3 (2.2e5), 63.8 / 80.4, and 64 such
+// replicas 289 / 264.
+bool large_bricks(const mfe_engine *e, const int s[3], int order) {
+  constexpr long long kFill = 256;  // CUs
+  long long nb = 1;
+  for (int m = 0; m < 3; ++m) nb *= s[m] / brick_edge(s[m], order, true);
+  const long long points = e->prec == MFE_PREC_MIXED ? 1 << 17 : 1 << 16;
+  return nb >= kFill || (long long)e->np * order * order * order <= points * nb;
 }
 
 void free_all(mfe_engine *e) {
@@ -1147,10 +1166,10 @@ int mfe_set_ewald(mfe_engine *e, int32_t kind, double alpha, int32_t order,
         e->plan[m] = make_plan(e->s[m]);
         if (!plan_ok(e->plan[m])) return fail(e, MFE_E_BAD_PARAM, "mesh has a prime factor > 32");
       }
-      // bricks of the spreading and gather blocks: the largest edges of
-      // brick_edge whose tile a CU's LDS holds (62 x 62 x 24 at order 6:
-      // edges 31, 31 and 8; with 12 the tile is 172 KB)
-      bool large = true;
+      // bricks of the spreading and gather blocks, the large ones only where
+      // a CU's LDS holds their tile (62 x 62 x 24 at order 6: edges 31, 31
+      // and 8; with 12 the tile is 172 KB)
+      bool large = large_bricks(e, e->s, order);
       size_t ext, planes;
       for (;; large = false) {
         ext = 1;

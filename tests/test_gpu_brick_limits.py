@@ -1,6 +1,7 @@
-"""Meshes whose brick tiles come near the LDS of a CU: axes of 2 x 31 points
-beside an axis whose largest brick would not fit with them, against the
-oracle."""
+"""The choice of the brick edges where it turns, against the oracle: tiles
+near the LDS of a CU (axes of 2 x 31 points beside an axis whose largest
+brick would not fit with them) and the particles per brick above which few
+bricks are made smaller."""
 import numpy as np
 import pytest
 
@@ -55,3 +56,11 @@ def against_oracle(mesh, order, n, prec, ftol):
 @pytest.mark.parametrize("prec,ftol", [("fp64", 1e-10), ("mixed", 1e-5)])
 def test_small_edge_beside_large_ones(mesh, order, n, prec, ftol):
     against_oracle(mesh, order, n, prec, ftol)
+
+
+# 24^3 at order 6 is eight bricks of edge 12 up to 2^16 (FP64) or 2^17 (mixed)
+# stencil points per brick, 2427 and 4854 particles, then 27 of edge 8
+@pytest.mark.parametrize("n", [2427, 2428, 4854, 4855])
+@pytest.mark.parametrize("prec,ftol", [("fp64", 1e-10), ("mixed", 1e-5)])
+def test_few_crowded_bricks(n, prec, ftol):
+    against_oracle((24, 24, 24), 6, n, prec, ftol)
