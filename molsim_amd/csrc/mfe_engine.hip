@@ -187,6 +187,7 @@ void free_all(mfe_engine *e) {
   dfree(e->b_id); dfree(e->b_slot); dfree(e->rec_frac); dfree(e->rec_meta);
   dfree(e->spread_tiles);
   dfree(e->mc_ia); dfree(e->mc_rtm); dfree(e->mc_old); dfree(e->mc_part);
+  dfree(e->mc_fac);
   if (e->mc_spec) (void)hipFree(e->mc_spec);
   e->mc_spec = nullptr;
   e->mc_spec_bytes = 0;
@@ -1554,6 +1555,18 @@ mfe::McMove mc_move(mfe_engine *e, const std::vector<int> &ia, const double *rtm
 // (valid once the stream is synchronized)
 double *mc_results(mfe_engine *e) { return reinterpret_cast<double *>(e->h_mc); }
 
+// the factor table of a move of natm particles, or null where the passes over
+// the spectrum form the factors themselves (k_mc_fac)
+double *mc_factors(mfe_engine *e, int natm) {
+  if (natm < mfe::mc_table_min()) return nullptr;
+  const size_t n = 4 * (size_t)natm * (e->s[0] + e->s[1] + e->s[2]);
+  if (e->mc_fac_cap < n) {
+    dalloc(e->mc_fac, n);
+    e->mc_fac_cap = n;
+  }
+  return e->mc_fac;
+}
+
 // the kept spectrum (the complex mesh's size, FP64 values on both precision
 // paths; a new buffer is not a valid one) and room for the positions of
 // natm moved particles
@@ -1725,6 +1738,8 @@ int mfe_mc_delta_rec(mfe_engine *e, int32_t natm, const int32_t *ianatm, const d
     MFE_HIP_TRY(hipSetDevice(e->device));
     mc_buffers(e, natm);
     mc_spectrum_buffers(e, natm);
+    // what an accept takes of the last trial is overwritten from here on
+    e->mc_last_ia.clear();
     const mfe::McMove mv = mc_move(e, ia, rtm);
     sync_view(e);
     const mfe::Group &G = e->grp;
@@ -1738,7 +1753,7 @@ int mfe_mc_delta_rec(mfe_engine *e, int32_t natm, const int32_t *ianatm, const d
     }
     // the energy change over the spectrum, the blocks' parts added in order
     double *part = mc_results(e);
-    const int nb = mfe::launch_mc_rec(G, mv, e->mc_spec, e->mc_old, part);
+    const int nb = mfe::launch_mc_rec(G, mv, e->mc_spec, e->mc_old, mc_factors(e, natm), part);
     MFE_HIP_TRY(hipStreamSynchronize(e->stream));
     double h = 0.0;
     for (int b = 0; b < nb; ++b) h += part[b];
@@ -1787,7 +1802,8 @@ int mfe_mc_accept(mfe_engine *e, int32_t natm, const int32_t *ianatm, const doub
     // the trial's change added to the kept spectrum, and the accepted
     // positions, then NList(iSimulationStep) as after an upload
     const bool small = natm <= mfe::kMcArg;
-    mfe::launch_mc_accept(G, mv, small, keep ? e->mc_spec : nullptr, e->mc_old);
+    mfe::launch_mc_accept(G, mv, small, keep ? e->mc_spec : nullptr, e->mc_old,
+                          keep ? mc_factors(e, natm) : nullptr);
     if (!small) {
       if (!e->ro_stage) dalloc(e->ro_stage, 3 * (size_t)e->max_np);
       MFE_HIP_TRY(hipMemcpyAsync(e->ro_stage, e->ro, 3 * (size_t)e->np * sizeof(double),

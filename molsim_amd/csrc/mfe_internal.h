@@ -574,10 +574,11 @@ struct mfe_engine {
   int *b_count = nullptr, *b_start = nullptr, *b_id = nullptr, *b_slot = nullptr;
   // Monte Carlo trial moves: the moved particles, trial and current
   // positions on the device (the first two for moves of more than kMcArg),
-  // and the pair part's block partials
+  // the pair part's block partials and the factors of larger moves
   int *mc_ia = nullptr;
-  double *mc_rtm = nullptr, *mc_old = nullptr, *mc_part = nullptr;
+  double *mc_rtm = nullptr, *mc_old = nullptr, *mc_part = nullptr, *mc_fac = nullptr;
   int mc_cap = 0, mc_old_cap = 0;
+  size_t mc_fac_cap = 0;
   // the kept spectrum (forward transform of the current configuration's
   // mesh, valid while mc_cached)
   void *mc_spec = nullptr;
@@ -737,15 +738,20 @@ struct McMove {
 };
 // most blocks (and parts of the sum) of a trial's pass over the spectrum
 constexpr int kMcRecBlocks = 1024;
-// Monte Carlo trial move, reciprocal part (mc_rec_body): the energy change
+// Monte Carlo trial move, reciprocal part (mc_pass): the energy change
 // (without EpsiFourPi) over the kept spectrum spec as part[b] of each of the
-// returned number of blocks (device-visible memory), the moved particles'
-// current positions into old[3 natm].  One replica.
-int launch_mc_rec(const Group &g, const McMove &mv, void *spec, double *old, double *part);
-// an accepted move, the last that launch_mc_rec was given: place (at most
-// kMcArg particles): launch_set_positions with it in place; with spec also
-// spec += its change
-void launch_mc_accept(const Group &g, const McMove &mv, bool place, void *spec, double *old);
+// returned number of blocks (device-visible memory).  Moves of mc_table_min()
+// particles and more need fac, room for their factors (2 natm (s1 + s2 + s3)
+// complex FP64 values), and leave them there; without fac the moved
+// particles' current positions are left in old[3 natm].  One replica.
+int mc_table_min();
+int launch_mc_rec(const Group &g, const McMove &mv, void *spec, double *old, void *fac,
+                  double *part);
+// an accepted move, the last that launch_mc_rec was given (with the same old
+// and fac): place (at most kMcArg particles): launch_set_positions with it in
+// place; with spec also spec += its change
+void launch_mc_accept(const Group &g, const McMove &mv, bool place, void *spec, double *old,
+                      const void *fac);
 // the z forward transform of the complex mesh into out (no Green function)
 void fft_z_forward(const Group &g, void *out);
 // Monte Carlo trial move, pair part: out[0] the two-body energy change,

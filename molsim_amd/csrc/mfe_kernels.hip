@@ -1691,26 +1691,16 @@ __global__ void __launch_bounds__(256) k_mc_place(int natm, const int *__restric
 // to the rounding of the spreading's products.  One replica, fewer than
 // 2^31 points, kx fastest.
 //
-// A block takes tiles of kMcTile consecutive spectrum points (four per
-// thread, their D in registers) and forms the factors that the tile needs
-// in LDS: x factors c(kx) with the charge folded in, and per mesh row
-// (ky, kz) the product of its y and z factors, each for the current (n = 0)
-// and the trial (1) position of up to `chunk` moved particles at a time.
-// The roots exp(-2 pi i p / s) of all axes come first, one per thread, so a
-// factor is ORDER products with table values at exactly reduced phases.
-// apply == false writes the block's part of the energy change to
-// part[block] (the host adds the parts in block order) and block 0 keeps
-// the current positions in `old`; apply == true adds D to F for the move
-// just tried, from those.
-// A trial costs one launch, bound by the latencies of roots, factors and
-// spectrum: 8.6 us for one particle in an 80^3 mesh.  The factor tables, the
-// pass and the sum as kernels of their own took 7.5, 4.6 and 3.8 us (the
-// call 31 us, now 24.5).  Two points per thread and twice the blocks
-// measured 8.8 us.
+// A block takes tiles of 256 P consecutive spectrum points (P per thread,
+// their D in registers) and holds the factors that the tile needs in LDS, of
+// up to `chunk` moved particles at a time: x factors c(kx) with the charge
+// folded in, and per mesh row (ky, kz) the product of its y and z factors,
+// each for the current (n = 0) and the trial (1) position (McLds).  apply ==
+// false writes the block's part of the energy change to part[block] (the
+// host adds the parts in block order); apply == true adds D to F.
 constexpr int kMcPoints = 4;
-constexpr int kMcTile = 256 * kMcPoints;
 // mesh rows that a tile can touch
-__host__ __device__ inline int mc_rows(int hx) { return (kMcTile - 1) / hx + 2; }
+__host__ __device__ inline int mc_rows(int hx, int P) { return (256 * P - 1) / hx + 2; }
 
 __device__ __forceinline__ int mc_ia(const McMove &mv, int a) {
   return mv.natm <= kMcArg ? mv.ia_v[a] : mv.ia[a];
@@ -1719,92 +1709,45 @@ __device__ __forceinline__ double mc_rtm(const McMove &mv, int k) {
   return mv.natm <= kMcArg ? mv.rtm_v[k] : mv.rtm[k];
 }
 
-template <typename R, int ORDER>
-__device__ __forceinline__ void mc_rec_body(const SysDev &V, const McMove &mv, int chunk,
-                                            double2 *__restrict__ F, double *__restrict__ old,
-                                            bool apply, double *__restrict__ part, int blk,
-                                            int nblk) {
-  extern __shared__ __align__(16) unsigned char mc_lds[];
-  const SpmeGeom &g = V.sg;
+// fill(a, trial, x, row): the factor of moved particle a at wavenumber x >= 0
+// of the x axis, or (x < 0) the product of its factors along mesh row `row`
+template <int P, typename Fill>
+__device__ __forceinline__ void mc_pass(const SysDev &V, int natm, int chunk, double2 *lds,
+                                        double2 *__restrict__ F, bool apply,
+                                        double *__restrict__ part, int blk, int nblk,
+                                        Fill fill) {
   const SpmeAxes &ax = V.ax;
-  const int s0 = g.s[0], s1 = g.s[1], s2 = g.s[2], hx = V.hx;
+  const int s0 = V.sg.s[0], s1 = V.sg.s[1], s2 = V.sg.s[2], hx = V.hx;
   const unsigned n = (unsigned)hx * s1 * s2;
-  const int rows = mc_rows(hx);
-  double2 *root = reinterpret_cast<double2 *>(mc_lds);        // [s0 + s1 + s2]
-  double2 *fx = root + s0 + s1 + s2;                          // [2 chunk][hx]
-  double2 *fr = fx + 2 * chunk * hx;                          // [2 chunk][rows]
-  for (int k = threadIdx.x; k < s0 + s1 + s2; k += blockDim.x) {
-    const int m = k < s0 ? 0 : (k < s0 + s1 ? 1 : 2);
-    const int ph = k - (m == 0 ? 0 : (m == 1 ? s0 : s0 + s1));
-    double sn, cs;
-    sincospi(-2.0 * (double)ph / (double)(m == 0 ? s0 : (m == 1 ? s1 : s2)), &sn, &cs);
-    root[k] = make_double2(cs, sn);
-  }
-  if (!apply && blk == 0)
-    for (int k = threadIdx.x; k < 3 * mv.natm; k += blockDim.x)
-      old[k] = V.ro[3 * mc_ia(mv, k / 3) + k % 3];
-  // the factor of an axis of sm points (its roots at rt) at wavenumber k
-  auto factor = [&](double x, double dk, int sm, const double2 *rt, int k) -> double2 {
-    const double u = dk * x;
-    const double f = floor(u);
-    int pt = (int)f % sm;
-    pt += pt < 0 ? sm : 0;
-    R w[ORDER];
-    bspline<R, ORDER>((R)(u - f), w, nullptr);
-    // the phase k (pt - j) reduced to [0, s): pt, k < s < 2^15
-    int ph = (int)(((unsigned)k * (unsigned)pt) % (unsigned)sm);
-    double re = 0.0, im = 0.0;
-#pragma unroll
-    for (int j = 0; j < ORDER; ++j) {
-      const double2 c = rt[ph];
-      re += (double)w[j] * c.x;
-      im += (double)w[j] * c.y;
-      ph -= k;
-      ph += ph < 0 ? sm : 0;
-    }
-    return make_double2(re, im);
-  };
+  const int rows = mc_rows(hx, P);
+  double2 *fx = lds;                     // [2 chunk][hx]
+  double2 *fr = fx + 2 * chunk * hx;     // [2 chunk][rows]
   double acc = 0.0;
-  for (unsigned e0 = (unsigned)blk * kMcTile; e0 < n; e0 += (unsigned)nblk * kMcTile) {
+  for (unsigned e0 = (unsigned)blk * (256 * P); e0 < n; e0 += (unsigned)nblk * (256 * P)) {
     const unsigned r0 = e0 / (unsigned)hx;
-    const unsigned r1 = (min(e0 + kMcTile, n) - 1) / (unsigned)hx;
+    const unsigned r1 = (min(e0 + 256 * P, n) - 1) / (unsigned)hx;
     const int nr = (int)(r1 - r0) + 1, ne = hx + nr;
-    double2 v[kMcPoints];
-    double dr[kMcPoints], di[kMcPoints];
+    double2 v[P];
+    double dr[P], di[P];
 #pragma unroll
-    for (int u = 0; u < kMcPoints; ++u) {
+    for (int u = 0; u < P; ++u) {
       v[u] = F[min(e0 + u * 256 + threadIdx.x, n - 1)];
       dr[u] = 0.0;
       di[u] = 0.0;
     }
-    for (int a0 = 0; a0 < mv.natm; a0 += chunk) {
-      const int na = min(chunk, mv.natm - a0);
+    for (int a0 = 0; a0 < natm; a0 += chunk) {
+      const int na = min(chunk, natm - a0);
       // the roots are written, the last chunk's factors read
       __syncthreads();
       for (int t = threadIdx.x; t < 2 * na * ne; t += blockDim.x) {
         const int row = t / ne, k = t - row * ne;
-        const int a = a0 + (row >> 1), i = mc_ia(mv, a);
-        double r[3];
-#pragma unroll
-        for (int m = 0; m < 3; ++m)
-          r[m] = (row & 1) ? mc_rtm(mv, 3 * a + m) : (apply ? old[3 * a + m] : V.ro[3 * i + m]);
-        if (k < hx) {
-          const double2 c = factor(r[0], g.dkdr[0], s0, root, k);
-          // the splines' divisors with the charge
-          const double q = (double)(R)V.q[i] * kSplineScale<ORDER, 0>;
-          fx[row * hx + k] = make_double2(c.x * q, c.y * q);
-        } else {
-          const unsigned rr = r0 + (unsigned)(k - hx), kz = rr / (unsigned)s1;
-          const double2 cy = factor(r[1], g.dkdr[1], s1, root + s0,
-                                    (int)(rr - kz * (unsigned)s1));
-          const double2 cz = factor(r[2], g.dkdr[2], s2, root + s0 + s1, (int)kz);
-          fr[row * rows + k - hx] =
-              make_double2(cy.x * cz.x - cy.y * cz.y, cy.x * cz.y + cy.y * cz.x);
-        }
+        const double2 c = fill(a0 + (row >> 1), row & 1, k < hx ? k : -1,
+                               r0 + (unsigned)max(k - hx, 0));
+        (k < hx ? fx[row * hx + k] : fr[row * rows + k - hx]) = c;
       }
       __syncthreads();
 #pragma unroll
-      for (int u = 0; u < kMcPoints; ++u) {
+      for (int u = 0; u < P; ++u) {
         const unsigned e = min(e0 + u * 256 + threadIdx.x, n - 1), r = e / (unsigned)hx;
         const int kx = (int)(e - r * (unsigned)hx), kr = (int)(r - r0);
         for (int a = 0; a < 2 * na; a += 2) {
@@ -1816,7 +1759,7 @@ __device__ __forceinline__ void mc_rec_body(const SysDev &V, const McMove &mv, i
       }
     }
 #pragma unroll
-    for (int u = 0; u < kMcPoints; ++u) {
+    for (int u = 0; u < P; ++u) {
       const unsigned e = e0 + u * 256 + threadIdx.x;
       if (e >= n) continue;
       if (apply) {
@@ -1841,12 +1784,154 @@ __device__ __forceinline__ void mc_rec_body(const SysDev &V, const McMove &mv, i
   if (threadIdx.x == 0) part[blk] = t;
 }
 
+// the roots exp(-2 pi i p / s) of the three axes, by the whole block
+__device__ __forceinline__ void mc_roots(const SpmeGeom &g, double2 *root) {
+  const int s0 = g.s[0], s1 = g.s[1], s2 = g.s[2];
+  for (int k = threadIdx.x; k < s0 + s1 + s2; k += blockDim.x) {
+    const int m = k < s0 ? 0 : (k < s0 + s1 ? 1 : 2);
+    const int ph = k - (m == 0 ? 0 : (m == 1 ? s0 : s0 + s1));
+    double sn, cs;
+    sincospi(-2.0 * (double)ph / (double)(m == 0 ? s0 : (m == 1 ? s1 : s2)), &sn, &cs);
+    root[k] = make_double2(cs, sn);
+  }
+}
+
+// the factor of an axis of sm points (its roots at rt) at wavenumber k:
+// ORDER products with roots at exactly reduced phases
+template <typename R, int ORDER>
+__device__ __forceinline__ double2 mc_factor(double x, double dk, int sm, const double2 *rt,
+                                             int k) {
+  const double u = dk * x;
+  const double f = floor(u);
+  int pt = (int)f % sm;
+  pt += pt < 0 ? sm : 0;
+  R w[ORDER];
+  bspline<R, ORDER>((R)(u - f), w, nullptr);
+  // the phase k (pt - j) reduced to [0, s): pt, k < s < 2^15
+  int ph = (int)(((unsigned)k * (unsigned)pt) % (unsigned)sm);
+  double re = 0.0, im = 0.0;
+#pragma unroll
+  for (int j = 0; j < ORDER; ++j) {
+    const double2 c = rt[ph];
+    re += (double)w[j] * c.x;
+    im += (double)w[j] * c.y;
+    ph -= k;
+    ph += ph < 0 ? sm : 0;
+  }
+  return make_double2(re, im);
+}
+__device__ __forceinline__ double2 mc_mul(double2 a, double2 b) {
+  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+}
+// a moved particle's charge with the splines' divisors
+template <typename R, int ORDER>
+__device__ __forceinline__ double mc_charge(const SysDev &V, int i) {
+  return (double)(R)V.q[i] * kSplineScale<ORDER, 0>;
+}
+
+// Moves of fewer than kMcTable particles: each block forms the factors of its
+// tile from the roots, so a trial costs one launch, bound by the latencies
+// of roots, factors and spectrum: 8.6 us for one particle in an 80^3 mesh
+// (the factors, the pass and the sum as kernels of their own took 7.5, 4.6
+// and 3.8 us).  Two points per thread and twice the blocks measured 8.8 us.
+// Block 0 of a trial keeps the current positions in `old`; the accept takes
+// the change of the move just tried from those.
+template <typename R, int ORDER>
+__device__ __forceinline__ void mc_rec_body(const SysDev &V, const McMove &mv, int chunk,
+                                            double2 *__restrict__ F, double *__restrict__ old,
+                                            bool apply, double *__restrict__ part, int blk,
+                                            int nblk) {
+  extern __shared__ __align__(16) unsigned char mc_lds[];
+  const SpmeGeom &g = V.sg;
+  const int s0 = g.s[0], s1 = g.s[1], s2 = g.s[2];
+  double2 *root = reinterpret_cast<double2 *>(mc_lds);        // [s0 + s1 + s2]
+  mc_roots(g, root);
+  if (!apply && blk == 0)
+    for (int k = threadIdx.x; k < 3 * mv.natm; k += blockDim.x)
+      old[k] = V.ro[3 * mc_ia(mv, k / 3) + k % 3];
+  mc_pass<kMcPoints>(
+      V, mv.natm, chunk, root + s0 + s1 + s2, F, apply, part, blk, nblk,
+      [&](int a, int trial, int x, unsigned row) -> double2 {
+        const int i = mc_ia(mv, a);
+        double r[3];
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+          r[m] = trial ? mc_rtm(mv, 3 * a + m) : (apply ? old[3 * a + m] : V.ro[3 * i + m]);
+        if (x >= 0) {
+          const double2 c = mc_factor<R, ORDER>(r[0], g.dkdr[0], s0, root, x);
+          const double q = mc_charge<R, ORDER>(V, i);
+          return make_double2(c.x * q, c.y * q);
+        }
+        const unsigned kz = row / (unsigned)s1;
+        return mc_mul(mc_factor<R, ORDER>(r[1], g.dkdr[1], s1, root + s0,
+                                          (int)(row - kz * (unsigned)s1)),
+                      mc_factor<R, ORDER>(r[2], g.dkdr[2], s2, root + s0 + s1, (int)kz));
+      });
+}
+
 template <typename R, int ORDER>
 __global__ void __launch_bounds__(256) k_mc_rec(const SysDev *__restrict__ sys, const McMove mv,
                                                 int chunk, double2 *spec, double *old,
                                                 double *part) {
   mc_rec_body<R, ORDER>(sys[0], mv, chunk, spec, old, false, part, (int)blockIdx.x,
                         (int)gridDim.x);
+}
+
+// Moves of kMcTable particles and more: a launch of its own forms the factors
+// of all moved particles, fac[(2 a + n) (s1 + s2 + s3) + axis offset + k], the
+// charge in those of the x axis; the trial's pass and the accept's take them
+// from there.  Formed in every block they are the time of a larger move: 64
+// particles, order 6, meshes of 80^3 97 us (66 from the table), of 48^3 96
+// (42); 500 particles 613 (352) and 612 (175).  The table costs a launch, so
+// for one or two particles the trial is up to 0.7 us faster without it
+// (128^3).  Small meshes take one point per thread, so that their tiles
+// occupy the chip: 24^3, 64 particles 68 us with four, 39 with one.
+constexpr int kMcTable = 3;
+template <typename R, int ORDER>
+__global__ void __launch_bounds__(256) k_mc_fac(const SysDev *__restrict__ sys, const McMove mv,
+                                                double2 *__restrict__ fac) {
+  extern __shared__ __align__(16) unsigned char mc_lds[];
+  const SysDev &V = sys[0];
+  const SpmeGeom &g = V.sg;
+  const int s0 = g.s[0], s1 = g.s[1], s2 = g.s[2], ns = s0 + s1 + s2;
+  double2 *root = reinterpret_cast<double2 *>(mc_lds);
+  mc_roots(g, root);
+  __syncthreads();
+  const long long total = 2ll * mv.natm * ns;
+  for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < total;
+       t += (long long)gridDim.x * blockDim.x) {
+    const int row = (int)(t / ns), k0 = (int)(t - (long long)row * ns);
+    const int a = row >> 1, i = mc_ia(mv, a);
+    const int m = k0 < s0 ? 0 : (k0 < s0 + s1 ? 1 : 2);
+    const int off = m == 0 ? 0 : (m == 1 ? s0 : s0 + s1);
+    const double x = (row & 1) ? mc_rtm(mv, 3 * a + m) : V.ro[3 * i + m];
+    const double2 c = mc_factor<R, ORDER>(x, g.dkdr[m], g.s[m], root + off, k0 - off);
+    const double q = m == 0 ? mc_charge<R, ORDER>(V, i) : 1.0;
+    fac[t] = make_double2(c.x * q, c.y * q);
+  }
+}
+
+template <int P>
+__device__ __forceinline__ void mc_tab_body(const SysDev &V, int natm, int chunk,
+                                            double2 *__restrict__ F,
+                                            const double2 *__restrict__ fac, bool apply,
+                                            double *__restrict__ part, int blk, int nblk) {
+  extern __shared__ __align__(16) unsigned char mc_lds[];
+  const int s0 = V.sg.s[0], s1 = V.sg.s[1], ns = s0 + s1 + V.sg.s[2];
+  mc_pass<P>(V, natm, chunk, reinterpret_cast<double2 *>(mc_lds), F, apply, part, blk, nblk,
+             [&](int a, int trial, int x, unsigned row) -> double2 {
+               const double2 *f = fac + (size_t)(2 * a + trial) * ns;
+               if (x >= 0) return f[x];
+               const unsigned kz = row / (unsigned)s1;
+               return mc_mul(f[s0 + (int)(row - kz * (unsigned)s1)], f[s0 + s1 + (int)kz]);
+             });
+}
+
+template <int P>
+__global__ void __launch_bounds__(256) k_mc_tab(const SysDev *__restrict__ sys, int natm,
+                                                int chunk, double2 *spec,
+                                                const double2 *__restrict__ fac, double *part) {
+  mc_tab_body<P>(sys[0], natm, chunk, spec, fac, false, part, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // UTwoBodyANew/UTwoBodyAOld (Src/denergy.F90:289-495) for a trial move of
@@ -2841,8 +2926,9 @@ __global__ void __launch_bounds__(kBlock) k_set_positions(const SysDev *__restri
 // positions are set apart) place a move of up to kMcArg particles and update
 // the displacements, the others add the trial's change to the kept spectrum
 // (none where no spectrum is kept).  That change is taken from `old`, the
-// positions before the move, so the two parts are independent: 9.3 us in one
-// launch (50000 particles, 80^3 mesh), 4.6 and 5.9 us in two.
+// positions before the move, or from the trial's factor table, so the two
+// parts are independent: 9.3 us in one launch (one of 50000 particles, 80^3
+// mesh), 4.6 and 5.9 us in two.
 template <typename R, int ORDER>
 __global__ void __launch_bounds__(kBlock) k_mc_accept(const SysDev *__restrict__ sys,
                                                       const McMove mv, int nset, int chunk,
@@ -2852,6 +2938,18 @@ __global__ void __launch_bounds__(kBlock) k_mc_accept(const SysDev *__restrict__
   else
     mc_rec_body<R, ORDER>(sys[0], mv, chunk, spec, old, true, nullptr, (int)blockIdx.x - nset,
                           (int)gridDim.x - nset);
+}
+// the same with the change from the trial's factor table
+template <int P>
+__global__ void __launch_bounds__(kBlock) k_mc_accept_tab(const SysDev *__restrict__ sys,
+                                                          const McMove mv, int nset, int chunk,
+                                                          double2 *spec,
+                                                          const double2 *__restrict__ fac) {
+  if ((int)blockIdx.x < nset)
+    set_positions_body(sys[0], nullptr, &mv);
+  else
+    mc_tab_body<P>(sys[0], mv.natm, chunk, spec, fac, true, nullptr, (int)blockIdx.x - nset,
+                   (int)gridDim.x - nset);
 }
 
 // NList's r2max2 (Src/nlist.F90:602-608) is the largest r2 that is not a
@@ -3723,21 +3821,24 @@ void launch_mc_place(const Group &g, int natm, const int *ia, const double *rtm,
                      ro_stage);
 }
 
-// moved particles whose factors a block holds at a time: up to eight, as
-// many as 32 KB of LDS take beside the roots
-static int mc_chunk(const Group &g, int natm) {
+// points per thread, blocks, moved particles whose factors a block holds at a
+// time (as many as 32 KB of LDS take beside the roots) and dynamic LDS of a
+// pass over the spectrum
+struct McPass {
+  int P, nb, chunk;
+  size_t lds;
+};
+static McPass mc_plan(const Group &g, int natm, bool table) {
   const int hx = g.mc_s[0] / 2 + 1;
-  const size_t per = 2 * (size_t)(hx + mc_rows(hx)) * sizeof(double2);
-  return (int)std::max<size_t>(1, std::min<size_t>({(size_t)natm, 8, (32 * 1024) / per}));
-}
-static size_t mc_lds_bytes(const Group &g, int chunk) {
-  const int hx = g.mc_s[0] / 2 + 1;
-  return ((size_t)(g.mc_s[0] + g.mc_s[1] + g.mc_s[2]) +
-          2 * (size_t)chunk * (hx + mc_rows(hx))) * sizeof(double2);
-}
-static int mc_rec_blocks(const Group &g) {
-  const size_t n = (size_t)(g.mc_s[0] / 2 + 1) * g.mc_s[1] * g.mc_s[2];
-  return (int)std::min<size_t>((n + kMcTile - 1) / kMcTile, kMcRecBlocks);
+  const size_t n = (size_t)hx * g.mc_s[1] * g.mc_s[2];
+  McPass p;
+  p.P = table && n < 256 * 256 * kMcPoints ? 1 : kMcPoints;
+  p.nb = (int)std::min<size_t>((n + 256 * p.P - 1) / (256 * p.P), kMcRecBlocks);
+  const size_t per = 2 * (size_t)(hx + mc_rows(hx, p.P)) * sizeof(double2);
+  p.chunk = (int)std::max<size_t>(1, std::min<size_t>(natm, (32 * 1024) / per));
+  p.lds = p.chunk * per;
+  if (!table) p.lds += (size_t)(g.mc_s[0] + g.mc_s[1] + g.mc_s[2]) * sizeof(double2);
+  return p;
 }
 
 // dynamic LDS above the default limit (meshes of about 1000 points along
@@ -3753,31 +3854,58 @@ static void mc_allow_lds(const void *kernel, size_t lds) {
     MFE_MC(T, 3) MFE_MC(T, 4) MFE_MC(T, 5) MFE_MC(T, 6) MFE_MC(T, 7) MFE_MC(T, 8) \
   }
 
-int launch_mc_rec(const Group &g, const McMove &mv, void *spec, double *old, double *part) {
-  const int nb = mc_rec_blocks(g), chunk = mc_chunk(g, mv.natm);
-  const size_t lds = mc_lds_bytes(g, chunk);
-#define MFE_MC(T, O)                                                                       \
-  case O:                                                                                  \
-    mc_allow_lds((const void *)k_mc_rec<T, O>, lds);                                       \
-    hipLaunchKernelGGL((k_mc_rec<T, O>), dim3(nb), dim3(256), lds, g.stream, g.d, mv,      \
-                       chunk, (double2 *)spec, old, part);                                 \
+int mc_table_min() { return kMcTable; }
+
+int launch_mc_rec(const Group &g, const McMove &mv, void *spec, double *old, void *fac,
+                  double *part) {
+  const McPass p = mc_plan(g, mv.natm, fac != nullptr);
+  const int ns = g.mc_s[0] + g.mc_s[1] + g.mc_s[2];
+  const int nf = (int)std::min(((long long)mv.natm * 2 * ns + 255) / 256, 1024ll);
+  double2 *f2 = (double2 *)fac, *s2 = (double2 *)spec;
+#define MFE_MC(T, O)                                                                        \
+  case O:                                                                                   \
+    if (fac) {                                                                              \
+      hipLaunchKernelGGL((k_mc_fac<T, O>), dim3(nf), dim3(256), ns * sizeof(double2),       \
+                         g.stream, g.d, mv, f2);                                            \
+      break;                                                                                \
+    }                                                                                       \
+    mc_allow_lds((const void *)k_mc_rec<T, O>, p.lds);                                      \
+    hipLaunchKernelGGL((k_mc_rec<T, O>), dim3(p.nb), dim3(256), p.lds, g.stream, g.d, mv,   \
+                       p.chunk, s2, old, part);                                             \
     break;
   if (g.prec == MFE_PREC_MIXED) { MFE_MC_CASES(float) }
   else { MFE_MC_CASES(double) }
 #undef MFE_MC
-  return nb;
+  if (fac && p.P == 1)
+    hipLaunchKernelGGL(k_mc_tab<1>, dim3(p.nb), dim3(256), p.lds, g.stream, g.d, mv.natm,
+                       p.chunk, s2, (const double2 *)f2, part);
+  else if (fac)
+    hipLaunchKernelGGL(k_mc_tab<kMcPoints>, dim3(p.nb), dim3(256), p.lds, g.stream, g.d,
+                       mv.natm, p.chunk, s2, (const double2 *)f2, part);
+  return p.nb;
 }
 
-void launch_mc_accept(const Group &g, const McMove &mv, bool place, void *spec, double *old) {
-  const int nset = place ? g.np_blocks : 0, nb = nset + (spec ? mc_rec_blocks(g) : 0);
+void launch_mc_accept(const Group &g, const McMove &mv, bool place, void *spec, double *old,
+                      const void *fac) {
+  const McPass p = spec ? mc_plan(g, mv.natm, fac != nullptr) : McPass{kMcPoints, 0, 1, 0};
+  const int nset = place ? g.np_blocks : 0, nb = nset + p.nb;
   if (!nb) return;
-  const int chunk = spec ? mc_chunk(g, mv.natm) : 1;
-  const size_t lds = spec ? mc_lds_bytes(g, chunk) : 0;
+  double2 *s2 = (double2 *)spec;
+  if (spec && fac) {
+    const double2 *f2 = (const double2 *)fac;
+    if (p.P == 1)
+      hipLaunchKernelGGL(k_mc_accept_tab<1>, dim3(nb), dim3(kBlock), p.lds, g.stream, g.d, mv,
+                         nset, p.chunk, s2, f2);
+    else
+      hipLaunchKernelGGL(k_mc_accept_tab<kMcPoints>, dim3(nb), dim3(kBlock), p.lds, g.stream,
+                         g.d, mv, nset, p.chunk, s2, f2);
+    return;
+  }
 #define MFE_MC(T, O)                                                                       \
   case O:                                                                                  \
-    mc_allow_lds((const void *)k_mc_accept<T, O>, lds);                                    \
-    hipLaunchKernelGGL((k_mc_accept<T, O>), dim3(nb), dim3(kBlock), lds, g.stream, g.d,    \
-                       mv, nset, chunk, (double2 *)spec, old);                             \
+    mc_allow_lds((const void *)k_mc_accept<T, O>, p.lds);                                  \
+    hipLaunchKernelGGL((k_mc_accept<T, O>), dim3(nb), dim3(kBlock), p.lds, g.stream, g.d,  \
+                       mv, nset, p.chunk, s2, old);                                        \
     return;
   if (spec && g.prec == MFE_PREC_MIXED) { MFE_MC_CASES(float) }
   else if (spec) { MFE_MC_CASES(double) }
