@@ -119,6 +119,12 @@ __device__ __forceinline__ void column_sums(const double *__restrict__ part, int
   }
 }
 
+// index of the pair of types i and j (Set_iptpt order: j >= i, j fastest)
+__device__ __forceinline__ int pair_index(int i, int j, int npt) {
+  const int a = min(i, j), b = max(i, j);
+  return a * npt - a * (a - 1) / 2 + b - a;
+}
+
 struct KahanF {
   float s = 0.f, c = 0.f;
   __device__ __forceinline__ void add(float v) {

@@ -1981,6 +1981,8 @@ int mfe_adjoint(mfe_engine *e, double *dE_dq, double *dE_dzat, double *dE_dsigat
   if (!e->have_pp) return fail(e, MFE_E_STATE, "mfe_set_pair_params not called");
   if (e->ewald == MFE_EWALD_STD)
     return fail(e, MFE_E_BAD_PARAM, "the adjoint covers SPME and no-Ewald systems");
+  if (!mfe::adjoint_fits(e->nptpt * e->nknot))
+    return fail(e, MFE_E_BAD_PARAM, "the adjoint's sums of the spline coefficients exceed a block's LDS");
   if (!e->list_valid) {
     rc = mfe_build_list(e);
     if (rc) return rc;
@@ -2072,7 +2074,7 @@ void fm_buffers(mfe_engine *e) {
 // surface term; forceo = force * ffac as UTotal leaves it
 void fm_forward(mfe_engine *e) {
   const mfe::Group &G = e->grp;
-  mfe::launch_fm_pair(G, false, nullptr, 0, e->np);
+  mfe::launch_fm_pair(G, false, nullptr, 0, e->np, e->npt, 0);
   if (G.ewald == MFE_EWALD_SPME) mfe::launch_spme(G, false, SP_BIN, SP_GATHER, mfe::GM_FIELD);
   if (G.chains) mfe::launch_bonds(G);
   if (G.surf) mfe::launch_surf(G);
@@ -2149,6 +2151,8 @@ int mfe_fm_loss_grad(mfe_engine *e, double *loss, double *dL_dzat, double *dL_ds
   if (rc) return rc;
   if (e->fm_nframes < 1 || e->fm_frame_np != e->np)
     return fail(e, MFE_E_STATE, "mfe_fm_set_frames first (for this np)");
+  if (!mfe::fm_fits(e->prec, e->npt, e->nptpt * e->nknot))
+    return fail(e, MFE_E_BAD_PARAM, "the gradient's sums of the spline coefficients exceed a block's LDS");
   return guarded(e, [&]() -> int {
     MFE_HIP_TRY(hipSetDevice(e->device));
     e->mc_cached = false;
@@ -2171,7 +2175,7 @@ int mfe_fm_loss_grad(mfe_engine *e, double *loss, double *dL_dzat, double *dL_ds
       fm_forward(e);
       mfe::launch_fm_resid(G, e->fm_tgt + n3 * f, part_r);
       mfe::launch_fm_acc(G, part_r, nb, 4, 1, e->fm_acc);
-      mfe::launch_fm_pair(G, true, part_p, ncolp, np);
+      mfe::launch_fm_pair(G, true, part_p, ncolp, np, npt, e->nptpt * e->nknot);
       mfe::launch_fm_acc(G, part_p, nb4, ncolp, ncolp, e->fm_acc + 1 + npt);
       if (G.ewald == MFE_EWALD_SPME) mfe::launch_fm_rec_backward(G);
       mfe::launch_fm_q(G, part_r, e->fm_qr, part_q);

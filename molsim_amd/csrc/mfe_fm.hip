@@ -89,17 +89,17 @@ __global__ void __launch_bounds__(kFmBlock) k_fm_pair(const SysDev *__restrict__
   extern __shared__ double sk[];
   __shared__ double sh[kFmBlock / 64];
   const int nk = V.nptpt * V.nknot;
-  // the types' parameters and pair indices in LDS (read per entry by the
-  // partner's type)
-  __shared__ R zat_s[MFE_MAX_TYPES], sig_s[MFE_MAX_TYPES], eps_s[MFE_MAX_TYPES];
-  __shared__ int pidx_s[MFE_MAX_TYPES * MFE_MAX_TYPES];
+  // the types' parameters in LDS (read per entry by the partner's type),
+  // behind the sums of the spline coefficients, which may take nearly all of
+  // a CU's LDS (fm_pair_lds)
+  R *zat_s = reinterpret_cast<R *>(sk + (BWD ? nk : 0));
+  R *sig_s = zat_s + V.npt, *eps_s = sig_s + V.npt;
   const PairParams &pp = V.pp;
   for (int k = threadIdx.x; k < V.npt; k += blockDim.x) {
     zat_s[k] = (R)pp.zat[k];
     sig_s[k] = (R)pp.sigat[k];
     eps_s[k] = (R)pp.epsat[k];
   }
-  for (int k = threadIdx.x; k < V.npt * V.npt; k += blockDim.x) pidx_s[k] = V.tab.pairidx[k];
   if (BWD)
     for (int k = threadIdx.x; k < nk; k += blockDim.x) sk[k] = 0.0;
   __syncthreads();
@@ -190,7 +190,7 @@ __global__ void __launch_bounds__(kFmBlock) k_fm_pair(const SysDev *__restrict__
           kn = knot_weights((double)r2d > 0.0 ? sqrt(r2d) : 0.0, V.knot_r0, V.knot_dinv, V.nknot,
                             ki, w4, dw4);
           if (kn) {
-            pidx = pidx_s[ti * V.npt + tj];
+            pidx = pair_index(ti, tj, V.npt);
             if (!BWD) {
               const double *c = V.knot_c + (size_t)pidx * V.nknot + ki;
               const double dup =
@@ -419,22 +419,34 @@ inline dim3 grid1(int x, const Group &g) { return dim3(x > 0 ? x : 1, 1, g.R); }
 
 }  // namespace
 
-void launch_fm_pair(const Group &g, bool backward, double *part, int ncol, int np) {
+// the sums of nk spline coefficients and the types' parameters
+static size_t fm_pair_lds(int prec, int npt, int nk) {
+  return (size_t)nk * sizeof(double) +
+         3 * (size_t)npt * (prec == MFE_PREC_MIXED ? sizeof(float) : sizeof(double));
+}
+bool fm_fits(int prec, int npt, int nk) {
+  return fm_pair_lds(prec, npt, nk) + kFmBlock / 64 * sizeof(double) <= kCuLds;
+}
+
+void launch_fm_pair(const Group &g, bool backward, double *part, int ncol, int np, int npt,
+                    int nk) {
   const int nb = (np + kFmBlock / kFmLanes - 1) / (kFmBlock / kFmLanes);
-  const size_t lds = backward ? (size_t)std::max(ncol, 1) * sizeof(double) : 0;
+  const size_t lds = fm_pair_lds(g.prec, npt, backward ? nk : 0);
   if (g.prec == MFE_PREC_MIXED) {
+    allow_lds((const void *)k_fm_pair<float, true>, lds);
     if (backward)
       hipLaunchKernelGGL((k_fm_pair<float, true>), grid1(nb, g), dim3(kFmBlock), lds, g.stream,
                          g.d, part, ncol);
     else
-      hipLaunchKernelGGL((k_fm_pair<float, false>), grid1(nb, g), dim3(kFmBlock), 0, g.stream,
+      hipLaunchKernelGGL((k_fm_pair<float, false>), grid1(nb, g), dim3(kFmBlock), lds, g.stream,
                          g.d, part, ncol);
   } else {
+    allow_lds((const void *)k_fm_pair<double, true>, lds);
     if (backward)
       hipLaunchKernelGGL((k_fm_pair<double, true>), grid1(nb, g), dim3(kFmBlock), lds, g.stream,
                          g.d, part, ncol);
     else
-      hipLaunchKernelGGL((k_fm_pair<double, false>), grid1(nb, g), dim3(kFmBlock), 0, g.stream,
+      hipLaunchKernelGGL((k_fm_pair<double, false>), grid1(nb, g), dim3(kFmBlock), lds, g.stream,
                          g.d, part, ncol);
   }
 }

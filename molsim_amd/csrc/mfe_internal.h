@@ -697,6 +697,11 @@ void launch_spme(const Group &g, bool energy, int first_stage, int last_stage,
 void launch_adjoint(const Group &g, int np, int npt, int ncol, double *part, double *out,
                     double *dro);
 int adjoint_blocks(int np);  // rows of its partials
+// whether the sums of nk spline coefficients fit a block's LDS
+bool adjoint_fits(int nk);
+bool fm_fits(int prec, int npt, int nk);
+// a launch with dynamic LDS above the runtime's default limit
+void allow_lds(const void *kernel, size_t lds);
 // the standard Ewald sum: structure factors, then the forces from them
 void launch_std_factors(const Group &g);
 void launch_std_forces(const Group &g);
@@ -782,7 +787,8 @@ void launch_fill_double(double *p, int n, double v, hipStream_t s);
 // ncol columns); the residual and its partials [|r|^2, q r]; the
 // reciprocal part (residual mesh spread, convolved, potential gathered);
 // dL/dq per particle with per-type partials; column sums into acc
-void launch_fm_pair(const Group &g, bool backward, double *part, int ncol, int np);
+void launch_fm_pair(const Group &g, bool backward, double *part, int ncol, int np, int npt,
+                    int nk);
 int fm_pair_blocks(int np);
 void launch_fm_resid(const Group &g, const double *tgt, double *part);
 void launch_fm_rec_backward(const Group &g);

@@ -2581,12 +2581,11 @@ __global__ void __launch_bounds__(kBlock) k_adjoint(const SysDev *__restrict__ s
   const int np = V.np;
   if ((int)blockIdx.x * kAdjPer >= np) return;
   extern __shared__ double sk[];
-  __shared__ double sh[kBlock];
+  __shared__ double sh[kBlock / 64];
   const int nk = V.nptpt * V.nknot;
-  // the types' parameters and pair indices in LDS (read per entry by the
-  // partner's type)
+  // the types' parameters in LDS (read per entry by the partner's type); the
+  // sums of the spline coefficients may take nearly all of it (adjoint_lds)
   __shared__ double zat_s[MFE_MAX_TYPES], sig_s[MFE_MAX_TYPES], eps_s[MFE_MAX_TYPES];
-  __shared__ int pidx_s[MFE_MAX_TYPES * MFE_MAX_TYPES];
   const PairParams &pp = V.pp;
   const TableDev &t = V.tab;
   for (int k = threadIdx.x; k < V.npt; k += blockDim.x) {
@@ -2594,7 +2593,6 @@ __global__ void __launch_bounds__(kBlock) k_adjoint(const SysDev *__restrict__ s
     sig_s[k] = pp.sigat[k];
     eps_s[k] = pp.epsat[k];
   }
-  for (int k = threadIdx.x; k < t.npt * t.npt; k += blockDim.x) pidx_s[k] = t.pairidx[k];
   for (int k = threadIdx.x; k < nk; k += blockDim.x) sk[k] = 0.0;
   __syncthreads();
   const Box b = V.box;
@@ -2650,7 +2648,7 @@ __global__ void __launch_bounds__(kBlock) k_adjoint(const SysDev *__restrict__ s
           int ki;
           double w[4], dw[4];
           if (knot_weights(r, V.knot_r0, V.knot_dinv, V.nknot, ki, w, dw)) {
-            const int pidx = pidx_s[ti * t.npt + tj];
+            const int pidx = pair_index(ti, tj, t.npt);
             const double *c = V.knot_c + (size_t)pidx * V.nknot + ki;
             eu += 0.5 * (c[0] * w[0] + c[1] * w[1] + c[2] * w[2] + c[3] * w[3]);
             for (int m = 0; m < 4; ++m) atomicAdd(&sk[pidx * V.nknot + ki + m], 0.5 * w[m]);
@@ -3841,9 +3839,7 @@ static McPass mc_plan(const Group &g, int natm, bool table) {
   return p;
 }
 
-// dynamic LDS above the default limit (meshes of about 1000 points along
-// each axis)
-static void mc_allow_lds(const void *kernel, size_t lds) {
+void allow_lds(const void *kernel, size_t lds) {
   if (lds > 60 * 1024)
     (void)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
 }
@@ -3869,7 +3865,7 @@ int launch_mc_rec(const Group &g, const McMove &mv, void *spec, double *old, voi
                          g.stream, g.d, mv, f2);                                            \
       break;                                                                                \
     }                                                                                       \
-    mc_allow_lds((const void *)k_mc_rec<T, O>, p.lds);                                      \
+    allow_lds((const void *)k_mc_rec<T, O>, p.lds);                                      \
     hipLaunchKernelGGL((k_mc_rec<T, O>), dim3(p.nb), dim3(256), p.lds, g.stream, g.d, mv,   \
                        p.chunk, s2, old, part);                                             \
     break;
@@ -3903,7 +3899,7 @@ void launch_mc_accept(const Group &g, const McMove &mv, bool place, void *spec, 
   }
 #define MFE_MC(T, O)                                                                       \
   case O:                                                                                  \
-    mc_allow_lds((const void *)k_mc_accept<T, O>, p.lds);                                  \
+    allow_lds((const void *)k_mc_accept<T, O>, p.lds);                                  \
     hipLaunchKernelGGL((k_mc_accept<T, O>), dim3(nb), dim3(kBlock), p.lds, g.stream, g.d,  \
                        mv, nset, p.chunk, s2, old);                                        \
     return;
@@ -4186,10 +4182,13 @@ void launch_collect(const Group &g, int *fl, double *en, int nen) {
   hipLaunchKernelGGL(k_collect, grid(1, g), dim3(64), 0, g.stream, g.d, fl, en, nen);
 }
 
+// the sums of the spline coefficients
+static size_t adjoint_lds(int nk) { return (size_t)std::max(nk, 1) * sizeof(double); }
+
 void launch_adjoint(const Group &g, int np, int npt, int ncol, double *part, double *out,
                     double *dro) {
-  // LDS of the knot accumulators: the largest replica's nptpt*nknot doubles
-  const size_t lds = (size_t)std::max(ncol - 1, 1) * sizeof(double);
+  const size_t lds = adjoint_lds(ncol - 1 - 2 * npt);
+  allow_lds((const void *)k_adjoint, lds);
   hipLaunchKernelGGL(k_adjoint, grid(g.np_blocks * kAdjLanes, g), dim3(kBlock), lds, g.stream,
                      g.d);
   double *zpart = part + (size_t)adjoint_blocks(np) * ncol;
@@ -4201,6 +4200,9 @@ void launch_adjoint(const Group &g, int np, int npt, int ncol, double *part, dou
                      g.stream, zpart, g.np_blocks, npt, out + ncol);
 }
 int adjoint_blocks(int np) { return (np + kAdjPer - 1) / kAdjPer; }
+bool adjoint_fits(int nk) {
+  return adjoint_lds(nk) + (kBlock / 64 + 3 * MFE_MAX_TYPES) * sizeof(double) <= kCuLds;
+}
 
 void launch_set_positions(const Group &g, const double *ro_new) {
   hipLaunchKernelGGL(k_set_positions, grid(g.np_blocks, g), dim3(kBlock), 0, g.stream, g.d,
