@@ -747,8 +747,11 @@ bool mfe_launch_utotal(const mfe::Group &g, unsigned flags, int mode, double dt,
   // launch also finalizes each particle (forceo only) and reduces the
   // partials.  With the kick the finalize phase reads and writes velocities
   // and accelerations too, scattered in brick order: a separate launch in
-  // particle order is faster then.
-  const bool gather_fin = g.ewald == MFE_EWALD_SPME && !g.chains && !g.surf && mode == 0;
+  // particle order is faster then.  The finalize phase has static LDS of
+  // its own (384 bytes), which the largest FP64 tiles leave no room for.
+  constexpr size_t kFinLds = 512;
+  const bool gather_fin = g.ewald == MFE_EWALD_SPME && !g.chains && !g.surf && mode == 0 &&
+                          g.lds_gather + kFinLds <= mfe::kCuLds;
   if (gather_fin) {
     const mfe::FinArgs fa{energy ? 1 : 0, skin ? 1 : 0, bd ? 1 : 0, mode, dt};
     mfe::launch_spme(g, energy, first, SP_GATHER, mfe::GM_FORCE, &fa);

@@ -58,6 +58,13 @@ def test_small_edge_beside_large_ones(mesh, order, n, prec, ftol):
     against_oracle(mesh, order, n, prec, ftol)
 
 
+# bricks of 17 x 29 x 29 at order 4: a tile of exactly 160 KB, which has no room
+# for an odd plane nor, in FP64, for a launch's own LDS beside it
+@pytest.mark.parametrize("prec,ftol", [("fp64", 1e-10), ("mixed", 1e-5)])
+def test_tile_of_a_whole_lds(prec, ftol):
+    against_oracle((34, 58, 58), 4, 600, prec, ftol)
+
+
 # 24^3 at order 6 is eight bricks of edge 12 up to 2^16 (FP64) or 2^17 (mixed)
 # stencil points per brick, 2427 and 4854 particles, then 27 of edge 8
 @pytest.mark.parametrize("n", [2427, 2428, 4854, 4855])
