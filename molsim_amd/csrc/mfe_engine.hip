@@ -205,9 +205,7 @@ void free_all(mfe_engine *e) {
   dfree(e->adj_part); dfree(e->adj_out); dfree(e->adj_dro);
   dfree(e->fm_ro); dfree(e->fm_tgt); dfree(e->fm_fld); dfree(e->fm_res); dfree(e->fm_res_s);
   dfree(e->fm_vec); dfree(e->fm_part); dfree(e->fm_acc); dfree(e->fm_qr);
-  if (e->ring) e->ring->release();
-  delete e->ring;
-  e->ring = nullptr;
+  e->ring.reset();
   if (e->h_en) (void)hipHostFree(e->h_en);
   if (e->h_flags) (void)hipHostFree(e->h_flags);
   e->h_en = nullptr;
@@ -821,7 +819,7 @@ int mfe_create(const mfe_config *cfg, mfe_engine **out) {
     MFE_HIP_TRY(hipSetDevice(e->device));
     MFE_HIP_TRY(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
     MFE_HIP_TRY(mfe::side_create(e->side));
-    e->ring = new mfe::DownloadRing();
+    e->ring = mfe::device_ring(e->device);
     hipDeviceProp_t prop;
     MFE_HIP_TRY(hipGetDeviceProperties(&prop, e->device));
     e->ncu = prop.multiProcessorCount;

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <memory>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -587,8 +588,8 @@ struct mfe_engine {
   // of more than kMcArg particles, so its copies run on the stream
   char *h_mc = nullptr;
   size_t h_mc_bytes = 0;
-  // pinned slots of large downloads (made on the first one)
-  mfe::DownloadRing *ring = nullptr;
+  // pinned slots of large downloads, shared with the device's other engines
+  std::shared_ptr<mfe::DownloadRing> ring;
   bool mc_cached = false;
   // the move of the last mfe_mc_delta_rec (0-based indices, positions):
   // mfe_mc_accept of the same move keeps its trial mesh and E_rec

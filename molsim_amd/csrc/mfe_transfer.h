@@ -7,6 +7,8 @@
 #include <atomic>
 #include <cmath>
 #include <cstring>
+#include <map>
+#include <memory>
 #include <mutex>
 #include <system_error>
 #include <thread>
@@ -21,10 +23,20 @@ namespace mfe {
 // into it runs on one thread, page faults included.  Here the data go
 // through a ring of pinned slots, and threads that live for the call copy
 // each slot out.  Measured, runtime -> ring: positions, velocities and
-// accelerations of a million particles into new arrays (72 MB) 6.7 -> 2.6 ms,
-// of 200000 (14.4 MB) 0.99 -> 0.78 ms; forces of 100000 (2.4 MB) 0.171 ->
-// 0.157 ms new, 0.149 -> 0.122 ms into kept arrays; below two slots nothing
-// overlaps.
+// accelerations of a million particles into new arrays (72 MB) 5.4 -> 2.4 ms,
+// of 200000 (14.4 MB) 1.07 -> 0.90 ms, into kept arrays 0.79 -> 0.53; forces
+// of 100000 (2.4 MB) 0.171 -> 0.157 ms new, 0.149 -> 0.122 ms into kept
+// arrays; below two slots nothing overlaps.
+//
+// The engines of a device share one ring, which the last of them frees.  The
+// first touch of its pages costs the host 0.1 ms per MB with all threads
+// (0.38 ms with one), so with a ring of its own every engine's first download
+// had been slower than the runtime's wherever the caller's memory had pages:
+// 3.6 MB 0.29 -> 1.0 ms, 14.4 MB 2.0 -> 2.6, now 0.24 and 0.95 from the second
+// engine on.  (Leaving the first downloads to the runtime instead cost more
+// where that memory had none: 14.4 MB 2.3 and 2.4 ms for the first two, 2.5
+// and 0.9 through a new ring.)  A download that finds the ring in use by
+// another engine's takes the runtime's copy.
 struct DownloadRing {
   // half of a slot is used below kHalfBelow, where its copies are too few to
   // overlap (3.0 ms with half slots for the 72 MB)
@@ -35,32 +47,40 @@ struct DownloadRing {
   static constexpr int kLag = 10;
   static constexpr int kThreads = 6;
 
-  std::mutex mu;  // downloads of one engine from several threads take turns
+  std::mutex mu;
   char *pin = nullptr;
   size_t bytes = 0;
   hipEvent_t ev[kSlots] = {};
 
-  // room for `need` bytes of slots (no more than a download has)
-  void create(size_t need) {
+  // the slot size of a download of `total` bytes, with the slots made
+  size_t take(size_t total) {
+    const size_t slot = total < kHalfBelow ? kSlot / 2 : kSlot;
+    if (bytes >= kSlots * slot) return slot;
     for (hipEvent_t &x : ev)
       if (!x) MFE_HIP_TRY(hipEventCreateWithFlags(&x, hipEventDisableTiming));
-    if (bytes >= need) return;
     if (pin) MFE_HIP_TRY(hipHostFree(pin));
     pin = nullptr;
     bytes = 0;
-    MFE_HIP_TRY(hipHostMalloc((void **)&pin, need));
-    bytes = need;
+    MFE_HIP_TRY(hipHostMalloc((void **)&pin, kSlots * slot));
+    bytes = kSlots * slot;
+    return slot;
   }
-  void release() {
+  ~DownloadRing() {
     if (pin) (void)hipHostFree(pin);
-    pin = nullptr;
-    bytes = 0;
-    for (hipEvent_t &x : ev) {
+    for (hipEvent_t &x : ev)
       if (x) (void)hipEventDestroy(x);
-      x = nullptr;
-    }
   }
 };
+
+// the device's ring, shared by the engines that hold it
+inline std::shared_ptr<DownloadRing> device_ring(int device) {
+  static std::mutex mu;
+  static std::map<int, std::weak_ptr<DownloadRing>> rings;
+  std::lock_guard<std::mutex> turn(mu);
+  std::shared_ptr<DownloadRing> r = rings[device].lock();
+  if (!r) rings[device] = r = std::make_shared<DownloadRing>();
+  return r;
+}
 
 constexpr size_t kDownloadRingMin = 2 << 20;
 
@@ -76,23 +96,24 @@ inline void download(DownloadRing &ring, int device, const std::vector<DownloadP
                      hipStream_t s, bool wait = true) {
   size_t total = 0;
   for (const DownloadPart &p : parts) total += p.bytes;
-  if (total < kDownloadRingMin) {
+  std::unique_lock<std::mutex> turn(ring.mu, std::defer_lock);
+  size_t slot = 0;
+  if (total >= kDownloadRingMin) {
+    MFE_HIP_TRY(hipSetDevice(device));
+    if (turn.try_lock()) slot = ring.take(total);
+  }
+  if (!slot) {
     for (const DownloadPart &p : parts)
       MFE_HIP_TRY(hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, s));
     if (wait) MFE_HIP_TRY(hipStreamSynchronize(s));
     return;
   }
-  MFE_HIP_TRY(hipSetDevice(device));
-  std::lock_guard<std::mutex> turn(ring.mu);
-  const size_t slot = total < DownloadRing::kHalfBelow ? DownloadRing::kSlot / 2
-                                                       : DownloadRing::kSlot;
   std::vector<DownloadPart> c;
   for (const DownloadPart &p : parts)
     for (size_t o = 0; o < p.bytes; o += slot)
       c.push_back({(char *)p.dst + o, (const char *)p.src + o, std::min(slot, p.bytes - o)});
   constexpr int K = DownloadRing::kSlots;
   const int n = (int)c.size();
-  ring.create(std::min(n, K) * slot);
   std::atomic<int> ready{0}, next{0}, stop{0};
   std::vector<std::atomic<int>> done(n);
   for (auto &d : done) d.store(0, std::memory_order_relaxed);
@@ -111,15 +132,19 @@ inline void download(DownloadRing &ring, int device, const std::vector<DownloadP
       copy_out(k);
     }
   };
-  // the threads end with the call, also when a copy fails
-  struct Joined {
+  // the threads end with the call and no copy into the slots outlives it,
+  // also when one fails
+  struct Ended {
     std::vector<std::thread> t;
     std::atomic<int> &stop;
-    ~Joined() {
+    hipStream_t s;
+    bool complete;
+    ~Ended() {
       stop.store(1);
       for (std::thread &x : t) x.join();
+      if (!complete) (void)hipStreamSynchronize(s);
     }
-  } pool{{}, stop};
+  } pool{{}, stop, s, false};
   pool.t.reserve(DownloadRing::kThreads);
   auto issue = [&](int k) {
     MFE_HIP_TRY(hipMemcpyAsync(ring.pin + (k % K) * slot, c[k].src, c[k].bytes,
@@ -146,6 +171,7 @@ inline void download(DownloadRing &ring, int device, const std::vector<DownloadP
     }
   }
   for (int k = 0; k < n; ++k) finished(k);
+  pool.complete = true;
 }
 
 // whether every coordinate of n particles lies in the box [-L2, L2] (NaN
