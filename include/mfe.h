@@ -388,9 +388,10 @@ int mfe_fm_loss_grad(mfe_engine *e, double *loss, double *dL_dzat,
    launch where the replicas allow it (mfe_batch_step_bd).  The replicas
    must share device, precision, Ewald kind and SPME order; box, N, mesh,
    tables and cutoffs are per replica.  Each replica computes exactly what
-   its engine computes alone.  Results stay in the engines (mfe_download_forces,
-   mfe_download_state, mfe_get_energy) or come back together through
-   mfe_batch_get_energies.  The engines must outlive the batch; a set-up
+   its engine computes alone, bit for bit (in the persistent launch, up to
+   the rounding of sums in another order).  Results stay in the engines
+   (mfe_download_forces, mfe_download_state, mfe_get_energy) or come back
+   together through mfe_batch_get_energies.  The engines must outlive the batch; a set-up
    call on an engine is picked up at the batch's next call.  On an error
    mfe_batch_failed_replica names the first failing replica. */
 typedef struct mfe_batch mfe_batch;

@@ -248,13 +248,14 @@ namespace {
 // Where the caller has not said, batches of fewer than two replicas per CU
 // replay the per-stage graph: a replica's persistent step takes a CU's time
 // however many CUs stand idle, and the per-stage launches spread every
-// replica over the chip.  Per BD step, persistent against per-stage: 8
-// replicas of up to 4000 ions (rc 18 A, meshes 18-36) 812 / 83 us, 96: 935 /
-// 288, 384: 1191 / 911; 96 of up to 1000 ions 254 / 157; 512 at rc 20 A and
-// meshes 16-48 1604 / 1169, 1024: 2241 / 2337.  The schedules cross between
-// two and four replicas per CU, depending on their sizes; from two on the
-// persistent launch stays the default, whose results do not depend on the
-// batch a replica is in, and the autotuner times both.
+// replica over the chip.  Per BD step, persistent / per-stage, replicas of
+// 500 to 4000 ions, rc 18 A, meshes 18-36: 8 replicas 800 / 77 us, 96: 957 /
+// 254, 512: 1335 / 1053; 300 of 125 to 1000 ions 386 / 283.  At 512 replicas
+// the two are level for the plan that the autotuner finds for a force error
+// of 1e-3 (meshes 16-36 at order 4: 1148 / 1156), and at 1024 for larger
+// meshes too (16-48: 2241 / 2337); between those sizes the per-stage
+// launches are up to a quarter faster for some sets.  From two replicas per
+// CU on the persistent launch stays the default; the autotuner times both.
 bool persist_eligible(const mfe_batch *b, size_t *lds) {
   if (b->persist == 0) return false;
   if (b->persist < 0 && (int)b->eng.size() < 2 * std::max(b->eng[0]->ncu, 1)) return false;

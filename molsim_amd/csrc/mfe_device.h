@@ -60,9 +60,9 @@ __device__ __forceinline__ double wave_sum(double x) {
   return (read_lane(x, 0) + read_lane(x, 16)) + (read_lane(x, 32) + read_lane(x, 48));
 }
 
-// Block-wide sum (max) in a fixed order: wave_sum (a shuffle tree) inside
-// each wavefront, then the wavefront results in wavefront order.  Every thread
-// gets the result; sh needs one slot per wavefront.
+// Block-wide sum (max) in a fixed order: wave_sum (for the maximum a shuffle
+// tree) inside each wavefront, then the wavefront results in wavefront order.
+// Every thread gets the result; sh needs one slot per wavefront.
 __device__ __forceinline__ double block_sum(double v, double *sh) {
   v = wave_sum(v);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;

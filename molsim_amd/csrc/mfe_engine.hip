@@ -313,9 +313,14 @@ void set_cell_geom(mfe_engine *e) {
 
 // log2 of the lanes sharing a particle in the list build: they test four
 // candidates each of a row of three cells at a time, so short rows keep one
-// lane busy; long ones are split as far as the particles leave the chip's
-// ~260,000 resident threads idle (beyond that the split only adds partly
-// filled batches).
+// lane busy, and long ones are split as far as that fills the chip's 524,288
+// threads (16 lanes) or twice that (4).  A whole rebuild with 1 / 4 / 16
+// lanes: 66000 particles, rows of 5: 48.8 / 48.3 / 104 us, of 9: 68 / 53 /
+// 107, of 48: 184 / 114 / 118; rows of 24, 4000 particles: 76 / 38 / 29,
+// 16000: 78 / 41 / 41, 32000: 79 / 48 / 62, and of 44 there 158 / 69 / 67, of
+// 280 706 / 283 / 207; beyond 262144 particles the split of rows up to 25
+// costs more than it gives (300000, rows of 18: 182 / 212 / 395), of longer
+// ones it would gain a little (of 45: 379 / 334 / 422).
 int list_lsh_for(const mfe_engine *e) {
   const double row = 3.0 * e->np / std::max(e->cg.ncells, 1);
   if (row < 8.0) return 0;

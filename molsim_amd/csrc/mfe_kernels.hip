@@ -1325,7 +1325,7 @@ __global__ void k_spme_clear(const SysDev *__restrict__ sys) {
 // barrier between particles) and loads the record of its next item before
 // its own adds, so the load latency hides behind them.
 // 1024 threads share one brick's tile; without other LDS two blocks fit a
-// CU at 16-point bricks of order <= 7.
+// CU at 16-point bricks of order <= 6 (at order 7 a tile is 83 KB).
 constexpr int kSpreadThreads = 1024;
 
 template <typename R, int ORDER>
@@ -1537,70 +1537,57 @@ __device__ __forceinline__ void gather_body(const SysDev *__restrict__ sys, FinA
       fn = load_rec(frac + 4 * (first + pn));
       mn = meta[first + pn];
     }
-    double ex = 0.0, ey = 0.0, ez = 0.0, ep = 0.0;
-    if (l < ORDER) {
-      R v[3][ORDER], d[3][ORDER];
-      bspline<R, ORDER>(f.x, v[0], d[0]);
-      bspline<R, ORDER>(f.y, v[1], d[1]);
-      bspline<R, ORDER>(f.z, v[2], d[2]);
-      // brick-local coordinates inside the staged region
-      const int lx = (md.x & 1023) - o0 + ORDER - 1;
-      const int ly = ((md.x >> 10) & 1023) - o1 + ORDER - 1;
-      const int lz = ((md.x >> 20) & 1023) - o2 + ORDER - 1;
-      Acc3<R> acc;
-      double pacc = 0.0;
+    R v[3][ORDER], d[3][ORDER];
+    bspline<R, ORDER>(f.x, v[0], d[0]);
+    bspline<R, ORDER>(f.y, v[1], d[1]);
+    bspline<R, ORDER>(f.z, v[2], d[2]);
+    // brick-local coordinates inside the staged region
+    const int lx = (md.x & 1023) - o0 + ORDER - 1;
+    const int ly = ((md.x >> 10) & 1023) - o1 + ORDER - 1;
+    const int lz = ((md.x >> 20) & 1023) - o2 + ORDER - 1;
+    Acc3<R> acc;
+    double pacc = 0.0;
 #pragma unroll
-      for (int kz = 0; kz < kPlanes; ++kz) {
-        const int iz = l + GL * kz;
-        if (iz >= ORDER) break;
-        // weights of plane iz, selected among this step's GL planes
-        R vz = v[2][0], dz = d[2][0];
+    for (int kz = 0; kz < kPlanes; ++kz) {
+      const int iz = l + GL * kz;
+      if (iz >= ORDER) break;
+      // weights of plane iz, selected without indexing registers
+      R vz = v[2][0], dz = d[2][0];
 #pragma unroll
-        for (int k = 1; k < ORDER; ++k)
-          if (iz == k) {
-            vz = v[2][k];
-            dz = d[2][k];
-          }
-        const R *plane = tile + (size_t)(lz - iz) * E1 * E0;
-#pragma unroll
-        for (int iy = 0; iy < ORDER; ++iy) {
-          const R *row = plane + (ly - iy) * E0;
-          R sx = R(0), sdx = R(0);
-#pragma unroll
-          for (int ix = 0; ix < ORDER; ++ix) {
-            const R qv = row[lx - ix];
-            sx += v[0][ix] * qv;
-            sdx += d[0][ix] * qv;
-          }
-          if (MODE != GM_POTONLY) {
-            acc.add(0, sdx * (v[1][iy] * vz));
-            acc.add(1, sx * (d[1][iy] * vz));
-            acc.add(2, sx * (v[1][iy] * dz));
-          }
-          if (MODE == GM_POT || MODE == GM_POTONLY) pacc += (double)sx * (double)(v[1][iy] * vz);
+      for (int k = 1; k < ORDER; ++k)
+        if (iz == k) {
+          vz = v[2][k];
+          dz = d[2][k];
         }
-      }
-      ex = acc.get(0) * kSplineScale<ORDER, 1>;
-      ey = acc.get(1) * kSplineScale<ORDER, 1>;
-      ez = acc.get(2) * kSplineScale<ORDER, 1>;
-      ep = pacc * kSplineScale<ORDER, 0>;
-    }
-    // the GL lanes of a particle are all in or all out of the loop
-    if constexpr (GL == 2) {
-      // the lane pair within a quad, by DPP
-      ex += quad_swap<kXor1>(ex);
-      ey += quad_swap<kXor1>(ey);
-      ez += quad_swap<kXor1>(ez);
-      if (MODE == GM_POT || MODE == GM_POTONLY) ep += quad_swap<kXor1>(ep);
-    } else {
+      const R *plane = tile + (size_t)(lz - iz) * E1 * E0;
 #pragma unroll
-      for (int w = 1; w < GL; w <<= 1) {
-        ex += __shfl_xor(ex, w, GL);
-        ey += __shfl_xor(ey, w, GL);
-        ez += __shfl_xor(ez, w, GL);
-        if (MODE == GM_POT || MODE == GM_POTONLY) ep += __shfl_xor(ep, w, GL);
+      for (int iy = 0; iy < ORDER; ++iy) {
+        const R *row = plane + (ly - iy) * E0;
+        R sx = R(0), sdx = R(0);
+#pragma unroll
+        for (int ix = 0; ix < ORDER; ++ix) {
+          const R qv = row[lx - ix];
+          sx += v[0][ix] * qv;
+          sdx += d[0][ix] * qv;
+        }
+        if (MODE != GM_POTONLY) {
+          acc.add(0, sdx * (v[1][iy] * vz));
+          acc.add(1, sx * (d[1][iy] * vz));
+          acc.add(2, sx * (v[1][iy] * dz));
+        }
+        if (MODE == GM_POT || MODE == GM_POTONLY) pacc += (double)sx * (double)(v[1][iy] * vz);
       }
     }
+    double ex = acc.get(0) * kSplineScale<ORDER, 1>;
+    double ey = acc.get(1) * kSplineScale<ORDER, 1>;
+    double ez = acc.get(2) * kSplineScale<ORDER, 1>;
+    double ep = pacc * kSplineScale<ORDER, 0>;
+    // both lanes of a particle are in or out of the loop: the lane pair within
+    // a quad, by DPP
+    ex += quad_swap<kXor1>(ex);
+    ey += quad_swap<kXor1>(ey);
+    ez += quad_swap<kXor1>(ez);
+    if (MODE == GM_POT || MODE == GM_POTONLY) ep += quad_swap<kXor1>(ep);
     if (owner) {
       // q fld rounded before the pair force is added (no contraction): the
       // same sum as the finalize forms from force and force_rec
@@ -3200,7 +3187,7 @@ __device__ __forceinline__ double block_prefix_max(double v, double *wm, double 
 }
 
 // exclusive prefix sum of cnt[0..n) into start[0..n], start[n] = total;
-// the counts are left zero, as every rebuild expects them (ph_scan_offset)
+// the counts are left zero, as every rebuild expects them (ph_cell_rank)
 __device__ __forceinline__ void block_scan_counts(int *cnt, int *start, int n, int *wsum) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
   int carry = 0;
