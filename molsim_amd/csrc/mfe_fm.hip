@@ -117,6 +117,10 @@ __global__ void __launch_bounds__(kFmBlock) k_fm_pair(const SysDev *__restrict__
     const double xi = V.ro_s[3 * tt], yi = V.ro_s[3 * tt + 1], zi = V.ro_s[3 * tt + 2];
     ti = V.type_s[tt];
     const R qi = zat_s[ti], si = sig_s[ti], ei = eps_s[ti];
+    // the pair index of each partner type, a byte each
+    unsigned long long ptp = 0;
+    for (int k = 0; k < V.npt; ++k)
+      ptp |= (unsigned long long)pair_index(ti, k, V.npt) << (8 * k);
     R rxi = 0, ryi = 0, rzi = 0;
     if (BWD) {
       rxi = (R)V.fm_res_s[3 * tt];
@@ -190,7 +194,7 @@ __global__ void __launch_bounds__(kFmBlock) k_fm_pair(const SysDev *__restrict__
           kn = knot_weights((double)r2d > 0.0 ? sqrt(r2d) : 0.0, V.knot_r0, V.knot_dinv, V.nknot,
                             ki, w4, dw4);
           if (kn) {
-            pidx = pair_index(ti, tj, V.npt);
+            pidx = (int)((ptp >> (8 * tj)) & 0xff);
             if (!BWD) {
               const double *c = V.knot_c + (size_t)pidx * V.nknot + ki;
               const double dup =
