@@ -359,13 +359,16 @@ int read_flags(mfe_engine *e) {
 int skin_and_rebuild(mfe_engine *e) {
   const mfe::Group &G = e->grp;
   mfe::launch_skin(G);
+  // -1 stays where the launch did not run (the runtime's last error may be
+  // that of any earlier call of the thread)
+  e->h_flags[1] = -1;
   if (!mfe::launch_finalize_rebuild(G, 0u, false, -1, 0.0, false, e->h_flags)) {
     mfe::launch_reduce(G, 0u, true, false);
     mfe::launch_nlist_rebuild(G, true);
     return read_flags(e);
   }
-  MFE_HIP_TRY(hipGetLastError());
   MFE_HIP_TRY(hipStreamSynchronize(e->stream));
+  if (e->h_flags[1] < 0) return fail(e, MFE_E_HIP, "the skin test's launch failed");
   return e->h_flags[1] ? read_flags(e) : mfe_map_flag_error(e, e->h_flags[0]);
 }
 
@@ -751,10 +754,9 @@ bool mfe_launch_utotal(const mfe::Group &g, unsigned flags, int mode, double dt,
   // partials.  With the kick the finalize phase reads and writes velocities
   // and accelerations too, scattered in brick order: a separate launch in
   // particle order is faster then.  The finalize phase has static LDS of
-  // its own (384 bytes), which the largest FP64 tiles leave no room for.
-  constexpr size_t kFinLds = 512;
+  // its own, which the largest FP64 tiles leave no room for.
   const bool gather_fin = g.ewald == MFE_EWALD_SPME && !g.chains && !g.surf && mode == 0 &&
-                          g.lds_gather + kFinLds <= mfe::kCuLds;
+                          g.lds_gather + mfe::kGatherFinLds <= mfe::kCuLds;
   if (gather_fin) {
     const mfe::FinArgs fa{energy ? 1 : 0, skin ? 1 : 0, bd ? 1 : 0, mode, dt};
     mfe::launch_spme(g, energy, first, SP_GATHER, mfe::GM_FORCE, &fa);

@@ -166,6 +166,8 @@ constexpr int kBarWords = kBarGen + kBarStride;
 constexpr int kScanBlocks = 256;
 // LDS of a CU, the most that a block can have
 constexpr size_t kCuLds = 160 * 1024;
+// static LDS of the gather with the finalize phase (384 bytes), rounded up
+constexpr size_t kGatherFinLds = 512;
 // threads per block of the pair kernel and its dynamic LDS budget
 constexpr int kPairBlock = 512;
 // blocks of the persistent pair kernel (two per CU)

@@ -4211,6 +4211,8 @@ void mfe_allow_big_spread_lds(int prec, int bytes) {
   int &al = allowed[prec == MFE_PREC_MIXED ? 1 : 0];
   if (bytes <= al) return;
   al = bytes;
+  // the gather with the finalize phase has static LDS of its own
+  const int fin = std::min(bytes, (int)(mfe::kCuLds - mfe::kGatherFinLds));
 #define MFE_ATTR(R, O)                                                              \
   (void)hipFuncSetAttribute((const void *)mfe::k_spread_ptr<R, O>(),                 \
                             hipFuncAttributeMaxDynamicSharedMemorySize, bytes);        \
@@ -4218,7 +4220,7 @@ void mfe_allow_big_spread_lds(int prec, int bytes) {
     (void)hipFuncSetAttribute(mfe::k_gather_ptr<R, O>(gm, false),                     \
                               hipFuncAttributeMaxDynamicSharedMemorySize, bytes);      \
   (void)hipFuncSetAttribute(mfe::k_gather_ptr<R, O>(mfe::GM_FORCE, true),             \
-                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes);        \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, fin);          \
   (void)hipFuncSetAttribute(mfe::k_fm_spread_ptr<R, O>(),                             \
                             hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   if (prec == MFE_PREC_MIXED) {

@@ -36,6 +36,11 @@ def against_oracle(mesh, order, n, prec, ftol):
     eng.set_neighbor("vlist", 1.0, 0)
     eng.upload_positions(ro)
     f, en = eng.utotal()
+    # positions that move with the list kept: nothing of the set-up above is
+    # reported by a later call
+    eng.upload_positions(np.clip(ro + 0.01, -box / 2, box / 2))
+    eng.upload_positions(ro)
+    assert rel_rms(eng.utotal()[0], f) <= ftol
     eng.close()
     orc = O.Oracle(box, types, zat[types - 1], O.Tables(tab.ubuf, tab.iubuflow, tab.nugrid,
                    tab.r2umin, None), 0.5, ewald="spm", alpha=0.4, epsi_four_pi=EFP,
