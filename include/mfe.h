@@ -343,7 +343,10 @@ int mfe_set_pair_params(mfe_engine *e, const mfe_pot_1_6_12 *spec);
    B-spline in r with nknot coefficients c[p][k] on [r_lo, r_hi) and zero
    outside: u_p(r) = sum_k c[p][k] B_k(r), B_k the cubic B-spline on knots
    r_lo + (j-3) h, h = (r_hi - r_lo)/(nknot-3).  Applied in every UTotal
-   (forces and energies); nknot = 0 removes it. */
+   (forces and energies); nknot = 0 removes it.  mfe_adjoint and
+   mfe_fm_loss_grad sum the coefficients' derivatives in a CU's LDS and
+   return MFE_E_BAD_PARAM for tables that it does not hold (nptpt*nknot
+   beyond about 20,450). */
 int mfe_set_knots(mfe_engine *e, int32_t nknot, double r_lo, double r_hi,
                   const double *c);
 /* One UTotal at the current positions and the gradient of the model
