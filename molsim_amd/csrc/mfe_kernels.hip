@@ -816,7 +816,7 @@ k_pair(const SysDev *__restrict__ sys, int energy, int pgrid, int skin) {
       V.force[3 * io + 2] = fz;
     }
     if (energy && !kRegE) {
-      // pair-type energies of this chunk: a shuffle tree in each
+      // pair-type energies of this chunk: wave_sum in each
       // wavefront, added to the wavefront's own LDS row
       for (int k = 0; k < P; ++k) {
         double v = 0.0;
@@ -833,7 +833,7 @@ k_pair(const SysDev *__restrict__ sys, int energy, int pgrid, int skin) {
   if (err) atomicOr(&flags[0], err);
   if (energy) {
     if (kRegE) {
-      // the pair-type energies of all chunks: a shuffle tree in each
+      // the pair-type energies of all chunks: wave_sum in each
       // wavefront
 #pragma unroll
       for (int k = 0; k < NA; ++k) {
@@ -1111,7 +1111,7 @@ __device__ __forceinline__ void pair_f_body(const SysDev *__restrict__ sys, int 
       V.force[3 * io + 2] = fz;
     }
     if (energy) {
-      // pair-type energies of this chunk: a shuffle tree in each
+      // pair-type energies of this chunk: wave_sum in each
       // wavefront, added to the wavefront's own LDS row
       for (int k = 0; k < P; ++k) {
         double v = 0.0;
